@@ -36,41 +36,16 @@
 
 #include <algorithm>
 
-#include "amf_internal.h"
-#include "amf_kernel_util.h"
+#include "amf_attn.h"
+#include "amf_prefill.h"
 
 namespace {
 
-using amf::u32x4;
-using amf::f32x4;
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
+using namespace amf;
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxD = 256;
 constexpr int kAccPerLane = kMaxD / 64;
-constexpr float kLog2e = 1.4426950408889634f;
-
-struct AttnArgs {
-  const void* q;
-  const void* k;
-  const void* v;
-  const float* mask;
-  int64_t ms0, ms1, ms2, ms3;  // mask strides over (batch, q head, q row, kv token)
-  void* out;
-  int64_t batch;
-  int32_t num_q_heads, num_kv_heads;
-  int64_t q_len, kv_len;
-  int32_t head_dim;
-  float scale;
-  // INT4_SYM K/V (split path only): k and v point at packed codes (element
-  // 8 w + n of a row in nibble n of code word w), these at the fp16
-  // per-channel scales [head_dim].
-  const _Float16* k_scales;
-  const _Float16* v_scales;
-};
-
 template <int DT>
 __device__ __forceinline__ float elem(const void* p, int64_t i) {
   if constexpr (DT == AMF_DTYPE_F32) {
@@ -232,9 +207,6 @@ __global__ __launch_bounds__(kThreads) void dense_attn_kernel(AttnArgs a) {
 #endif
 constexpr int64_t kSplitWaves = AMF_DENSE_SPLIT_WAVES;  // waves one launch aims for
 constexpr int64_t kMinChunks = AMF_DENSE_MIN_CHUNKS;     // 64-token chunks per split, at least
-constexpr int kPartPad = 4;            // a split partial: acc[D], m, l, 2 pad (16-byte rows)
-constexpr int64_t kXcds = 8;           // XCDs of the chip, dealt workgroups round-robin
-
 // Query heads one wave of the split kernel serves: up to 4 of a GQA group
 // of G, so that it loads (and for INT4 dequantizes) each K/V row once for
 // all of them.
@@ -257,8 +229,6 @@ inline void dense_splits(int64_t rows, int hpw, int64_t kv_len, int64_t* n_split
   *split_tokens = per * 64;
   *n_splits = (chunks + per - 1) / per;
 }
-
-inline bool split_head_dim(int32_t D) { return D == 64 || D == 128 || D == 256; }
 
 // Sum over the LPR lanes of a row group (lanes LPR g .. LPR g + LPR - 1).
 template <int LPR>
@@ -295,40 +265,6 @@ __device__ __forceinline__ float across_groups_max(float x) {
   return x;
 }
 
-// INT4 = true: K and V are INT4_SYM codes, dequantized as the codec's restore
-// does, (code - 8) * scale in fp32 rounded to DT (the dtype the restore would
-// write and q's dtype), so the scores see the values a decompressed tensor
-// holds.  (code - 8) * s is taken as fma(code, s, -8 s): the exact product
-// fits fp32 (4 + 11 bits), so the single rounding of the fma is exact too.
-// The nibbles go to bytes first (even elements in w & 0x0F0F0F0F, odd ones
-// in (w >> 4) & 0x0F0F0F0F), so that v_cvt_f32_ubyte0..3 convert them; the
-// empty asm keeps the compiler from folding that back into a bit-field
-// extract per element.
-template <int DT>
-__device__ __forceinline__ float round_to(float y) {
-  if constexpr (DT == AMF_DTYPE_BF16) {
-    return (float)(__bf16)y;
-  } else if constexpr (DT == AMF_DTYPE_F16) {
-    amf::keep_f32(y);
-    return (float)(_Float16)y;
-  } else {
-    return y;
-  }
-}
-
-// The 8 exact products (code - 8) * scale of one code word, before rounding.
-__device__ __forceinline__ void int4_sym_vals(uint32_t w, const float (&s)[8], const float (&z)[8],
-                                              float (&y)[8]) {
-  uint32_t ev = w & 0x0F0F0F0Fu, od = (w >> 4) & 0x0F0F0F0Fu;
-  asm("" : "+v"(ev));
-  asm("" : "+v"(od));
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    y[2 * i] = __builtin_fmaf((float)((ev >> (8 * i)) & 0xFFu), s[2 * i], z[2 * i]);
-    y[2 * i + 1] = __builtin_fmaf((float)((od >> (8 * i)) & 0xFFu), s[2 * i + 1], z[2 * i + 1]);
-  }
-}
-
 // a.lo * b.lo + a.hi * b.hi + c for two bf16 or fp16 pairs (fp32 products
 // and sum).
 template <int DT>
@@ -340,70 +276,6 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, a), __builtin_bit_cast(f16x2_t, b),
                                   c, false);
 }
-
-// One lane's 8 elements of a K/V row as loaded (lane c of a row group holds
-// dims 8c .. 8c + 7 of a head_dim-D row): a code word for INT4, else 16
-// (bf16/fp16) or 32 (fp32) bytes.  decode() gives them as fp32; pairs()
-// (bf16/fp16 only) as four DT pairs, elements 2i and 2i + 1 in word i.
-template <int DT, bool INT4>
-struct RawRow {  // bf16 / fp16
-  u32x4 w;
-  static __device__ __forceinline__ RawRow load(const void* base, int64_t r, int c, int D) {
-    return RawRow{*reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + r * D +
-                                                  8 * c)};
-  }
-  __device__ __forceinline__ void decode(const float (&)[8], const float (&)[8],
-                                         float (&x)[8]) const {
-    amf::unpack8<DT == AMF_DTYPE_BF16>(w, x);
-  }
-  __device__ __forceinline__ void pairs(const float (&)[8], const float (&)[8],
-                                        uint32_t (&pr)[4]) const {
-    pr[0] = w.x;
-    pr[1] = w.y;
-    pr[2] = w.z;
-    pr[3] = w.w;
-  }
-};
-
-template <>
-struct RawRow<AMF_DTYPE_F32, false> {
-  f32x4 lo, hi;
-  static __device__ __forceinline__ RawRow load(const void* base, int64_t r, int c, int D) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + r * D + 8 * c);
-    return RawRow{p[0], p[1]};
-  }
-  __device__ __forceinline__ void decode(const float (&)[8], const float (&)[8],
-                                         float (&x)[8]) const {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      x[e] = lo[e];
-      x[4 + e] = hi[e];
-    }
-  }
-};
-
-template <int DT>
-struct RawRow<DT, true> {
-  uint32_t w;
-  static __device__ __forceinline__ RawRow load(const void* base, int64_t r, int c, int D) {
-    return RawRow{static_cast<const uint32_t*>(base)[r * (D / 8) + c]};
-  }
-  __device__ __forceinline__ void decode(const float (&s)[8], const float (&z)[8],
-                                         float (&x)[8]) const {
-    float y[8];
-    int4_sym_vals(w, s, z, y);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = round_to<DT>(y[e]);
-  }
-  __device__ __forceinline__ void pairs(const float (&s)[8], const float (&z)[8],
-                                        uint32_t (&pr)[4]) const {
-    float y[8];
-    int4_sym_vals(w, s, z, y);
-    // round to nearest even, as decode() and the restore do
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pr[i] = amf::pack2<DT == AMF_DTYPE_BF16>(y[2 * i], y[2 * i + 1]);
-  }
-};
 
 #ifndef AMF_DENSE_BATCH
 #define AMF_DENSE_BATCH 8
@@ -1051,7 +923,9 @@ void launch_split_gh(const AttnArgs& a, float* part, int64_t split_tokens, int64
         <<<grid, 64, 0, st>>>(a, part, split_tokens, n_splits, units);
 }
 
-void launch_merge(const AttnArgs& a, int32_t out_dtype, int64_t rows, const float* part,
+}  // namespace
+
+void amf::launch_merge(const AttnArgs& a, int32_t out_dtype, int64_t rows, const float* part,
                   int64_t n_splits, hipStream_t st) {
   const dim3 mgrid((unsigned)rows);
 #define AMF_MERGE(OUT)                                                                            \
@@ -1070,6 +944,8 @@ void launch_merge(const AttnArgs& a, int32_t out_dtype, int64_t rows, const floa
   }
 #undef AMF_MERGE
 }
+
+namespace {
 
 template <int DT, bool INT4>
 void launch_split(const AttnArgs& a, int32_t out_dtype, int64_t rows, float* part,
@@ -1160,11 +1036,10 @@ int check_attn_args(const char* who, int32_t dtype, int32_t out_dtype, int64_t b
   return ok();
 }
 
-}  // namespace
-
-extern "C" int64_t amf_dense_attn_workspace_bytes(int64_t batch, int32_t num_q_heads,
-                                                  int32_t num_kv_heads, int64_t q_len,
-                                                  int64_t kv_len, int32_t head_dim) {
+// Workspace bytes of the one-row split launch; 0 when the shape takes the
+// single-pass kernel.
+int64_t split_workspace_bytes(int64_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+                              int64_t q_len, int64_t kv_len, int32_t head_dim) {
   if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
       q_len <= 0 || kv_len <= 0 || !split_head_dim(head_dim) || batch > 0x7FFFFFFF ||
       q_len > 0x7FFFFFFF)
@@ -1177,6 +1052,31 @@ extern "C" int64_t amf_dense_attn_workspace_bytes(int64_t batch, int32_t num_q_h
   // workgroups; a shape beyond one launch takes the single-pass kernel.
   if (rows > (0x7FFFFFFF - kXcds * num_q_heads) / n_splits) return 0;
   return rows * n_splits * (int64_t)(head_dim + kPartPad) * (int64_t)sizeof(float);
+}
+
+// The many-row kernel's plan for a call with this workspace: as many splits
+// as it has room for (one split needs none).
+bool plan_prefill(const AttnArgs& a, int32_t dtype, int64_t workspace_bytes, PrefillPlan* p) {
+  if (dtype == AMF_DTYPE_F32) return false;
+  const int64_t room = std::max<int64_t>(
+      1, workspace_bytes / prefill_split_bytes(a.batch, a.num_q_heads, a.q_len, a.head_dim));
+  return prefill_plan(a.batch, a.num_q_heads, a.num_kv_heads, a.q_len, a.kv_len, a.head_dim, room,
+                      p);
+}
+
+}  // namespace
+
+extern "C" int64_t amf_dense_attn_workspace_bytes(int64_t batch, int32_t num_q_heads,
+                                                  int32_t num_kv_heads, int64_t q_len,
+                                                  int64_t kv_len, int32_t head_dim) {
+  const int64_t need =
+      split_workspace_bytes(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim);
+  PrefillPlan p;
+  if (need > 0 && prefill_plan(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim,
+                               kMaxPrefillSplits, &p) && p.n_splits > 1)
+    return std::max<int64_t>(
+        need, p.n_splits * prefill_split_bytes(batch, num_q_heads, q_len, head_dim));
+  return need;
 }
 
 extern "C" int amf_dense_attn(const void* q, const void* k, const void* v, int32_t dtype,
@@ -1203,13 +1103,18 @@ extern "C" int amf_dense_attn(const void* q, const void* k, const void* v, int32
              softmax_scale, nullptr, nullptr};
   hipStream_t st = as_stream(stream);
   const int64_t need =
-      amf_dense_attn_workspace_bytes(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim);
+      split_workspace_bytes(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim);
   if (need > 0 && vec8 && ((uintptr_t)q % 16) == 0 && workspace && workspace_bytes >= need &&
       ((uintptr_t)workspace % 16) == 0) {
+    float* part = static_cast<float*>(workspace);
+    PrefillPlan plan;
+    if (plan_prefill(a, dtype, workspace_bytes, &plan)) {
+      launch_prefill(a, dtype, out_dtype, false, part, plan, st);
+      return check_launch(who);
+    }
     int64_t n_splits = 1, split_tokens = 64;
     dense_splits(rows, heads_per_wave(num_q_heads, num_kv_heads), kv_len, &n_splits,
                  &split_tokens);
-    float* part = static_cast<float*>(workspace);
     if (dtype == AMF_DTYPE_F32)
       launch_split<AMF_DTYPE_F32, false>(a, out_dtype, rows, part, split_tokens, n_splits, st);
     else if (dtype == AMF_DTYPE_BF16)
@@ -1265,7 +1170,7 @@ extern "C" int amf_int4_sym_dense_attn(const void* q, int32_t dtype, const void*
     return check_launch(who);
   }
   const int64_t need =
-      amf_dense_attn_workspace_bytes(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim);
+      split_workspace_bytes(batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim);
   if (need == 0)
     return fail(AMF_ERR_UNSUPPORTED, "%s: %lld query rows exceed one launch", who,
                 (long long)rows);
@@ -1279,6 +1184,11 @@ extern "C" int amf_int4_sym_dense_attn(const void* q, int32_t dtype, const void*
   // the MFMA kernel addresses a (batch, KV head) row of codes with 32-bit offsets
   const bool mfma = head_dim == 128 && !mask && dtype != AMF_DTYPE_F32 &&
                     kv_len < ((int64_t)1 << 32) / 64;
+  PrefillPlan plan;
+  if (!mfma && plan_prefill(a, dtype, workspace_bytes, &plan)) {
+    launch_prefill(a, dtype, out_dtype, true, part, plan, st);
+    return check_launch(who);
+  }
   if (mfma && dtype == AMF_DTYPE_BF16)
     launch_int4_mfma<AMF_DTYPE_BF16>(a, out_dtype, rows, part, split_tokens, n_splits, st);
   else if (mfma)

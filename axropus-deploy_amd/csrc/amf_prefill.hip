@@ -1,0 +1,445 @@
+// amf_prefill.hip - dense attention of many query rows (chunked prefill,
+// verification of drafted tokens) on MFMA tiles: the q_len > 1 form of
+// amf_dense_attn and of the masked / head_dim 64 and 256 forms of
+// amf_int4_sym_dense_attn, for bf16 and fp16.
+//
+// The query rows of one (batch, KV head) - its GQA group's heads times q_len
+// - are the columns of 32x32x16 tiles, so each K/V tile staged in LDS serves
+// 32 rows per wave.  The scores are formed transposed, S^T = K Q^T: a lane
+// then holds one query row (column lane % 32) with 16 tokens of a 32-token
+// tile, the softmax statistics of a row are per-lane scalars (one exchange
+// with lane ^ 32 for the maximum), and the weights are already in the
+// B-operand layout of O^T = V^T P^T, whose k slots take the tokens in the
+// order the scores leave them.  V^T comes out of LDS through the transposing
+// read (ds_read_b64_tr_b16).
+//
+// Precision.  The bf16 / fp16 products of Q and K are exact and summed in
+// fp32, as the one-row kernel's v_dot2 does.  The softmax weights are fp32
+// and enter the PV tiles as a sum of 16-bit terms: three bf16 terms hold an
+// fp32 weight exactly, two fp16 terms (scaled by 2^15) hold it to 22 bits of
+// itself and 2^-38 of the row's largest.  Accumulators, maxima and sums are
+// fp32.  (Two bf16 terms would take 103 instead of 114 us at 32 / 8 heads, 512
+// rows, 4096 tokens, but are 16 bits.)
+#include <algorithm>
+
+#include "amf_attn.h"
+#include "amf_prefill.h"
+
+namespace {
+
+using namespace amf;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef s16x4 __attribute__((address_space(3))) lds_s16x4;
+
+template <int DT>
+__device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
+  if constexpr (DT == AMF_DTYPE_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+// Tokens of a staged tile: 64, or 32 where 64 rows would take too much LDS
+// (head_dim 256) or too many registers in flight per lane (one wave).
+constexpr int tile_tokens(int D, int NW) { return D == 256 || NW == 1 ? 32 : 64; }
+
+// LDS row strides in bytes.  K rows are read as 16-byte vectors of 32
+// consecutive rows: 16 more than the row moves each by 4 banks.  V rows are
+// read by the transposing read, 4 rows of 64 bytes per half wave: 64 more
+// than the row puts them 16 banks apart.
+constexpr int k_stride(int D) { return 2 * D + 16; }
+constexpr int v_stride(int D) { return 2 * D + 64; }
+
+// 16-bit terms of a softmax weight.
+template <int DT>
+constexpr int weight_terms() {
+  return DT == AMF_DTYPE_BF16 ? 3 : 2;
+}
+// The fp16 weights carry 2^15, so that their low terms stay representable.
+template <int DT>
+constexpr float weight_shift() {
+  return DT == AMF_DTYPE_F16 ? 15.0f : 0.0f;
+}
+
+// Terms of the weights p0 and p1 (low and high half of each word).  A positive
+// weight has only positive terms, a zero one only zeros: inf in V then gives
+// inf under a positive weight (mixed signs or a zero term would make it NaN)
+// and NaN under a zero one, as the product with the weight itself does.  Each
+// bf16 term is the top half of the bit pattern below the remainder's, so the
+// next remainder is positive and exact and the third fits 8 bits; fp16 terms
+// are rounded toward zero from below and raised to the least subnormal.
+template <int DT>
+__device__ __forceinline__ void weight_split(float p0, float p1,
+                                             uint32_t (&w)[weight_terms<DT>()]) {
+  if constexpr (DT == AMF_DTYPE_BF16) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t a = __builtin_elementwise_sub_sat(f2u(p0), 1u) & 0xFFFF0000u;
+      const uint32_t b = __builtin_elementwise_sub_sat(f2u(p1), 1u) & 0xFFFF0000u;
+      w[k] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+      p0 -= u2f(a);
+      p1 -= u2f(b);
+    }
+    w[2] = __builtin_amdgcn_perm(f2u(p1), f2u(p0), 0x07060302u);
+  } else {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 least = __builtin_bit_cast(u16x2, min(f2u(p0), 1u) | (min(f2u(p1), 1u) << 16));
+    auto raised = [&](uint32_t x) {
+      return __builtin_bit_cast(
+          uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), least));
+    };
+    w[0] = raised(__builtin_bit_cast(
+        uint32_t,
+        __builtin_amdgcn_cvt_pkrtz(u2f(__builtin_elementwise_sub_sat(f2u(p0), 1u)),
+                                   u2f(__builtin_elementwise_sub_sat(f2u(p1), 1u)))));
+    p0 = fmaxf(p0 - half_lo<false>(w[0]), 0.0f);
+    p1 = fmaxf(p1 - half_hi<false>(w[0]), 0.0f);
+    w[1] = raised(pack2<false>(p0, p1));
+  }
+}
+
+// Measured (bf16, 32 / 8 heads, head_dim 128, causal mask): 512 rows x 4096
+// tokens 1285 -> 111 us (25 -> 290 TFLOP/s), 128 rows x 8192 tokens 913 ->
+// 67 us; the one-row kernel ran every row's products on the VALU and read
+// K/V from L2 once per row.  Now bound by the chain staging -> scores ->
+// softmax -> PV of two waves per SIMD (254 VGPRs), not by the MFMAs (27 us).
+//
+// NW waves of 32 query rows each share the K/V tiles.  Unit u is (b, KV head, split), served by `tiles`
+// workgroups; with xcd_map they take consecutive slots of one XCD (its L2
+// holds the unit's K/V), else they are consecutive workgroups.
+template <int DT, int D, int NW, bool INT4>
+__global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
+    AttnArgs a, int out_dtype, float* part, int64_t split_tokens, int64_t n_splits, int64_t units,
+    int tiles, bool xcd_map) {
+  constexpr int BT = tile_tokens(D, NW), KS = k_stride(D), VS = v_stride(D);
+  constexpr int LPR = D / 8;                     // 16-byte chunks per K/V row
+  constexpr int CH = BT * LPR / (64 * NW);       // chunks per lane of a tile
+  constexpr int RSTEP = 64 * NW / LPR;           // rows between a lane's chunks
+  static_assert(CH >= 1 && (64 * NW) % LPR == 0, "a tile is whole chunks per lane");
+  constexpr int TERMS = weight_terms<DT>();
+  using Raw = RawRow<DT, INT4>;
+  __shared__ __attribute__((aligned(16))) uint8_t k_lds[BT * KS];
+  __shared__ __attribute__((aligned(16))) uint8_t v_lds[BT * VS];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lc = lane & 31, h = lane >> 5;
+  const int64_t id = blockIdx.x;
+  int64_t u;
+  int tile;
+  if (xcd_map) {
+    const int64_t slot = id / kXcds;
+    tile = (int)(slot % tiles);
+    u = (slot / tiles) * kXcds + id % kXcds;
+  } else {
+    tile = (int)(id % tiles);
+    u = id / tiles;
+  }
+  if (u >= units) return;
+  const int64_t split = u % n_splits, bkv = u / n_splits;
+  const int hkv = (int)(bkv % a.num_kv_heads);
+  const int64_t b = bkv / a.num_kv_heads;
+  const int G = a.num_q_heads / a.num_kv_heads;
+  const int64_t T = a.kv_len;
+  const int64_t t_begin = split * split_tokens, t_end = min(T, t_begin + split_tokens);
+  const int64_t kv_base = (b * a.num_kv_heads + hkv) * T;
+
+  // This lane's query row: rows run over (query token, head of the group),
+  // head fastest, so the lanes of a wave share mask rows.
+  const int64_t M = (int64_t)G * a.q_len;
+  const int64_t row = ((int64_t)tile * NW + wave) * 32 + lc;
+  const bool row_ok = row < M;
+  const int64_t tq = (row_ok ? row : 0) / G;
+  const int head = hkv * G + (int)((row_ok ? row : 0) % G);
+  const int64_t qrow = (b * a.num_q_heads + head) * a.q_len + tq;
+  u32x4 qb[D / 16];  // B operand: dims 16 ks + 8 h .. + 7
+  {
+    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + qrow * D + 8 * h;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) qb[ks] = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
+  }
+  const float qs = a.scale * kLog2e;
+  const float* mrow = a.mask ? a.mask + b * a.ms0 + (int64_t)head * a.ms1 + tq * a.ms2 : nullptr;
+  // four mask values at once where every group of four tokens is aligned and
+  // lies inside or outside the row as a whole
+  const bool mvec = a.ms3 == 1 && T % 4 == 0 && (reinterpret_cast<uintptr_t>(a.mask) & 15) == 0 &&
+                    ((a.ms0 | a.ms1 | a.ms2) & 3) == 0;
+
+  // staging: chunk (row r0 + RSTEP i, dims 8 c ..) of the tile
+  const int c = tid % LPR, r0 = tid / LPR;
+  float ksc[8], kz[8], vsc[8], vz[8];
+  if constexpr (INT4) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      ksc[e] = (float)a.k_scales[8 * c + e];
+      vsc[e] = (float)a.v_scales[8 * c + e];
+      kz[e] = -8.0f * ksc[e];
+      vz[e] = -8.0f * vsc[e];
+    }
+  }
+  Raw kr[CH], vr[CH];
+  auto fetch = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int64_t t = t0 + r0 + RSTEP * i;
+      kr[i] = Raw::load(a.k, kv_base + (t < t_end ? t : t_begin), c, D);
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int64_t t = t0 + r0 + RSTEP * i;
+      vr[i] = Raw::load(a.v, kv_base + (t < t_end ? t : t_begin), c, D);
+    }
+  };
+  // rows past the split are zeros (their scores are -inf below)
+  auto stage = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int r = r0 + RSTEP * i;
+      const bool in = t0 + r < t_end;
+      uint32_t kp[4], vp[4];
+      kr[i].pairs(ksc, kz, kp);
+      vr[i].pairs(vsc, vz, vp);
+      *reinterpret_cast<u32x4*>(k_lds + r * KS + 16 * c) =
+          in ? u32x4{kp[0], kp[1], kp[2], kp[3]} : u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) =
+          in ? u32x4{vp[0], vp[1], vp[2], vp[3]} : u32x4{0, 0, 0, 0};
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.0f;  // l_run: this lane's tokens
+  f32x16 acc[D / 32];
+#pragma unroll
+  for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[d][i] = 0.0f;
+
+  // addresses of this lane's LDS reads
+  const uint8_t* k_rd = k_lds + lc * KS + 16 * h;
+  const int l16 = lane & 15;
+  const uint8_t* v_rd = v_lds + (4 * h + (l16 >> 2)) * VS + 32 * ((lane >> 4) & 1) + 8 * (l16 & 3);
+
+  fetch(t_begin);
+  for (int64_t t0 = t_begin; t0 < t_end; t0 += BT) {
+    __syncthreads();  // the previous tile has been read
+    stage(t0);
+    __syncthreads();
+    // token of score element i of block tb: t0 + 32 tb + 8 (i / 4) + 4 h + i % 4
+    f32x4 mk[BT / 32][4];
+    if (mrow) {
+#pragma unroll
+      for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int64_t t = t0 + 32 * tb + 8 * g + 4 * h;
+          if (mvec) {
+            mk[tb][g] = *reinterpret_cast<const f32x4*>(mrow + (t < t_end ? t : t_begin));
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              mk[tb][g][e] = mrow[(t + e < t_end ? t + e : t_begin) * a.ms3];
+          }
+        }
+    }
+    if (t0 + BT < t_end) fetch(t0 + BT);
+
+    f32x16 s[BT / 32];
+#pragma unroll
+    for (int tb = 0; tb < BT / 32; ++tb) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[tb][i] = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks)
+        s[tb] = mfma32<DT>(*reinterpret_cast<const u32x4*>(k_rd + 32 * tb * KS + 32 * ks), qb[ks],
+                           s[tb]);
+    }
+    const bool full = t0 + BT <= t_end;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float x = s[tb][i] * qs;
+        if (mrow) x = fmaf(mk[tb][i >> 2][i & 3], kLog2e, x);
+        if (!full && t0 + 32 * tb + 8 * (i >> 2) + 4 * h + (i & 3) >= t_end) x = -INFINITY;
+        s[tb][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx);
+    // a row with every score so far -inf keeps l = 0 and acc = 0
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    if (__any(m_new > m_run)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
+    }
+    m_run = m_new;
+    const float m_sub = m_use - weight_shift<DT>();
+
+#pragma unroll
+    for (int st = 0; st < BT / 16; ++st) {
+      // weights of the step's 16 tokens in 16-bit terms, 8 per lane
+      u32x4 pb[TERMS];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float p0 = __builtin_amdgcn_exp2f(s[st >> 1][8 * (st & 1) + 2 * j] - m_sub);
+        const float p1 = __builtin_amdgcn_exp2f(s[st >> 1][8 * (st & 1) + 2 * j + 1] - m_sub);
+        l_run += p0;
+        l_run += p1;
+        uint32_t w[TERMS];
+        weight_split<DT>(p0, p1, w);
+#pragma unroll
+        for (int k = 0; k < TERMS; ++k) pb[k][j] = w[k];
+      }
+#pragma unroll
+      for (int d = 0; d < D / 32; ++d) {
+        const uint8_t* vp = v_rd + 16 * st * VS + 64 * d;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 8 * VS));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        const u32x4 va = {l2[0], l2[1], h2[0], h2[1]};
+#pragma unroll
+        for (int k = 0; k < TERMS; ++k) acc[d] = mfma32<DT>(va, pb[k], acc[d]);
+      }
+    }
+  }
+
+  const float l = l_run + __shfl_xor(l_run, 32);
+  if (!row_ok) return;
+  if (n_splits == 1) {
+    // a row whose scores are all -inf: 0 / 0 = NaN, as softmax gives
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int64_t o = qrow * D + 32 * d + 8 * g + 4 * h;
+        const f32x4 x = {acc[d][4 * g] / l, acc[d][4 * g + 1] / l, acc[d][4 * g + 2] / l,
+                         acc[d][4 * g + 3] / l};
+        store4(a.out, out_dtype, o, x);
+      }
+  } else {
+    float* pr = part + (qrow * n_splits + split) * (int64_t)(D + kPartPad);
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(pr + 32 * d + 8 * g + 4 * h) =
+            f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
+    if (h == 0) {
+      pr[D] = m_run;
+      pr[D + 1] = l;
+    }
+  }
+}
+
+constexpr int kFewSplits = 8;
+
+// out = sum_k 2^(m_k - M) acc_k / sum_k 2^(m_k - M) l_k over a row's splits,
+// one lane per four dims, each reading every (m, l) of its row itself: for up
+// to kFewSplits splits; more go to the one-row kernel's merge (a workgroup
+// per row).
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(void* out, int out_dtype, int64_t rows,
+                                                            const float* part, int n_splits) {
+  constexpr int Q = D / 4;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / Q;
+  const int quad = (int)(i % Q);
+  if (row >= rows) return;
+  const float* pr = part + row * n_splits * (int64_t)(D + kPartPad);
+  float M = -INFINITY;
+  for (int k = 0; k < n_splits; ++k) M = fmaxf(M, pr[k * (D + kPartPad) + D]);
+  float den = 0.0f;
+  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k = 0; k < n_splits; ++k) {
+    const float* p = pr + k * (D + kPartPad);
+    const float m = p[D];
+    const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+    den = fmaf(p[D + 1], f, den);
+    const f32x4 x = *reinterpret_cast<const f32x4*>(p + 4 * quad);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = fmaf(x[e], f, o[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = o[e] / den;
+  store4(out, out_dtype, row * D + 4 * quad, o);
+}
+
+template <int DT, int D, int NW, bool INT4>
+void launch_one(const AttnArgs& a, int32_t out_dtype, float* part, const PrefillPlan& p,
+                hipStream_t st) {
+  const int64_t units = a.batch * a.num_kv_heads * p.n_splits;
+  const bool xcd = units % kXcds == 0;
+  const dim3 grid((unsigned)(units * p.tiles));
+  prefill_attn_kernel<DT, D, NW, INT4><<<grid, 64 * NW, 0, st>>>(
+      a, out_dtype, part, p.split_tokens, p.n_splits, units, (int)p.tiles, xcd);
+  const int64_t rows = a.batch * a.num_q_heads * a.q_len;
+  if (p.n_splits > kFewSplits) {
+    launch_merge(a, out_dtype, rows, part, p.n_splits, st);
+  } else if (p.n_splits > 1) {
+    prefill_merge_kernel<D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), 256, 0, st>>>(
+        a.out, out_dtype, rows, part, (int)p.n_splits);
+  }
+}
+
+template <int DT, bool INT4>
+void launch_shape(const AttnArgs& a, int32_t out_dtype, float* part, const PrefillPlan& p,
+                  hipStream_t st) {
+#define AMF_PREFILL(DD)                                                           \
+  (p.waves == 1 ? launch_one<DT, DD, 1, INT4>(a, out_dtype, part, p, st)   \
+                : launch_one<DT, DD, 4, INT4>(a, out_dtype, part, p, st))
+  if (a.head_dim == 64)
+    AMF_PREFILL(64);
+  else if (a.head_dim == 128)
+    AMF_PREFILL(128);
+  else
+    AMF_PREFILL(256);
+#undef AMF_PREFILL
+}
+
+}  // namespace
+
+namespace amf {
+
+bool prefill_plan(int64_t batch, int32_t num_q_heads, int32_t num_kv_heads, int64_t q_len,
+                  int64_t kv_len, int32_t head_dim, int64_t max_splits, PrefillPlan* p) {
+  const int64_t M = (int64_t)(num_q_heads / num_kv_heads) * q_len;
+  if (q_len < 2 || M < kPrefillMinRows || !split_head_dim(head_dim)) return false;
+  p->waves = M <= 32 ? 1 : 4;
+  p->tiles = (M + 32 * p->waves - 1) / (32 * p->waves);
+  const int64_t base = batch * num_kv_heads * p->tiles;
+  const int64_t want = p->waves == 1 ? kPrefillGroups1 : kPrefillGroups4;
+  const int64_t chunks = (kv_len + 63) / 64;
+  int64_t n = (want + base - 1) / base;
+  const int64_t mc = p->waves == 1 ? kPrefillMinChunks1 : kPrefillMinChunks4;
+  n = std::min<int64_t>(n, (chunks + mc - 1) / mc);
+  n = std::max<int64_t>(1, std::min<int64_t>({n, max_splits, kMaxPrefillSplits}));
+  const int64_t per = (chunks + n - 1) / n;
+  p->split_tokens = per * 64;
+  p->n_splits = (chunks + per - 1) / per;
+  return base <= (0x7FFFFFFF) / p->n_splits;
+}
+
+int64_t prefill_split_bytes(int64_t batch, int32_t num_q_heads, int64_t q_len, int32_t head_dim) {
+  return batch * num_q_heads * q_len * (int64_t)(head_dim + kPartPad) * (int64_t)sizeof(float);
+}
+
+void launch_prefill(const AttnArgs& a, int32_t dtype, int32_t out_dtype, bool int4, float* part,
+                    const PrefillPlan& p, hipStream_t st) {
+  if (dtype == AMF_DTYPE_BF16)
+    int4 ? launch_shape<AMF_DTYPE_BF16, true>(a, out_dtype, part, p, st)
+         : launch_shape<AMF_DTYPE_BF16, false>(a, out_dtype, part, p, st);
+  else
+    int4 ? launch_shape<AMF_DTYPE_F16, true>(a, out_dtype, part, p, st)
+         : launch_shape<AMF_DTYPE_F16, false>(a, out_dtype, part, p, st);
+}
+
+}  // namespace amf

@@ -345,8 +345,9 @@ uint64_t amf_hash_tokens(const int32_t* tokens, int64_t n_tokens);
  * holds amf_dense_attn_workspace_bytes(...) bytes (non-zero only for
  * head_dim 64, 128 or 256 and kv_len > 0) and q, k, v are 16-byte aligned,
  * the KV tokens of each row are split over many waves (flash decoding) and
- * merged by a second launch; otherwise (NULL, too small) one workgroup per
- * query row runs the whole row.  Both give the same result to fp32 rounding.
+ * merged by a second launch (for bf16 / fp16 and q_len > 1 on MFMA tiles of
+ * query rows); otherwise (NULL, too small) one workgroup per query row runs
+ * the whole row.  All give the same result to fp32 rounding.
  * Calls sharing a workspace must be ordered on one stream.
  * Replaces the attention of fallback_fp16_kernel (kernels/dispatch.py:117-143),
  * which int4_decode_attention (int4_decode_attention.py:6-9) reaches for k/v
