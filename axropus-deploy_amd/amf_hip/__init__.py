@@ -107,6 +107,21 @@ SIGNATURES = {
         [_c_i32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_ptr, _c_i64, _c_i32, _c_i64, _c_i32,
          _c_i32, _c_i32, _c_ptr, _c_ptr],
     ),
+    "amf_int4_quant_gather_slots": (
+        _c_i32,
+        [_c_i32, _c_ptr, _c_i64, _c_i32, _c_i32, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i32, _c_i64,
+         _c_i32, _c_i32, _c_i32, _c_ptr, _c_ptr],
+    ),
+    "amf_fp8_dequant_scatter_slots": (
+        _c_i32,
+        [_c_i32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_i32, _c_ptr, _c_i64, _c_i32, _c_i64,
+         _c_i32, _c_i32, _c_i32, _c_ptr, _c_ptr],
+    ),
+    "amf_int4_dequant_scatter_slots": (
+        _c_i32,
+        [_c_i32, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_i32, _c_ptr, _c_i64, _c_i32, _c_i64,
+         _c_i32, _c_i32, _c_i32, _c_ptr, _c_ptr],
+    ),
     "amf_int4_decode_workspace_bytes": (_c_i64, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),
     "amf_int4_paged_decode_attn": (
         _c_i32,

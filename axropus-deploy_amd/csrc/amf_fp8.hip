@@ -62,27 +62,34 @@ constexpr int dtype_of() {
 // cache elements out), so each wave-wide store covers 1 KiB contiguously and
 // every cache line is written whole.  The chunk's head is fixed per lane when
 // 2048 elements (one workgroup pass) span whole rows of heads.
-template <int DT, bool PER_TENSOR>
+// SLOTS: the rows go to the cache rows of the tokens' slots.
+template <int DT, bool PER_TENSOR, bool SLOTS>
 __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
     const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
-    PageGeom g, int32_t* err_flag) {
+    PageGeom g, SlotRows rows, int32_t* err_flag) {
+  __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
   const PageWork pw = xcd_page_work(n_pages, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j;
   const int plane = pw.plane;
-  const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
-  if (dp < 0 || dp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
-    return;
+  uint8_t* __restrict__ out = reinterpret_cast<uint8_t*>(cache_planes[plane]);
+  if constexpr (SLOTS) {
+    slot_row_offsets(rows, j, s_row, err_flag);
+  } else {
+    const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
+    if (dp < 0 || dp >= pool) {
+      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      return;
+    }
+    out += dp * cache_stride;
   }
   const int page_elems = g.n_rows * g.head_dim;
   const int n8 = page_elems >> 3;
   const uint8_t* __restrict__ codes =
       reinterpret_cast<const uint8_t*>(code_planes[plane]) + j * (int64_t)page_elems;
   const float* __restrict__ params = reinterpret_cast<const float*>(param_planes[plane]);
-  uint8_t* __restrict__ out = reinterpret_cast<uint8_t*>(cache_planes[plane]) + dp * cache_stride;
   const float* __restrict__ page_scales = params + j * g.num_heads;
   const int tid = threadIdx.x;
   float s_fixed = 0.0f;
@@ -91,6 +98,7 @@ __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
   else if (g.head_const)
     s_fixed = page_scales[((tid * 8) / g.head_dim) % g.num_heads];
 
+  const uint32_t cpt = SLOTS ? (uint32_t)n8 / (uint32_t)rows.page_tokens : 1;  // chunks per row
   constexpr int U = AMF_RESTORE_UNROLL;
   for (int base = tid; base < n8; base += U * kThreads) {
     u32x2 c[U];
@@ -111,7 +119,13 @@ __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
         e4m3x4_to_f32(c[u][1], x + 4);
 #pragma unroll
         for (int q = 0; q < 8; ++q) x[q] = x[q] * s;
-        store8<DT>(out + (int64_t)k * (8 * elem_bytes<DT>()), x);
+        if constexpr (SLOTS) {
+          const uint32_t t = (uint32_t)k / cpt;
+          const int64_t off = s_row[t];
+          if (off >= 0) store8<DT>(out + off + (k - t * cpt) * (8 * elem_bytes<DT>()), x);
+        } else {
+          store8<DT>(out + (int64_t)k * (8 * elem_bytes<DT>()), x);
+        }
       }
     }
   }
@@ -693,6 +707,24 @@ const void* coop_kernel(int dt, int cpt) {
 #undef AMF_COOP
 }
 
+template <bool SLOTS>
+void launch_restore(int32_t format, int64_t n_pages, hipStream_t s, const uint64_t* code_planes,
+                    const uint64_t* param_planes, const uint64_t* cache_planes,
+                    int64_t cache_stride, int32_t cache_dtype, const int32_t* block_ids,
+                    int64_t pool, int32_t n_planes, const PageGeom& g, const SlotRows& rows,
+                    int32_t* err_flag) {
+  const dim3 grid = xcd_page_grid(n_pages, n_planes);
+  const bool pt = format == AMF_FMT_FP8_E4M3;
+  // the slot form's row table counts towards the pad
+  const unsigned pad = kRestoreLdsPad - (SLOTS ? kMaxSlotPage * sizeof(int64_t) : 0);
+#define AMF_LAUNCH(T)                                                                        \
+  fp8_dequant_scatter_kernel<DT, T, SLOTS><<<grid, kThreads, pad, s>>>(                      \
+      code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,       \
+      n_planes, g, rows, err_flag)
+  AMF_WITH_DTYPE(cache_dtype, if (pt) AMF_LAUNCH(true); else AMF_LAUNCH(false));
+#undef AMF_LAUNCH
+}
+
 constexpr int kCoopNotTaken = 1;
 
 // Per-tensor save through fp8_tensor_coop_kernel when the device supports a
@@ -773,15 +805,36 @@ extern "C" int amf_fp8_dequant_scatter(int32_t format, const uint64_t* code_plan
   if (n_pages * n_planes > 0x7FFFFFF0ll)
     return fail(AMF_ERR_UNSUPPORTED, "%s: %lld pages x %d planes exceed one launch", who,
                 (long long)n_pages, n_planes);
-  const dim3 grid = xcd_page_grid(n_pages, n_planes);
-  hipStream_t s = as_stream(stream);
-  const bool pt = format == AMF_FMT_FP8_E4M3;
-#define AMF_LAUNCH(T)                                                                       \
-  fp8_dequant_scatter_kernel<DT, T><<<grid, kThreads, kRestoreLdsPad, s>>>(                 \
-      code_planes, param_planes, cache_planes, cache_page_stride, block_ids, pool_pages,     \
-      n_pages, n_planes, g, err_flag)
-  AMF_WITH_DTYPE(cache_dtype, if (pt) AMF_LAUNCH(true); else AMF_LAUNCH(false));
-#undef AMF_LAUNCH
+  launch_restore<false>(format, n_pages, as_stream(stream), code_planes, param_planes,
+                        cache_planes, cache_page_stride, cache_dtype, block_ids, pool_pages,
+                        n_planes, g, SlotRows{}, err_flag);
+  return check_launch(who);
+}
+
+extern "C" int amf_fp8_dequant_scatter_slots(
+    int32_t format, const uint64_t* code_planes, const uint64_t* param_planes,
+    const uint64_t* cache_planes, int64_t cache_page_stride, int32_t cache_block,
+    int32_t cache_dtype, const int64_t* slot_mapping, int64_t pool_slots, int32_t n_planes,
+    int64_t n_slots, int32_t page_tokens, int32_t num_heads, int32_t head_dim, int32_t* err_flag,
+    void* stream) {
+  const char* who = "amf_fp8_dequant_scatter_slots";
+  if (format != AMF_FMT_FP8_E4M3 && format != AMF_FMT_FP8_E4M3_PH)
+    return fail(AMF_ERR_INVALID_ARG, "%s: format %d is not an FP8 format", who, format);
+  SlotRows rows;
+  int64_t n_pages = 0;
+  int rc = check_slot_codec(who, cache_planes, cache_page_stride, cache_block, cache_dtype,
+                            slot_mapping, pool_slots, code_planes, param_planes, n_planes,
+                            n_slots, page_tokens, num_heads, head_dim, &rows, &n_pages);
+  if (rc) return rc;
+  PageGeom g;
+  if ((rc = make_geom(who, page_tokens, num_heads, head_dim, 1, &g))) return rc;
+  if (n_pages == 0) return ok();
+  if (n_pages * n_planes > 0x7FFFFFF0ll)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: %lld pages x %d planes exceed one launch", who,
+                (long long)n_pages, n_planes);
+  launch_restore<true>(format, n_pages, as_stream(stream), code_planes, param_planes,
+                       cache_planes, cache_page_stride, cache_dtype, nullptr, 0, n_planes, g,
+                       rows, err_flag);
   return check_launch(who);
 }
 

@@ -58,21 +58,29 @@ __device__ __forceinline__ void load32(const uint8_t* p, float* x) {
 // wave-wide stores cover 1 KiB contiguously.  A page of more than 8 passes
 // of the workgroup is cut into `parts` workgroups of whole passes (a dense
 // tensor's page can hold millions of elements).
-template <int DT, bool CHANNEL>
+// SLOTS: the rows go to the cache rows of the tokens' slots.
+template <int DT, bool CHANNEL, bool SLOTS>
 __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
     const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
-    int parts, SymGeom g, int32_t* err_flag) {
+    int parts, SymGeom g, SlotRows rows, int32_t* err_flag) {
+  __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
   const PageWork pw = xcd_page_work(n_pages * parts, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j / parts;
   const int part = (int)(pw.j % parts);
   const int plane = pw.plane;
-  const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
-  if (dp < 0 || dp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
-    return;
+  uint8_t* __restrict__ out = reinterpret_cast<uint8_t*>(cache_planes[plane]);
+  if constexpr (SLOTS) {
+    slot_row_offsets(rows, j, s_row, err_flag);
+  } else {
+    const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
+    if (dp < 0 || dp >= pool) {
+      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      return;
+    }
+    out += dp * cache_stride;
   }
   const int page_elems = g.n_rows * g.head_dim;
   const int n8 = page_elems >> 3;
@@ -83,7 +91,6 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
   const uint32_t* __restrict__ codes =
       reinterpret_cast<const uint32_t*>(code_planes[plane]) + j * (int64_t)n8;
   const _Float16* __restrict__ params = reinterpret_cast<const _Float16*>(param_planes[plane]);
-  uint8_t* __restrict__ out = reinterpret_cast<uint8_t*>(cache_planes[plane]) + dp * cache_stride;
   const int tid = threadIdx.x;
   const float s_page = CHANNEL ? 0.0f : (float)params[j];
   // Channel scales of this lane's 8 dims; fixed while 8 * kThreads is a
@@ -94,6 +101,7 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
 #pragma unroll
     for (int q = 0; q < 8; ++q) s_ch[q] = (float)params[d0 + q];
   }
+  const uint32_t cpt = SLOTS ? (uint32_t)n8 / (uint32_t)rows.page_tokens : 1;  // chunks per row
   constexpr int U = AMF_SYM_RESTORE_UNROLL;
   for (int base = k_begin + tid; base < k_end; base += U * kThreads) {
     uint32_t c[U];
@@ -109,44 +117,80 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
         float x[8];
 #pragma unroll
         for (int n = 0; n < 8; ++n) x[n] = (nib(c[u], n) - 8.0f) * (CHANNEL ? s_ch[n] : s_page);
-        store8<DT>(out + (int64_t)k * (8 * elem_bytes<DT>()), x);
+        if constexpr (SLOTS) {
+          const uint32_t t = (uint32_t)k / cpt;
+          const int64_t off = s_row[t];
+          if (off >= 0) store8<DT>(out + off + (k - t * cpt) * (8 * elem_bytes<DT>()), x);
+        } else {
+          store8<DT>(out + (int64_t)k * (8 * elem_bytes<DT>()), x);
+        }
       }
     }
   }
 }
 
+constexpr int kBigThreads = 1024;
+
 // INT4_SYM_BLOCK save: page absmax -> scale -> codes; the page stays in
-// registers.  One lane = CPL 8-element chunks kThreads apart, so each load
+// registers.  One lane = CPL 8-element chunks NT apart, so each load
 // instruction of a wave covers 1 KiB of whole lines (non-temporal: read once)
-// and each code store 256 contiguous bytes.
-template <bool BF16, int CPL>
-__global__ __launch_bounds__(kThreads) void int4_symblock_quant_gather_kernel(
+// and each code store 256 contiguous bytes.  A lane holds at most 8 chunks up
+// to pages of 8192 chunks (at most 64 VGPRs: two workgroups of 1024 lanes a
+// CU, so that one loads while the other quantizes) and 16 up to 16384, a
+// dense entry's block of 128 tokens x 8 heads x 128 dims.  64 planes, bf16,
+// before (256 lanes: 32 chunks a lane up to 8192, two reads beyond) and now:
+// 32 blocks of 8 heads 225 -> 144 us (4.66 TB/s), 64 blocks of 4 heads 198 ->
+// 108 us (6.19 TB/s); one layer's 64 blocks of 8 heads 39 -> 16 us.
+// SLOTS: the page's rows are cache rows named by token slots (zeros past the
+// sequence's end), read in place instead of from a gathered copy.
+template <bool BF16, int CPL, int NT, bool SLOTS>
+__global__ __launch_bounds__(NT, NT > kThreads && CPL <= 8 ? 8 : 1) void
+int4_symblock_quant_gather_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    const uint64_t* __restrict__ param_planes, SymGeom g, int32_t* err_flag) {
+    const uint64_t* __restrict__ param_planes, SymGeom g, SlotRows rows, int32_t* err_flag) {
   const int64_t j = blockIdx.x;
   const int plane = blockIdx.y;
-  const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
-  if (sp < 0 || sp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
-    return;
-  }
+  __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
   const int n8 = (int)((int64_t)g.n_rows * g.head_dim / 8);
-  const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(
-      reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride);
+  const uint8_t* __restrict__ src = reinterpret_cast<const uint8_t*>(cache_planes[plane]);
+  if constexpr (SLOTS) {
+    slot_row_offsets(rows, j, s_row, err_flag);
+  } else {
+    const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
+    if (sp < 0 || sp >= pool) {
+      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      return;
+    }
+    src += sp * cache_stride;
+  }
   uint32_t* __restrict__ codes = reinterpret_cast<uint32_t*>(code_planes[plane]) + j * n8;
   _Float16* __restrict__ params = reinterpret_cast<_Float16*>(param_planes[plane]);
 
   u32x4 v[CPL];
+  if constexpr (SLOTS) {
+    const uint32_t cpt = (uint32_t)n8 / (uint32_t)rows.page_tokens;  // chunks per token row
 #pragma unroll
-  for (int i = 0; i < CPL; ++i) {
-    const int k = threadIdx.x + i * kThreads;
-    if (k < n8) v[i] = ld_stream(src + k);
+    for (int i = 0; i < CPL; ++i) {
+      const uint32_t k = threadIdx.x + i * NT;
+      v[i] = u32x4{0, 0, 0, 0};
+      if (k < (uint32_t)n8) {
+        const uint32_t t = k / cpt;
+        const int64_t off = s_row[t];
+        if (off >= 0) v[i] = ld_stream(reinterpret_cast<const u32x4*>(src + off) + (k - t * cpt));
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      const int k = threadIdx.x + i * NT;
+      if (k < n8) v[i] = ld_stream(reinterpret_cast<const u32x4*>(src) + k);
+    }
   }
   float m = 0.0f;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    if (threadIdx.x + i * kThreads < n8) {
+    if (threadIdx.x + i * NT < n8) {
       float x[8];
       unpack8<BF16>(v[i], x);
 #pragma unroll
@@ -154,44 +198,53 @@ __global__ __launch_bounds__(kThreads) void int4_symblock_quant_gather_kernel(
     }
   }
   m = wave_max_xor(m, 64);
-  __shared__ float s_wmax[kThreads / 64];
+  __shared__ float s_wmax[NT / 64];
   if ((threadIdx.x & 63) == 0) s_wmax[threadIdx.x >> 6] = m;
   __syncthreads();
   float amax = s_wmax[0];
 #pragma unroll
-  for (int w = 1; w < kThreads / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
+  for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
   // amf_codec.py:392-394: absmax.clamp_min(1e-8) / 7 in fp32.
   const float scale = fmaxf(amax, 1e-8f) / kSymMax;
   const float rscale = 1.0f / scale;
   if (threadIdx.x == 0) params[j] = (_Float16)scale;
+  // In the large workgroups, and for fp16, the words are unpacked again: kept
+  // from the maximum they would take twice the registers of the page itself
+  // (234 us instead of 144).
+  if constexpr (NT > kThreads || !BF16) {
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) asm("" : "+v"(v[i]));
+  }
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    const int k = threadIdx.x + i * kThreads;
+    const int k = threadIdx.x + i * NT;
     if (k < n8) {
       float x[8];
       unpack8<BF16>(v[i], x);
       uint32_t w = 0;
 #pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        float qv = __builtin_rintf(div_rn(x[n], scale, rscale));
-        qv = fminf(fmaxf(qv, -8.0f), 7.0f);
-        w |= (uint32_t)((int)qv + 8) << (4 * n);
-      }
+      for (int n = 0; n < 8; ++n)
+        w = push_code(w, div_rn_code(x[n], scale, rscale), -8.0f, 7.0f, 8.0f);
       st_stream(w, codes + k);
     }
   }
 }
 
-// INT4_SYM_BLOCK save of pages larger than the register-resident kernel
-// holds, and of fp32 caches: the page absmax in a first read, the codes in a
-// second (which hits in cache).  One lane = one 8-element chunk per step.
-// Same arithmetic as int4_symblock_quant_gather_kernel.
+// INT4_SYM_BLOCK save of pages larger than the register-resident kernels
+// hold, and of fp32 caches: the page absmax in a first read, the codes in a
+// second (which hits in cache).  One lane = one 8-element chunk per step,
+// kLoopUnroll of them loaded before any is used: a page is one workgroup
+// however large it is, so the bytes that workgroup keeps in flight set its
+// rate (a page of 2M elements 500 -> 121 us with 1024 lanes of 4 chunks for 256
+// of one).  Same arithmetic as int4_symblock_quant_gather_kernel.
+constexpr int kLoopUnroll = 4;
+
 template <int DT>
-__global__ __launch_bounds__(kThreads) void int4_symblock_quant_looped_kernel(
+__global__ __launch_bounds__(kBigThreads) void int4_symblock_quant_looped_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
     const uint64_t* __restrict__ param_planes, SymGeom g, int32_t* err_flag) {
-  constexpr int ES = elem_bytes<DT>();
+  constexpr int ES = elem_bytes<DT>(), U = kLoopUnroll;
   const int64_t j = blockIdx.x;
   const int plane = blockIdx.y;
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
@@ -205,33 +258,44 @@ __global__ __launch_bounds__(kThreads) void int4_symblock_quant_looped_kernel(
   uint32_t* __restrict__ codes = reinterpret_cast<uint32_t*>(code_planes[plane]) + j * n8;
   _Float16* __restrict__ params = reinterpret_cast<_Float16*>(param_planes[plane]);
   float m = 0.0f;
-  for (int64_t k = threadIdx.x; k < n8; k += kThreads) {
-    float x[8];
-    load8<DT>(src + k * (8 * ES), x);
+  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * kBigThreads) {
+    float x[U][8];
 #pragma unroll
-    for (int n = 0; n < 8; ++n) m = fmaxf(m, fabsf(x[n]));
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = k0 + u * kBigThreads;  // past the end: the lane's first chunk again
+      load8<DT>(src + (k < n8 ? k : k0) * (8 * ES), x[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int n = 0; n < 8; ++n) m = fmaxf(m, fabsf(x[u][n]));
   }
   m = wave_max_xor(m, 64);
-  __shared__ float s_wmax[kThreads / 64];
+  __shared__ float s_wmax[kBigThreads / 64];
   if ((threadIdx.x & 63) == 0) s_wmax[threadIdx.x >> 6] = m;
   __syncthreads();
   float amax = s_wmax[0];
 #pragma unroll
-  for (int w = 1; w < kThreads / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
+  for (int w = 1; w < kBigThreads / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
   const float scale = fmaxf(amax, 1e-8f) / kSymMax;
   const float rscale = 1.0f / scale;
   if (threadIdx.x == 0) params[j] = (_Float16)scale;
-  for (int64_t k = threadIdx.x; k < n8; k += kThreads) {
-    float x[8];
-    load8<DT>(src + k * (8 * ES), x);
-    uint32_t w = 0;
+  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * kBigThreads) {
+    float x[U][8];
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      float qv = __builtin_rintf(div_rn(x[n], scale, rscale));
-      qv = fminf(fmaxf(qv, -8.0f), 7.0f);
-      w |= (uint32_t)((int)qv + 8) << (4 * n);
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = k0 + u * kBigThreads;
+      load8<DT>(src + (k < n8 ? k : k0) * (8 * ES), x[u]);
     }
-    st_stream(w, codes + k);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = k0 + u * kBigThreads;
+      uint32_t w = 0;
+#pragma unroll
+      for (int n = 0; n < 8; ++n)
+        w = push_code(w, div_rn_code(x[u][n], scale, rscale), -8.0f, 7.0f, 8.0f);
+      if (k < n8) st_stream(w, codes + k);
+    }
   }
 }
 
@@ -359,11 +423,8 @@ __global__ __launch_bounds__(kThreads) void int4_channel_quant_gather_kernel(
       if (k < n8) {
         uint32_t w = 0;
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
-          float qv = __builtin_rintf(div_rn(x[u][n], sc[n], rc[n]));
-          qv = fminf(fmaxf(qv, -8.0f), 7.0f);
-          w |= (uint32_t)((int)qv + 8) << (4 * n);
-        }
+        for (int n = 0; n < 8; ++n)
+          w = push_code(w, div_rn_code(x[u][n], sc[n], rc[n]), -8.0f, 7.0f, 8.0f);
         st_stream(w, codes + k);
       }
     }
@@ -695,6 +756,62 @@ __global__ __launch_bounds__(kThreads) void int4_asym_quant_gather_kernel(
   }
 }
 
+// Chunks of a page the register-resident INT4_SYM_BLOCK save holds.
+constexpr int64_t kMaxRegChunks = 16 * kBigThreads;
+
+// The register-resident INT4_SYM_BLOCK save of pages of n8 <= kMaxRegChunks
+// chunks of 8 bf16 / fp16 elements.
+template <bool SLOTS>
+void launch_symblock_quant(bool bf16, int64_t n8, dim3 grid, hipStream_t s,
+                           const uint64_t* cache_planes, int64_t cache_stride,
+                           const int32_t* block_ids, int64_t pool, const uint64_t* code_planes,
+                           const uint64_t* param_planes, const SymGeom& g, const SlotRows& rows,
+                           int32_t* err_flag) {
+#define AMF_LAUNCH(C, NT)                                                                     \
+  (bf16 ? int4_symblock_quant_gather_kernel<true, C, NT, SLOTS><<<grid, NT, 0, s>>>(          \
+              cache_planes, cache_stride, block_ids, pool, code_planes, param_planes, g,      \
+              rows, err_flag)                                                                 \
+        : int4_symblock_quant_gather_kernel<false, C, NT, SLOTS><<<grid, NT, 0, s>>>(         \
+              cache_planes, cache_stride, block_ids, pool, code_planes, param_planes, g,      \
+              rows, err_flag))
+  if (n8 <= 256) AMF_LAUNCH(1, 256);
+  else if (n8 <= 512) AMF_LAUNCH(2, 256);
+  else if (n8 <= 1024) AMF_LAUNCH(4, 256);
+  else if (n8 <= 2048) AMF_LAUNCH(8, 256);
+  else if (n8 <= 4096) AMF_LAUNCH(8, 512);
+  else if (n8 <= 8192) AMF_LAUNCH(8, kBigThreads);
+  else AMF_LAUNCH(16, kBigThreads);
+#undef AMF_LAUNCH
+}
+
+// The symmetric restore (page or slot form) after validation.
+template <bool SLOTS>
+int launch_sym_restore(const char* who, int32_t format, int64_t n_pages, hipStream_t s,
+                       const uint64_t* code_planes, const uint64_t* param_planes,
+                       const uint64_t* cache_planes, int64_t cache_stride, int32_t cache_dtype,
+                       const int32_t* block_ids, int64_t pool, int32_t n_planes,
+                       const SymGeom& g, const SlotRows& rows, int32_t* err_flag) {
+  const bool ch = format == AMF_FMT_INT4_SYM;
+  if (ch && (8 * kThreads) % g.head_dim != 0)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: head_dim %d must divide %d", who, g.head_dim,
+                8 * kThreads);
+  if (n_pages == 0) return ok();
+  // pages beyond 8 workgroup passes are split over workgroups of 8 passes
+  const int64_t n8 = (int64_t)g.n_rows * g.head_dim / 8;
+  const int parts = (int)std::max<int64_t>(1, n8 / (8 * kThreads));
+  if (n_pages * parts * n_planes > 0x7FFFFFF0ll)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: %lld pages x %d parts x %d planes exceed one launch",
+                who, (long long)n_pages, parts, n_planes);
+  const dim3 grid = xcd_page_grid(n_pages * parts, n_planes);
+#define AMF_LAUNCH(C)                                                                        \
+  int4_sym_dequant_scatter_kernel<DT, C, SLOTS><<<grid, kThreads, 0, s>>>(                   \
+      code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,       \
+      n_planes, parts, g, rows, err_flag)
+  AMF_WITH_DTYPE(cache_dtype, if (ch) AMF_LAUNCH(true); else AMF_LAUNCH(false));
+#undef AMF_LAUNCH
+  return check_launch(who);
+}
+
 int check_int4_format(const char* who, int32_t format) {
   if (format != AMF_FMT_INT4_SYM_BLOCK && format != AMF_FMT_INT4_SYM &&
       format != AMF_FMT_INT4_ASYM_G32)
@@ -774,23 +891,61 @@ extern "C" int amf_int4_dequant_scatter(int32_t format, const uint64_t* code_pla
   }
   SymGeom g;
   if ((rc = make_sym_geom(who, block_size, num_heads, head_dim, 1, &g))) return rc;
-  const bool ch = format == AMF_FMT_INT4_SYM;
-  if (ch && (8 * kThreads) % head_dim != 0)
-    return fail(AMF_ERR_UNSUPPORTED, "%s: head_dim %d must divide %d", who, head_dim, 8 * kThreads);
-  if (n_pages == 0) return ok();
-  // pages beyond 8 workgroup passes are split over workgroups of 8 passes
+  return launch_sym_restore<false>(who, format, n_pages, as_stream(stream), code_planes,
+                                   param_planes, cache_planes, cache_page_stride, cache_dtype,
+                                   block_ids, pool_pages, n_planes, g, SlotRows{}, err_flag);
+}
+
+extern "C" int amf_int4_dequant_scatter_slots(
+    int32_t format, const uint64_t* code_planes, const uint64_t* param_planes,
+    const uint64_t* cache_planes, int64_t cache_page_stride, int32_t cache_block,
+    int32_t cache_dtype, const int64_t* slot_mapping, int64_t pool_slots, int32_t n_planes,
+    int64_t n_slots, int32_t page_tokens, int32_t num_heads, int32_t head_dim, int32_t* err_flag,
+    void* stream) {
+  const char* who = "amf_int4_dequant_scatter_slots";
+  int rc = check_int4_format(who, format);
+  if (rc) return rc;
+  if (format == AMF_FMT_INT4_ASYM_G32)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: the symmetric formats only", who);
+  SlotRows rows;
+  int64_t n_pages = 0;
+  rc = check_slot_codec(who, cache_planes, cache_page_stride, cache_block, cache_dtype,
+                        slot_mapping, pool_slots, code_planes, param_planes, n_planes, n_slots,
+                        page_tokens, num_heads, head_dim, &rows, &n_pages);
+  if (rc) return rc;
+  SymGeom g;
+  if ((rc = make_sym_geom(who, page_tokens, num_heads, head_dim, 1, &g))) return rc;
+  return launch_sym_restore<true>(who, format, n_pages, as_stream(stream), code_planes,
+                                  param_planes, cache_planes, cache_page_stride, cache_dtype,
+                                  nullptr, 0, n_planes, g, rows, err_flag);
+}
+
+extern "C" int amf_int4_quant_gather_slots(
+    int32_t format, const uint64_t* cache_planes, int64_t cache_page_stride, int32_t cache_block,
+    int32_t cache_dtype, const int64_t* slot_mapping, int64_t pool_slots,
+    const uint64_t* code_planes, const uint64_t* param_planes, int32_t n_planes, int64_t n_slots,
+    int32_t page_tokens, int32_t num_heads, int32_t head_dim, int32_t* err_flag, void* stream) {
+  const char* who = "amf_int4_quant_gather_slots";
+  int rc = check_int4_format(who, format);
+  if (rc) return rc;
+  SlotRows rows;
+  int64_t n_pages = 0;
+  rc = check_slot_codec(who, cache_planes, cache_page_stride, cache_block, cache_dtype,
+                        slot_mapping, pool_slots, code_planes, param_planes, n_planes, n_slots,
+                        page_tokens, num_heads, head_dim, &rows, &n_pages);
+  if (rc) return rc;
+  SymGeom g;
+  if ((rc = make_sym_geom(who, page_tokens, num_heads, head_dim, 1, &g))) return rc;
   const int64_t n8 = (int64_t)g.n_rows * g.head_dim / 8;
-  const int parts = (int)std::max<int64_t>(1, n8 / (8 * kThreads));
-  if (n_pages * parts * n_planes > 0x7FFFFFF0ll)
-    return fail(AMF_ERR_UNSUPPORTED, "%s: %lld pages x %d parts x %d planes exceed one launch",
-                who, (long long)n_pages, parts, n_planes);
-  const dim3 sgrid = xcd_page_grid(n_pages * parts, n_planes);
-#define AMF_LAUNCH(C)                                                                        \
-  int4_sym_dequant_scatter_kernel<DT, C><<<sgrid, kThreads, 0, s>>>(                          \
-      code_planes, param_planes, cache_planes, cache_page_stride, block_ids, pool_pages,      \
-      n_pages, n_planes, parts, g, err_flag)
-  AMF_WITH_DTYPE(cache_dtype, if (ch) AMF_LAUNCH(true); else AMF_LAUNCH(false));
-#undef AMF_LAUNCH
+  if (format != AMF_FMT_INT4_SYM_BLOCK || cache_dtype == AMF_DTYPE_F32 || n8 > kMaxRegChunks)
+    return fail(AMF_ERR_UNSUPPORTED,
+                "%s: INT4_SYM_BLOCK pages of at most %lld bf16 / fp16 elements only", who,
+                (long long)(8 * kMaxRegChunks));
+  if (n_pages == 0) return ok();
+  launch_symblock_quant<true>(cache_dtype == AMF_DTYPE_BF16, n8,
+                              dim3((unsigned)n_pages, (unsigned)n_planes), as_stream(stream),
+                              cache_planes, cache_page_stride, nullptr, 0, code_planes,
+                              param_planes, g, rows, err_flag);
   return check_launch(who);
 }
 
@@ -837,29 +992,17 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
   if (n_pages == 0) return ok();
   if (format == AMF_FMT_INT4_SYM_BLOCK) {
     const int64_t n8 = (int64_t)g.n_rows * g.head_dim / 8;
-    const int64_t cpl = (n8 + kThreads - 1) / kThreads;  // chunks per lane
-    // Pages that fit lanes' registers (up to 32 chunks of 8 elements per lane)
-    // take the single-read kernel; larger pages and fp32 caches the two-read one.
-    if (cpl > 32 || cache_dtype == AMF_DTYPE_F32) {
-      AMF_WITH_DTYPE(cache_dtype, int4_symblock_quant_looped_kernel<DT><<<grid, kThreads, 0, s>>>(
-                                      cache_planes, cache_page_stride, block_ids, pool_pages,
-                                      code_planes, param_planes, g, err_flag));
+    // Pages that fit lanes' registers (at most kMaxRegChunks chunks) take the
+    // single-read kernel; larger pages and fp32 caches the two-read one.
+    if (cache_dtype == AMF_DTYPE_F32 || n8 > kMaxRegChunks) {
+      AMF_WITH_DTYPE(cache_dtype,
+                     int4_symblock_quant_looped_kernel<DT><<<grid, kBigThreads, 0, s>>>(
+                         cache_planes, cache_page_stride, block_ids, pool_pages, code_planes,
+                         param_planes, g, err_flag));
       return check_launch(who);
     }
-#define AMF_LAUNCH(B, C)                                                                        \
-  int4_symblock_quant_gather_kernel<B, C><<<grid, kThreads, 0, s>>>(                            \
-      cache_planes, cache_page_stride, block_ids, pool_pages, code_planes, param_planes, g, \
-      err_flag)
-#define AMF_LAUNCH_R(B)                     \
-  if (cpl <= 1) AMF_LAUNCH(B, 1);           \
-  else if (cpl <= 2) AMF_LAUNCH(B, 2);      \
-  else if (cpl <= 4) AMF_LAUNCH(B, 4);      \
-  else if (cpl <= 8) AMF_LAUNCH(B, 8);      \
-  else if (cpl <= 16) AMF_LAUNCH(B, 16);    \
-  else AMF_LAUNCH(B, 32)
-    if (bf16) { AMF_LAUNCH_R(true); } else { AMF_LAUNCH_R(false); }
-#undef AMF_LAUNCH_R
-#undef AMF_LAUNCH
+    launch_symblock_quant<false>(bf16, n8, grid, s, cache_planes, cache_page_stride, block_ids,
+                                 pool_pages, code_planes, param_planes, g, SlotRows{}, err_flag);
     return check_launch(who);
   }
   // AMF_FMT_INT4_SYM: absmax pass, then the quant pass (which also writes the fp16 scales).

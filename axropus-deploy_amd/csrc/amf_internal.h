@@ -66,4 +66,27 @@ int check_codec_geometry(const char* who, const uint64_t* cache_planes,
                          int32_t n_planes, int64_t n_pages, int32_t block_size,
                          int32_t num_heads, int32_t head_dim);
 
+// The slot form of a codec launch: token t of the sequence is the cache row
+// of slot slots[t] (slot = block * cache_block + offset), and codec page j
+// holds tokens page_tokens * j onwards, the last page padded past n_tokens.
+struct SlotRows {
+  const int64_t* slots;
+  int64_t n_tokens;
+  int64_t pool_slots;
+  int64_t page_stride;  // bytes between cache pages
+  int64_t row_bytes;    // bytes of a token row
+  int32_t cache_block;  // rows per cache page
+  int32_t page_tokens;  // tokens per codec page, at most kMaxSlotPage
+};
+constexpr int kMaxSlotPage = 256;
+
+// Validation of the slot-form codec entry points; fills rows and the number
+// of codec pages.
+int check_slot_codec(const char* who, const uint64_t* cache_planes, int64_t cache_page_stride,
+                     int32_t cache_block, int32_t cache_dtype, const int64_t* slot_mapping,
+                     int64_t pool_slots, const uint64_t* code_planes,
+                     const uint64_t* param_planes, int32_t n_planes, int64_t n_slots,
+                     int32_t page_tokens, int32_t num_heads, int32_t head_dim, SlotRows* rows,
+                     int64_t* n_pages);
+
 }  // namespace amf

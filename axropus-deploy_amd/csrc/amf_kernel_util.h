@@ -8,6 +8,7 @@
 
 #include "../../include/amf_hip.h"
 #include "amf_device.h"
+#include "amf_internal.h"
 
 namespace amf {
 
@@ -50,6 +51,27 @@ __device__ __forceinline__ PageWork xcd_page_work(int64_t n_pages, int n_planes)
 
 inline dim3 xcd_page_grid(int64_t n_pages, int n_planes) {
   return dim3((unsigned)(8 * xcd_page_items_per_xcd(n_pages, n_planes)));
+}
+
+// ---- token slots ----------------------------------------------------------------
+// Byte offsets from the plane's base of the rows of page j, in LDS; -1 for
+// tokens past the end and for slots outside the pool (flagged).  Ends with a
+// barrier.
+__device__ __forceinline__ void slot_row_offsets(const SlotRows& s, int64_t j, int64_t* tab,
+                                                 int32_t* err_flag) {
+  for (int i = threadIdx.x; i < s.page_tokens; i += blockDim.x) {
+    const int64_t t = j * s.page_tokens + i;
+    int64_t off = -1;
+    if (t < s.n_tokens) {
+      const int64_t sl = s.slots[t];
+      if (sl >= 0 && sl < s.pool_slots)
+        off = sl / s.cache_block * s.page_stride + sl % s.cache_block * s.row_bytes;
+      else if (err_flag)
+        atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    }
+    tab[i] = off;
+  }
+  __syncthreads();
 }
 
 // ---- streaming loads / stores -------------------------------------------------
@@ -253,6 +275,30 @@ __device__ __forceinline__ float div_rn(float x, float b, float rb) {
   (void)rb;
   return x / b;
 #endif
+}
+
+// x / b as div_rn gives it, but without the sign of a zero: for codes, which
+// only see the rounded integer.
+__device__ __forceinline__ float div_rn_code(float x, float b, float rb) {
+#if AMF_MARKSTEIN_DIV
+  const float q = x * rb;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, x), rb, q);
+#else
+  (void)rb;
+  return x / b;
+#endif
+}
+
+// Pushes the 4-bit code clamp(rint(q), lo, hi) + bias into w from the top:
+// after eight pushes nibble n holds the n-th code.  lo and hi are whole, so
+// clamping first gives the same integer; adding 1.5 * 2^23 + bias (bias even)
+// rounds to it to nearest even and leaves it in the low mantissa bits; a NaN
+// takes lo.  Four operations with the shift, where rint, two-sided clamp,
+// conversion, bias and insertion take seven.
+__device__ __forceinline__ uint32_t push_code(uint32_t w, float q, float lo, float hi,
+                                              float bias) {
+  const float t = __builtin_amdgcn_fmed3f(q, lo, hi) + (12582912.0f + bias);
+  return __builtin_amdgcn_alignbit(f2u(t), w, 4);
 }
 
 // ---- small reductions -------------------------------------------------------

@@ -59,6 +59,40 @@ int check_codec_geometry(const char* who, const uint64_t* cache_planes,
   return ok();
 }
 
+int check_slot_codec(const char* who, const uint64_t* cache_planes, int64_t cache_page_stride,
+                     int32_t cache_block, int32_t cache_dtype, const int64_t* slot_mapping,
+                     int64_t pool_slots, const uint64_t* code_planes,
+                     const uint64_t* param_planes, int32_t n_planes, int64_t n_slots,
+                     int32_t page_tokens, int32_t num_heads, int32_t head_dim, SlotRows* rows,
+                     int64_t* n_pages) {
+  if (cache_block <= 0 || page_tokens <= 0 || n_slots < 0)
+    return fail(AMF_ERR_INVALID_ARG, "%s: bad cache_block=%d page_tokens=%d n_slots=%lld", who,
+                cache_block, page_tokens, (long long)n_slots);
+  if (page_tokens > kMaxSlotPage)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: page_tokens %d > %d", who, page_tokens, kMaxSlotPage);
+  if (!slot_mapping && n_slots > 0)
+    return fail(AMF_ERR_INVALID_ARG, "%s: null slot_mapping", who);
+  *n_pages = n_slots / page_tokens + (n_slots % page_tokens != 0);
+  // the cache's own geometry: pages of cache_block rows
+  if (pool_slots <= 0)
+    return fail(AMF_ERR_INVALID_ARG, "%s: bad pool_slots %lld", who, (long long)pool_slots);
+  const int rc = check_codec_geometry(who, cache_planes, cache_page_stride, cache_dtype, nullptr,
+                                      1, code_planes, param_planes, n_planes, *n_pages,
+                                      cache_block, num_heads, head_dim);
+  if (rc) return rc;
+  if ((int64_t)page_tokens * num_heads * head_dim > 0x7FFFFFFF)
+    return fail(AMF_ERR_UNSUPPORTED, "%s: pages of %d tokens x %d heads x %d dims are too large",
+                who, page_tokens, num_heads, head_dim);
+  rows->slots = slot_mapping;
+  rows->n_tokens = n_slots;
+  rows->pool_slots = pool_slots;
+  rows->page_stride = cache_page_stride;
+  rows->row_bytes = (int64_t)num_heads * head_dim * cache_elem_bytes(cache_dtype);
+  rows->cache_block = cache_block;
+  rows->page_tokens = page_tokens;
+  return ok();
+}
+
 }  // namespace amf
 
 extern "C" int amf_abi_version(void) { return AMF_ABI_VERSION; }

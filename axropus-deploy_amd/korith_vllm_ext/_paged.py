@@ -644,3 +644,56 @@ def scatter_slots(in_planes: Sequence[int], in_row_stride: int, view: CacheView,
         _ptr(slots.on(dev)), view.pool_pages * view.block_size, len(view.planes), n,
         _row_bytes(view), _ptr(err_flag), amf_hip.stream_handle(dev),
     )
+
+
+# Largest INT4 block page (elements) that the slot-form save holds, and most
+# tokens of a page in the slot forms (include/amf_hip.h).
+_SLOT_SAVE_ELEMS = 131072
+_SLOT_PAGE_TOKENS = 256
+
+
+def slot_save_fits(layout: BlobLayout, dtype: torch.dtype) -> bool:
+    """Whether quant_gather_slots takes this layout from a cache of dtype."""
+    return (layout.fmt == FMT_INT4_BLOCK and dtype in (torch.bfloat16, torch.float16)
+            and layout.block_size <= _SLOT_PAGE_TOKENS and layout.page_elems <= _SLOT_SAVE_ELEMS)
+
+
+def slot_restore_fits(layout: BlobLayout) -> bool:
+    """Whether dequant_scatter_slots takes this layout."""
+    return (layout.fmt in _FMT_IDS and layout.fmt != FMT_INT4_ASYM_G32
+            and layout.block_size <= _SLOT_PAGE_TOKENS)
+
+
+def quant_gather_slots(layout: BlobLayout, view: CacheView, slots: SlotMap,
+                       blob_bases: Sequence[int], planes_per_blob: int) -> None:
+    """Quantize the cache rows of `slots` (layout.n_pages pages of
+    layout.block_size tokens, the last one padded with zeros) of every plane
+    into the blobs at blob_bases, reading each row where it is."""
+    layout.validate()
+    dev = view.device
+    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    amf_hip.call(
+        "amf_int4_quant_gather_slots", layout.fmt_id, _ptr(amf_hip.address_table(view.planes, dev)),
+        view.page_stride, view.block_size, amf_hip.dtype_tag(view.dtype), _ptr(slots.on(dev)),
+        view.pool_pages * view.block_size, _ptr(tables.codes), _ptr(tables.params),
+        len(view.planes), slots.n, layout.block_size, view.num_heads, view.head_dim, None,
+        amf_hip.stream_handle(dev),
+    )
+
+
+def dequant_scatter_slots(layout: BlobLayout, blob_bases: Sequence[int], planes_per_blob: int,
+                          view: CacheView, slots: SlotMap, n: int) -> None:
+    """Dequantize the first n tokens of every plane of the blobs at blob_bases
+    into the cache rows of the first n slots."""
+    layout.validate()
+    dev = view.device
+    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    fn = ("amf_fp8_dequant_scatter_slots" if layout.family == "fp8"
+          else "amf_int4_dequant_scatter_slots")
+    amf_hip.call(
+        fn, layout.fmt_id, _ptr(tables.codes), _ptr(tables.params),
+        _ptr(amf_hip.address_table(view.planes, dev)), view.page_stride, view.block_size,
+        amf_hip.dtype_tag(view.dtype), _ptr(slots.on(dev)), view.pool_pages * view.block_size,
+        len(view.planes), n, layout.block_size, view.num_heads, view.head_dim, None,
+        amf_hip.stream_handle(dev),
+    )

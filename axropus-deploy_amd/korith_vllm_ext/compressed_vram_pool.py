@@ -528,8 +528,10 @@ class CompressedVRAMPool:
         Slots that come in aligned runs as long as the format's dense pages
         (whole vLLM blocks of that length, or of any multiple of it when the
         cache's pages are unpadded) are quantized straight from the cache (one
-        launch for all layers); any other mapping is first gathered into a
-        dense buffer by the slot kernel."""
+        launch for all layers), and so is any mapping in int4_sym_block (its
+        128-token blocks span several vLLM pages) from a 16-bit cache; any
+        other mapping is first gathered into a dense buffer by the slot
+        kernel."""
         fmt = format or self.default_format
         if len(gpu_cache) == 0:
             return False
@@ -552,6 +554,11 @@ class CompressedVRAMPool:
             layout = self._layout(fmt, T // page, page, H, D, view.dtype)
             return self._insert(prefix_hash, fmt, layout, pview, ids, T, (2, T, H, D),
                                 view.dtype, savings_ms)
+        if fmt == FMT_INT4_BLOCK and view.dtype in (torch.bfloat16, torch.float16):
+            layout = self._layout(fmt, -(-T // page), page, H, D, view.dtype)
+            if _paged.slot_save_fits(layout, view.dtype):
+                return self._insert(prefix_hash, fmt, layout, view, None, T, (2, T, H, D),
+                                    view.dtype, savings_ms, slots=slots)
         staging = torch.empty(L, 2, T, H, D, dtype=view.dtype, device=view.device)
         outs = [staging[l, kv].data_ptr() for l in range(L) for kv in range(2)]
         _paged.gather_slots(view, slots, T, outs, H * D * staging.element_size())
@@ -575,10 +582,11 @@ class CompressedVRAMPool:
         tokens, len(slots)); reference: amf_kv_connector.py:345-385).  Returns
         n, or 0 when the entry has left the pool.
 
-        Slots in aligned runs as long as the entry's pages are written by the
-        codec kernel straight into the cache; otherwise the layers are
-        decompressed into a dense buffer and moved by the slot kernel (a raw
-        entry is moved by the slot kernel directly)."""
+        The codec kernel writes straight into the cache: whole pages where the
+        slots come in aligned runs as long as the entry's pages, token rows
+        otherwise (a raw entry is moved by the slot kernel).  Only
+        int4_asym_g32 entries in other slots are decompressed into a dense
+        buffer first."""
         with self._lock:
             if self._index.get(entry.prefix_hash) is not entry:
                 return 0
@@ -616,6 +624,8 @@ class CompressedVRAMPool:
             elif entry.format == FMT_RAW:
                 ins = [base + lay.code_offset(p) for base in bases for p in range(2)]
                 _paged.scatter_slots(ins, row, view, slots, n)
+            elif _paged.slot_restore_fits(lay):
+                _paged.dequant_scatter_slots(lay, bases, 2, view, slots, n)
             else:
                 pages = -(-n // P)
                 staging = torch.empty(2 * layers, pages, P, H, D, dtype=view.dtype,
@@ -665,7 +675,9 @@ class CompressedVRAMPool:
         return max(1, math.ceil(layout.total_bytes / self.block_bytes))
 
     def _insert(self, prefix_hash, fmt, layout, view, block_ids, n_tokens, shape, dtype,
-                savings_ms, keep=None) -> bool:
+                savings_ms, keep=None, slots: Optional[_paged.SlotMap] = None) -> bool:
+        """Save the pages block_ids of view (all of them in order when None;
+        the rows of `slots` when given) as the entry prefix_hash."""
         L = len(view.planes) // 2
         need = self._blocks_for(layout)
         with self._lock:
@@ -691,6 +703,8 @@ class CompressedVRAMPool:
                 outs = [b + layout.code_offset(p) for b in bases for p in range(2)]
                 _paged.gather_pages(view, block_ids, outs, layout.code_bytes_per_page,
                                     layout.n_pages)
+            elif slots is not None:
+                _paged.quant_gather_slots(layout, view, slots, bases, 2)
             else:
                 ws = _paged.quant_gather(layout, view, block_ids, bases, 2)
                 if fmt == FMT_FP8_E4M3:

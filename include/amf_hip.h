@@ -251,6 +251,50 @@ int amf_int4_dequant_scatter(int32_t format,
                              int32_t block_size, int32_t num_heads, int32_t head_dim,
                              int32_t* err_flag, void* stream);
 
+/* Token-slot forms of the codec launches: the rows of a codec page are the
+ * cache rows of consecutive tokens' slots instead of one cache page.  Codec
+ * page j holds tokens page_tokens * j .. of the n_slots tokens (page_tokens at
+ * most 256; codes and params laid out as for pages of page_tokens tokens, the
+ * last page padded), and slot s of a cache whose pages hold cache_block rows
+ * lives at plane + (s / cache_block) * cache_page_stride
+ * + (s % cache_block) * num_heads * head_dim * element size.  slot_mapping:
+ * device int64 array of n_slots slots in [0, pool_slots); others are skipped
+ * (restore) or read as zeros (save) and flagged in err_flag, as are the
+ * padding tokens without the flag.
+ * amf_int4_quant_gather_slots: AMF_FMT_INT4_SYM_BLOCK from a bf16 / fp16
+ * cache, pages of at most 131072 elements (AMF_ERR_UNSUPPORTED otherwise);
+ * the same bytes as a gather of the rows followed by amf_int4_quant_gather.
+ * amf_fp8_dequant_scatter_slots, amf_int4_dequant_scatter_slots: every FP8
+ * and symmetric INT4 format.
+ * Replace the flat[:, slots] gather and scatter around compress / decompress
+ * in korith_vllm_ext/amf_kv_connector.py:374-385, 411-422. */
+int amf_int4_quant_gather_slots(int32_t format,
+                                const uint64_t* cache_planes, int64_t cache_page_stride,
+                                int32_t cache_block, int32_t cache_dtype,
+                                const int64_t* slot_mapping, int64_t pool_slots,
+                                const uint64_t* code_planes, const uint64_t* param_planes,
+                                int32_t n_planes, int64_t n_slots, int32_t page_tokens,
+                                int32_t num_heads, int32_t head_dim,
+                                int32_t* err_flag, void* stream);
+
+int amf_fp8_dequant_scatter_slots(int32_t format,
+                                  const uint64_t* code_planes, const uint64_t* param_planes,
+                                  const uint64_t* cache_planes, int64_t cache_page_stride,
+                                  int32_t cache_block, int32_t cache_dtype,
+                                  const int64_t* slot_mapping, int64_t pool_slots,
+                                  int32_t n_planes, int64_t n_slots, int32_t page_tokens,
+                                  int32_t num_heads, int32_t head_dim,
+                                  int32_t* err_flag, void* stream);
+
+int amf_int4_dequant_scatter_slots(int32_t format,
+                                   const uint64_t* code_planes, const uint64_t* param_planes,
+                                   const uint64_t* cache_planes, int64_t cache_page_stride,
+                                   int32_t cache_block, int32_t cache_dtype,
+                                   const int64_t* slot_mapping, int64_t pool_slots,
+                                   int32_t n_planes, int64_t n_slots, int32_t page_tokens,
+                                   int32_t num_heads, int32_t head_dim,
+                                   int32_t* err_flag, void* stream);
+
 /* ---- paged GQA decode attention over AMF_FMT_INT4_ASYM_G32 pages --------
  * q, out     : [num_seqs][num_q_heads][head_dim]; q_dtype is AMF_DTYPE_BF16
  *              or AMF_DTYPE_F16, out_dtype one of those or AMF_DTYPE_F32
