@@ -32,7 +32,6 @@ struct PageGeom {
   int head_dim;
   int num_heads;
   int cpr_log2;      // log2(head_dim / 16)
-  int head_const;    // rows_per_iter % num_heads == 0: a lane's head never changes
   int pps;           // planes per scale group (per-tensor format)
 };
 
@@ -63,14 +62,14 @@ constexpr int dtype_of() {
 // every cache line is written whole.  The chunk's head is fixed per lane when
 // 2048 elements (one workgroup pass) span whole rows of heads.
 // SLOTS: the rows go to the cache rows of the tokens' slots.
-template <int DT, bool PER_TENSOR, bool SLOTS>
+template <int DT, bool PER_TENSOR, bool SLOTS, int TEAM>
 __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
     const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
     PageGeom g, SlotRows rows, int32_t* err_flag) {
   __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
-  const PageWork pw = xcd_page_work(n_pages, n_planes);
+  const PageWork pw = xcd_page_work<TEAM>(n_pages, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j;
   const int plane = pw.plane;
@@ -80,7 +79,7 @@ __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
   } else {
     const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
     if (dp < 0 || dp >= pool) {
-      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      if (threadIdx.x % TEAM == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
       return;
     }
     out += dp * cache_stride;
@@ -91,27 +90,29 @@ __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
       reinterpret_cast<const uint8_t*>(code_planes[plane]) + j * (int64_t)page_elems;
   const float* __restrict__ params = reinterpret_cast<const float*>(param_planes[plane]);
   const float* __restrict__ page_scales = params + j * g.num_heads;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x % TEAM;
+  // a pass of TEAM chunks spans whole tokens: a lane's head never changes
+  const bool head_const = (8 * TEAM) % (g.head_dim * g.num_heads) == 0;
   float s_fixed = 0.0f;
   if (PER_TENSOR)
     s_fixed = params[plane & 1];
-  else if (g.head_const)
+  else if (head_const)
     s_fixed = page_scales[((tid * 8) / g.head_dim) % g.num_heads];
 
   const uint32_t cpt = SLOTS ? (uint32_t)n8 / (uint32_t)rows.page_tokens : 1;  // chunks per row
   constexpr int U = AMF_RESTORE_UNROLL;
-  for (int base = tid; base < n8; base += U * kThreads) {
+  for (int base = tid; base < n8; base += U * TEAM) {
     u32x2 c[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < n8) c[u] = ld_stream(reinterpret_cast<const u32x2*>(codes) + k);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < n8) {
-        const float s = (PER_TENSOR || g.head_const)
+        const float s = (PER_TENSOR || head_const)
                             ? s_fixed
                             : page_scales[((k * 8) / g.head_dim) % g.num_heads];
         float x[8];
@@ -680,9 +681,6 @@ int make_geom(const char* who, int32_t block_size, int32_t num_heads, int32_t he
   g->head_dim = head_dim;
   g->num_heads = num_heads;
   g->cpr_log2 = __builtin_ctz(cpr);
-  // Restore passes advance 8 * kThreads elements; save passes kThreads / cpr rows.
-  g->head_const = ((kThreads * 8) % (head_dim * num_heads)) == 0 &&
-                  ((kThreads / cpr) % num_heads) == 0;
   g->pps = pps > 0 ? pps : 1;
   return ok();
 }
@@ -713,15 +711,22 @@ void launch_restore(int32_t format, int64_t n_pages, hipStream_t s, const uint64
                     int64_t cache_stride, int32_t cache_dtype, const int32_t* block_ids,
                     int64_t pool, int32_t n_planes, const PageGeom& g, const SlotRows& rows,
                     int32_t* err_flag) {
-  const dim3 grid = xcd_page_grid(n_pages, n_planes);
   const bool pt = format == AMF_FMT_FP8_E4M3;
   // the slot form's row table counts towards the pad
   const unsigned pad = kRestoreLdsPad - (SLOTS ? kMaxSlotPage * sizeof(int64_t) : 0);
-#define AMF_LAUNCH(T)                                                                        \
-  fp8_dequant_scatter_kernel<DT, T, SLOTS><<<grid, kThreads, pad, s>>>(                      \
-      code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,       \
-      n_planes, g, rows, err_flag)
-  AMF_WITH_DTYPE(cache_dtype, if (pt) AMF_LAUNCH(true); else AMF_LAUNCH(false));
+#define AMF_LAUNCH(T, TEAM)                                                                  \
+  fp8_dequant_scatter_kernel<DT, T, SLOTS, TEAM>                                             \
+      <<<xcd_page_grid<TEAM>(n_pages, n_planes), kThreads, TEAM == kPageTeam ? pad : 0, s>>>( \
+          code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,   \
+          n_planes, g, rows, err_flag)
+  if constexpr (!SLOTS) {
+    if ((int64_t)g.n_rows * g.head_dim <= 8 * kSmallPageChunks) {
+      AMF_WITH_DTYPE(cache_dtype, if (pt) AMF_LAUNCH(true, 64); else AMF_LAUNCH(false, 64));
+      return;
+    }
+  }
+  AMF_WITH_DTYPE(cache_dtype,
+                 if (pt) AMF_LAUNCH(true, kPageTeam); else AMF_LAUNCH(false, kPageTeam));
 #undef AMF_LAUNCH
 }
 

@@ -59,14 +59,14 @@ __device__ __forceinline__ void load32(const uint8_t* p, float* x) {
 // of the workgroup is cut into `parts` workgroups of whole passes (a dense
 // tensor's page can hold millions of elements).
 // SLOTS: the rows go to the cache rows of the tokens' slots.
-template <int DT, bool CHANNEL, bool SLOTS>
+template <int DT, bool CHANNEL, bool SLOTS, int TEAM>
 __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
     const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
     int parts, SymGeom g, SlotRows rows, int32_t* err_flag) {
   __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
-  const PageWork pw = xcd_page_work(n_pages * parts, n_planes);
+  const PageWork pw = xcd_page_work<TEAM>(n_pages * parts, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j / parts;
   const int part = (int)(pw.j % parts);
@@ -77,23 +77,23 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
   } else {
     const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
     if (dp < 0 || dp >= pool) {
-      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      if (threadIdx.x % TEAM == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
       return;
     }
     out += dp * cache_stride;
   }
   const int page_elems = g.n_rows * g.head_dim;
   const int n8 = page_elems >> 3;
-  // this workgroup's chunks: [k_begin, k_end), k_begin a multiple of kThreads
+  // this workgroup's chunks: [k_begin, k_end), k_begin a multiple of TEAM
   const int span = (n8 + parts - 1) / parts;
-  const int k_begin = part * ((span + kThreads - 1) / kThreads * kThreads);
-  const int k_end = min(n8, k_begin + (span + kThreads - 1) / kThreads * kThreads);
+  const int k_begin = part * ((span + TEAM - 1) / TEAM * TEAM);
+  const int k_end = min(n8, k_begin + (span + TEAM - 1) / TEAM * TEAM);
   const uint32_t* __restrict__ codes =
       reinterpret_cast<const uint32_t*>(code_planes[plane]) + j * (int64_t)n8;
   const _Float16* __restrict__ params = reinterpret_cast<const _Float16*>(param_planes[plane]);
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x % TEAM;
   const float s_page = CHANNEL ? 0.0f : (float)params[j];
-  // Channel scales of this lane's 8 dims; fixed while 8 * kThreads is a
+  // Channel scales of this lane's 8 dims; fixed while 8 * TEAM is a
   // multiple of head_dim (checked on the host).
   float s_ch[8];
   if (CHANNEL) {
@@ -103,16 +103,16 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
   }
   const uint32_t cpt = SLOTS ? (uint32_t)n8 / (uint32_t)rows.page_tokens : 1;  // chunks per row
   constexpr int U = AMF_SYM_RESTORE_UNROLL;
-  for (int base = k_begin + tid; base < k_end; base += U * kThreads) {
+  for (int base = k_begin + tid; base < k_end; base += U * TEAM) {
     uint32_t c[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < k_end) c[u] = ld_stream(codes + k);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < k_end) {
         float x[8];
 #pragma unroll
@@ -442,6 +442,7 @@ struct AsymGeom {
   int groups;          // head_dim / 32
   int hb_code_bytes;   // 16 * head_dim / 2   (one (page, head) code block)
   int hb_param_words;  // 16 * groups
+  int kpr_log2, h_log2;  // log2(head_dim / 8) and log2(num_heads), -1 unless powers of two
 };
 
 // Group quantizer: min / max over 32 values, then
@@ -493,23 +494,41 @@ __device__ __forceinline__ float param_zero(uint32_t w) {
 #endif
 constexpr int kKUnroll = AMF_ASYM_K_UNROLL;
 
-template <int DT>
+// TEAM lanes take a page (four pages a workgroup when it is small), and a V
+// item writes 8 / VSPLIT of its tokens, so that a page of few heads still has
+// an item for each lane.  P2: head_dim and the head count are powers of two,
+// so the items' indices are shifts.  80 layers x 777 pages of 1 x 128 235 ->
+// 113 us, 32 x 1000 of 2 x 128 153 -> 115 us (6.0 TB/s), 32 x 512 of 8 x 128
+// 245 -> 241 us.
+template <int DT, int TEAM, int VSPLIT, bool P2>
 __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
     const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, AsymGeom g, int32_t* err_flag) {
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, AsymGeom g,
+    int32_t* err_flag) {
   // A (page, plane) grid, page-major: all XCDs work on one plane at a time,
   // which measured faster here than the XCD-contiguous map of the other
   // restores (1.025 vs 1.065 ms at 32 layers x 2048 pages).
-  const int64_t j = blockIdx.x;
+  constexpr int kPages = kThreads / TEAM;
+  const int64_t j =
+      (int64_t)blockIdx.x * kPages +
+      (kPages > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM) : 0);
+  if (kPages > 1 && j >= n_pages) return;
+  const int tid = threadIdx.x % TEAM;
   const int plane = blockIdx.y;
   const bool is_v = (plane & 1) != 0;
   const int64_t dp = block_ids ? (int64_t)block_ids[j] : j;
   if (dp < 0 || dp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    if (tid == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
     return;
   }
   const int H = g.num_heads, D = g.head_dim, G = g.groups;
+  const int kpr = D / 8;  // 8-dim blocks per row
+  // quotient by, and remainder of, the block count and the head count
+  auto by_kpr = [&](int x) { return P2 ? x >> g.kpr_log2 : x / kpr; };
+  auto of_kpr = [&](int x) { return P2 ? x & (kpr - 1) : x % kpr; };
+  auto by_h = [&](int x) { return P2 ? x >> g.h_log2 : x / H; };
+  auto of_h = [&](int x) { return P2 ? x & (H - 1) : x % H; };
   const uint8_t* __restrict__ codes = reinterpret_cast<const uint8_t*>(code_planes[plane]) +
                                       j * (int64_t)H * g.hb_code_bytes;
   const uint32_t* __restrict__ params = reinterpret_cast<const uint32_t*>(param_planes[plane]) +
@@ -521,17 +540,16 @@ __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
     // 16-byte vector of the page, reads 4 code bytes and its group's param word.
     // kKUnroll items per lane have their code and param loads in flight
     // before any is converted.
-    const int kpr = D / 8;  // 8-dim blocks per row
     const int n_items = 16 * H * kpr;
-    for (int it0 = threadIdx.x; it0 < n_items; it0 += kThreads * kKUnroll) {
+    for (int it0 = tid; it0 < n_items; it0 += TEAM * kKUnroll) {
       uint32_t c[kKUnroll], pw[kKUnroll];
 #pragma unroll
       for (int u = 0; u < kKUnroll; ++u) {
-        const int it = it0 + u * kThreads;
+        const int it = it0 + u * TEAM;
         if (it < n_items) {
-          const int kk = it % kpr;
-          const int th = it / kpr;  // token * H + head
-          const int t = th / H, h = th % H;
+          const int kk = of_kpr(it);
+          const int th = by_kpr(it);  // token * H + head
+          const int t = by_h(th), h = of_h(th);
           const int ht = h * 16 + t;
           c[u] = ld_stream(reinterpret_cast<const uint32_t*>(codes + (int64_t)ht * (D / 2)) + kk);
           pw[u] = params[ht * G + (kk >> 2)];
@@ -539,7 +557,7 @@ __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
       }
 #pragma unroll
       for (int u = 0; u < kKUnroll; ++u) {
-        const int it = it0 + u * kThreads;
+        const int it = it0 + u * TEAM;
         if (it < n_items) {
           const float s = param_scale(pw[u]), z = param_zero(pw[u]);
           float x[8];
@@ -550,28 +568,32 @@ __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
       }
     }
   } else {
-    const int nb = D / 8;
-    const int n_items = H * nb * 2;
-    for (int it = threadIdx.x; it < n_items; it += kThreads) {
-      const int th = it & 1;
-      const int b = (it >> 1) % nb;
-      const int h = (it >> 1) / nb;
+    // Items (head, token half, part, 8-dim block), the block fastest: lanes
+    // next to each other write next to each other.
+    constexpr int NT = 8 / VSPLIT;  // tokens of an item
+    const int n_items = H * kpr * 2 * VSPLIT;
+    for (int it = tid; it < n_items; it += TEAM) {
+      const int b = of_kpr(it);
+      const int r = by_kpr(it);
+      const int i0 = r % VSPLIT * NT;
+      const int th = r / VSPLIT & 1;
+      const int h = r / (2 * VSPLIT);
       const u32x4* cp =
           reinterpret_cast<const u32x4*>(codes + (int64_t)h * g.hb_code_bytes + 64 * b + 32 * th);
       const u32x4 c0 = ld_stream(cp);
       const u32x4 c1 = ld_stream(cp + 1);
       const uint32_t w[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-      const u32x4* pp = reinterpret_cast<const u32x4*>(params + h * g.hb_param_words +
-                                                       (b >> 2) * 16 + 8 * th);
-      const u32x4 p0 = pp[0], p1 = pp[1];
-      const uint32_t pw[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+      const uint32_t* pp = params + h * g.hb_param_words + (b >> 2) * 16 + 8 * th + i0;
+      uint32_t pw[NT];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < NT; ++i) pw[i] = pp[i];
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
         const float s = param_scale(pw[i]), z = param_zero(pw[i]);
         float x[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) x[k] = nib(w[k], i) * s + z;
-        const int t = 8 * th + i;
+        for (int k = 0; k < 8; ++k) x[k] = nib(w[k], i0 + i) * s + z;
+        const int t = 8 * th + i0 + i;
         store8<DT>(out + elem_bytes<DT>() * ((int64_t)(t * H + h) * D + 8 * b), x);
       }
     }
@@ -802,12 +824,20 @@ int launch_sym_restore(const char* who, int32_t format, int64_t n_pages, hipStre
   if (n_pages * parts * n_planes > 0x7FFFFFF0ll)
     return fail(AMF_ERR_UNSUPPORTED, "%s: %lld pages x %d parts x %d planes exceed one launch",
                 who, (long long)n_pages, parts, n_planes);
-  const dim3 grid = xcd_page_grid(n_pages * parts, n_planes);
-#define AMF_LAUNCH(C)                                                                        \
-  int4_sym_dequant_scatter_kernel<DT, C, SLOTS><<<grid, kThreads, 0, s>>>(                   \
-      code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,       \
-      n_planes, parts, g, rows, err_flag)
-  AMF_WITH_DTYPE(cache_dtype, if (ch) AMF_LAUNCH(true); else AMF_LAUNCH(false));
+#define AMF_LAUNCH(C, TEAM)                                                                  \
+  int4_sym_dequant_scatter_kernel<DT, C, SLOTS, TEAM>                                        \
+      <<<xcd_page_grid<TEAM>(n_pages * parts, n_planes), kThreads, 0, s>>>(                  \
+          code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,   \
+          n_planes, parts, g, rows, err_flag)
+  if constexpr (!SLOTS) {
+    // a wave's pass of 512 elements keeps a lane's channels as well
+    if (n8 <= kSmallPageChunks && (!ch || 512 % g.head_dim == 0)) {
+      AMF_WITH_DTYPE(cache_dtype, if (ch) AMF_LAUNCH(true, 64); else AMF_LAUNCH(false, 64));
+      return check_launch(who);
+    }
+  }
+  AMF_WITH_DTYPE(cache_dtype,
+                 if (ch) AMF_LAUNCH(true, kPageTeam); else AMF_LAUNCH(false, kPageTeam));
 #undef AMF_LAUNCH
   return check_launch(who);
 }
@@ -847,6 +877,9 @@ int make_asym_geom(const char* who, int32_t block_size, int32_t num_heads, int32
   g->groups = head_dim / 32;
   g->hb_code_bytes = 16 * head_dim / 2;
   g->hb_param_words = 16 * g->groups;
+  auto log2_or = [](int x) { return (x & (x - 1)) == 0 ? __builtin_ctz(x) : -1; };
+  g->kpr_log2 = log2_or(head_dim / 8);
+  g->h_log2 = log2_or(num_heads);
   *lds_tables = (size_t)3 * 4 * 16 * num_heads * g->groups;
   *lds_staged = (size_t)16 * num_heads * head_dim * elem_size + *lds_tables;
   if (*lds_tables > (size_t)kAsymLdsBytes)
@@ -882,11 +915,22 @@ extern "C" int amf_int4_dequant_scatter(int32_t format, const uint64_t* code_pla
                              n_planes, &g, &lds_staged, &lds_tables)))
       return rc;
     if (n_pages == 0) return ok();
-    AMF_WITH_DTYPE(cache_dtype,
-                   int4_asym_dequant_scatter_kernel<DT>
-                   <<<dim3((unsigned)n_pages, (unsigned)n_planes), kThreads, 0, s>>>(
-                       code_planes, param_planes, cache_planes, cache_page_stride, block_ids,
-                       pool_pages, g, err_flag));
+#define AMF_LAUNCH(TEAM, VSPLIT, P2)                                                           \
+  AMF_WITH_DTYPE(cache_dtype,                                                                  \
+                 int4_asym_dequant_scatter_kernel<DT, TEAM, VSPLIT, P2>                        \
+                 <<<dim3((unsigned)((n_pages + kThreads / TEAM - 1) / (kThreads / TEAM)),      \
+                         (unsigned)n_planes),                                                  \
+                    kThreads, 0, s>>>(code_planes, param_planes, cache_planes,                 \
+                                      cache_page_stride, block_ids, pool_pages, n_pages, g,    \
+                                      err_flag))
+    const int64_t v_items = (int64_t)num_heads * head_dim / 8 * 2;
+    if (g.kpr_log2 < 0 || g.h_log2 < 0) AMF_LAUNCH(256, 1, false);
+    else if (8 * v_items > kSmallPageChunks && v_items < kThreads) AMF_LAUNCH(256, 2, true);
+    else if (8 * v_items > kSmallPageChunks) AMF_LAUNCH(256, 1, true);
+    else if (v_items <= 16) AMF_LAUNCH(64, 4, true);
+    else if (v_items <= 32) AMF_LAUNCH(64, 2, true);
+    else AMF_LAUNCH(64, 1, true);
+#undef AMF_LAUNCH
     return check_launch(who);
   }
   SymGeom g;

@@ -29,28 +29,46 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // read, lose with the pad).
 constexpr unsigned kRestoreLdsPad = 52u << 10;
 
+// A page takes one workgroup of kPageTeam lanes, or, when it is small (at most
+// kSmallPageChunks chunks of 8 elements: one or two KV heads of a
+// tensor-parallel rank), one wave, four pages to a workgroup: with a 4 KiB page
+// per workgroup the chip waits for workgroups to start.  80 layers x 777 pages
+// of 1 x 128, a workgroup / a wave per page, us: fp8_e4m3 279 / 138,
+// fp8_e4m3_ph 312 / 138, int4_sym 193 / 117; 32 x 1000 of 2 x 128: 164 / 148,
+// 205 / 146, 150 / 127.  Pages of 4 x 128 run at 5.2-5.6 TB/s as workgroups.
+constexpr int kPageTeam = 256;
+constexpr int64_t kSmallPageChunks = 512;
+
 struct PageWork {
   int64_t j;   // position in the gathered sequence
   int plane;
-  bool valid;  // false for the up to 7 padding workgroups
+  bool valid;  // false for the padding teams
 };
 
-__host__ __device__ inline int64_t xcd_page_items_per_xcd(int64_t n_pages, int n_planes) {
-  return (n_pages * n_planes + 7) / 8;
+// Workgroups of each XCD over n_pages x n_planes pages, TEAM lanes a page.
+template <int TEAM>
+__host__ __device__ inline uint32_t xcd_page_groups(int64_t n_pages, int n_planes) {
+  constexpr int kPages = kPageTeam / TEAM;
+  return (uint32_t)((n_pages * n_planes + 8 * kPages - 1) / (8 * kPages));
 }
 
+// n_pages * n_planes < 2^31 (checked on the host).
+template <int TEAM>
 __device__ __forceinline__ PageWork xcd_page_work(int64_t n_pages, int n_planes) {
-  const int64_t id = blockIdx.x;
-  const int64_t w = (id & 7) * xcd_page_items_per_xcd(n_pages, n_planes) + (id >> 3);
+  constexpr int kPages = kPageTeam / TEAM;
+  const uint32_t id = blockIdx.x;
+  uint32_t w = ((id & 7) * xcd_page_groups<TEAM>(n_pages, n_planes) + (id >> 3)) * kPages;
+  if constexpr (kPages > 1) w += __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM);
   PageWork r;
-  r.valid = w < n_pages * n_planes;
-  r.plane = (int)(w / n_pages);
-  r.j = w - (int64_t)r.plane * n_pages;
+  r.valid = w < (uint32_t)(n_pages * n_planes);
+  r.plane = (int)(w / (uint32_t)n_pages);
+  r.j = w - (uint32_t)r.plane * (uint32_t)n_pages;
   return r;
 }
 
+template <int TEAM>
 inline dim3 xcd_page_grid(int64_t n_pages, int n_planes) {
-  return dim3((unsigned)(8 * xcd_page_items_per_xcd(n_pages, n_planes)));
+  return dim3(8 * xcd_page_groups<TEAM>(n_pages, n_planes));
 }
 
 // ---- token slots ----------------------------------------------------------------
