@@ -415,28 +415,37 @@ __global__ __launch_bounds__(kCoopThreads) void fp8_tensor_coop_kernel(CoopArgs 
 // reduction and each half-wave quantizes as soon as its own loads land.
 // Chunk c of a head is token c / (head_dim / 8), dims 8 (c % (head_dim / 8))
 // ..+7: 16 consecutive lanes read one 256-byte row (bf16, head_dim 128).
-// A workgroup takes 8 heads per pass.
-template <int DT, int CPL>
+// A workgroup takes 8 heads per pass of one page, or (PACK, pages of fewer
+// heads) 8 consecutive (page, head) blocks of a plane.
+template <int DT, int CPL, bool PACK>
 __global__ __launch_bounds__(kThreads) void fp8_ph_quant_gather_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    const uint64_t* __restrict__ param_planes, PageGeom g, int32_t* err_flag) {
-  const int64_t j = blockIdx.x;
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages,
+    const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
+    PageGeom g, int32_t* err_flag) {
+  const int H = g.num_heads, D = g.head_dim;
+  const int lh = threadIdx.x & 31;
+  int64_t j = blockIdx.x;
+  int h = (int)(threadIdx.x >> 5);
+  if constexpr (PACK) {
+    const uint32_t u = blockIdx.x * (kThreads / 32) + (uint32_t)h;
+    j = u / (uint32_t)H;
+    h = (int)(u - (uint32_t)j * H);
+    if (j >= n_pages) return;
+  }
   const int plane = blockIdx.y;
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
   if (sp < 0 || sp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    if (lh == 0 && h == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
     return;
   }
-  const int H = g.num_heads, D = g.head_dim;
   const int64_t page_elems = (int64_t)g.n_rows * D;
   const uint8_t* __restrict__ src =
       reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride;
   uint8_t* __restrict__ codes = reinterpret_cast<uint8_t*>(code_planes[plane]) + j * page_elems;
   float* __restrict__ params = reinterpret_cast<float*>(param_planes[plane]) + j * H;
-  const int lh = threadIdx.x & 31;
   const int cpr = D >> 3;  // chunks per token row of one head
-  for (int h = (int)(threadIdx.x >> 5); h < H; h += kThreads / 32) {
+  for (; h < H; h += PACK ? H : kThreads / 32) {
     int64_t off[CPL];
     float x[CPL][8];
 #pragma unroll
@@ -922,11 +931,22 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
   const int64_t head_chunks = (int64_t)(g.n_rows / g.num_heads) * head_dim / 8;
   const int cpl = (int)(head_chunks / 32);
   if (!pt && cache_dtype != AMF_DTYPE_F32 && head_chunks % 32 == 0 &&
-      (cpl == 2 || cpl == 4 || cpl == 8 || cpl == 16)) {
+      n_pages * num_heads <= 0x7FFFFFF0ll && (cpl == 2 || cpl == 4 || cpl == 8 || cpl == 16)) {
+    // Pages that leave most of a workgroup's half-waves idle share workgroups:
+    // 80 layers x 777 pages of 1 head 181 -> 119 us; no gain from 2 heads on.
+    const bool pack = num_heads < 4;
+    const dim3 pgrid(
+        (unsigned)((n_pages * num_heads + kThreads / 32 - 1) / (kThreads / 32)),
+        (unsigned)n_planes);
 #define AMF_LAUNCH(C)                                                                          \
-  AMF_WITH_DTYPE(cache_dtype, fp8_ph_quant_gather_kernel<DT, C><<<grid, kThreads, 0, s>>>(     \
-                                  cache_planes, cache_page_stride, block_ids, pool_pages,      \
-                                  code_planes, param_planes, g, err_flag))
+  AMF_WITH_DTYPE(                                                                              \
+      cache_dtype,                                                                             \
+      if (pack) fp8_ph_quant_gather_kernel<DT, C, true><<<pgrid, kThreads, 0, s>>>(            \
+          cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, code_planes,        \
+          param_planes, g, err_flag);                                                          \
+      else fp8_ph_quant_gather_kernel<DT, C, false><<<grid, kThreads, 0, s>>>(                 \
+          cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, code_planes,        \
+          param_planes, g, err_flag))
     if (cpl == 2) AMF_LAUNCH(2);
     else if (cpl == 4) AMF_LAUNCH(4);
     else if (cpl == 8) AMF_LAUNCH(8);

@@ -465,10 +465,18 @@ __device__ __forceinline__ AsymParams asym_params(const float* x) {
   return p;
 }
 
-__device__ __forceinline__ uint32_t asym_code(float x, const AsymParams& p) {
+// Code n of eight into w, in order.  The wave-per-page save pushes it
+// (push_code), which needs fewer operations; with a workgroup per page the
+// compiler then holds so many chains at once that waves are lost (32 layers x
+// 500 pages of 4 x 128: 145 us against 133).
+template <int TEAM>
+__device__ __forceinline__ uint32_t asym_insert(uint32_t w, int n, float x,
+                                                const AsymParams& p) {
+  if constexpr (TEAM == 64)
+    return push_code(w, div_rn_code(x - p.mn, p.scale, p.rscale), 0.0f, kAsymLevels, 0.0f);
   float q = __builtin_rintf(div_rn(x - p.mn, p.scale, p.rscale));
   q = fminf(fmaxf(q, 0.0f), kAsymLevels);
-  return (uint32_t)q;
+  return w | (uint32_t)q << (4 * n);
 }
 
 __device__ __forceinline__ uint32_t asym_param_word(const AsymParams& p) {
@@ -600,31 +608,74 @@ __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
   }
 }
 
+// The lanes that save a page: the workgroup, or one wave of it (small pages,
+// four to a workgroup).  A wave's LDS accesses complete in order, so its sync
+// only keeps the compiler from moving them.
+template <int TEAM>
+__device__ __forceinline__ int team_lane() {
+  return (int)(TEAM == kThreads ? threadIdx.x : threadIdx.x % TEAM);
+}
+template <int TEAM>
+__device__ __forceinline__ void team_sync() {
+  if constexpr (TEAM == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// A page's bytes -> LDS, kStageUnroll 16-byte vectors per lane in flight.
+// (Padding the rows against the bank conflicts of the quantizers' 64-byte
+// reads measured slower: 140 vs 133 us at 32 layers x 500 pages of 4 x 128.)
+#ifndef AMF_ASYM_STAGE_UNROLL
+#define AMF_ASYM_STAGE_UNROLL 8
+#endif
+constexpr int kStageUnroll = AMF_ASYM_STAGE_UNROLL;
+
+template <int TEAM>
+__device__ __forceinline__ void stage_page(const uint8_t* __restrict__ src, int page_bytes,
+                                           uint8_t* lds) {
+  for (int o0 = team_lane<TEAM>() * 16; o0 < page_bytes; o0 += TEAM * 16 * kStageUnroll) {
+    u32x4 v[kStageUnroll];
+#pragma unroll
+    for (int u = 0; u < kStageUnroll; ++u) {
+      const int o = o0 + u * TEAM * 16;
+      if (o < page_bytes) v[u] = ld_stream(reinterpret_cast<const u32x4*>(src + o));
+    }
+#pragma unroll
+    for (int u = 0; u < kStageUnroll; ++u) {
+      const int o = o0 + u * TEAM * 16;
+      if (o < page_bytes) *reinterpret_cast<u32x4*>(lds + o) = v[u];
+    }
+  }
+}
+
 // Save of one page of a K plane: items (head, token, group) read 64 cache
 // bytes, write 16 code bytes and one param word.
 #ifndef AMF_ASYM_KSAVE_UNROLL
 #define AMF_ASYM_KSAVE_UNROLL 2
 #endif
 constexpr int kKSaveUnroll = AMF_ASYM_KSAVE_UNROLL;
-template <int DT>
+template <int DT, int TEAM, int KU>
 __device__ __forceinline__ void asym_quant_k(const uint8_t* __restrict__ src,
                                              uint8_t* __restrict__ codes,
                                              uint32_t* __restrict__ params, const AsymGeom& g) {
   const int H = g.num_heads, D = g.head_dim, G = g.groups;
   const int n_items = 16 * H * G;
   // Items in cache order (token, head, group) so the loads are contiguous;
-  // kKSaveUnroll items per lane are loaded before any is quantized.
-  for (int it0 = threadIdx.x; it0 < n_items; it0 += kThreads * kKSaveUnroll) {
-    float x[kKSaveUnroll][32];
+  // KU items per lane are loaded before any is quantized.
+  for (int it0 = team_lane<TEAM>(); it0 < n_items; it0 += TEAM * KU) {
+    float x[KU][32];
 #pragma unroll
-    for (int u = 0; u < kKSaveUnroll; ++u) {
-      const int it = it0 + u * kThreads;
+    for (int u = 0; u < KU; ++u) {
+      const int it = it0 + u * TEAM;
       if (it < n_items)
         load32<DT>(src + elem_bytes<DT>() * ((int64_t)(it / G) * D + 32 * (it % G)), x[u]);
     }
 #pragma unroll
-    for (int u = 0; u < kKSaveUnroll; ++u) {
-      const int it = it0 + u * kThreads;
+    for (int u = 0; u < KU; ++u) {
+      const int it = it0 + u * TEAM;
       if (it < n_items) {
         const int gi = it % G;
         const int th = it / G;  // token * H + head
@@ -635,7 +686,8 @@ __device__ __forceinline__ void asym_quant_k(const uint8_t* __restrict__ src,
         for (int q = 0; q < 4; ++q) {
           uint32_t w = 0;
 #pragma unroll
-          for (int n = 0; n < 8; ++n) w |= asym_code(x[u][8 * q + n], p) << (4 * n);
+          for (int n = 0; n < 8; ++n)
+            w = asym_insert<TEAM>(w, n, x[u][8 * q + n], p);
           c[q] = w;
         }
         const int ht = h * 16 + t;
@@ -652,12 +704,8 @@ __device__ __forceinline__ void asym_quant_k(const uint8_t* __restrict__ src,
 // into LDS first (when it fits); otherwise both phases read the page from
 // global memory, where the second read hits in cache.
 constexpr int kAsymLdsBytes = 64 * 1024;
-#ifndef AMF_ASYM_STAGE_UNROLL
-#define AMF_ASYM_STAGE_UNROLL 8
-#endif
-constexpr int kStageUnroll = AMF_ASYM_STAGE_UNROLL;
 
-template <int DT, bool STAGED>
+template <int DT, bool STAGED, int TEAM>
 __device__ __forceinline__ void asym_quant_v(const uint8_t* __restrict__ src,
                                              uint8_t* __restrict__ codes,
                                              uint32_t* __restrict__ params, const AsymGeom& g,
@@ -666,29 +714,14 @@ __device__ __forceinline__ void asym_quant_v(const uint8_t* __restrict__ src,
   const int H = g.num_heads, D = g.head_dim, G = g.groups;
   const int page_bytes = STAGED ? 16 * H * D * ES : 0;
   // phase 0: page -> LDS (cache layout)
-  if (STAGED) {
-    // kStageUnroll vectors per lane in flight before they are stored to LDS.
-    for (int o0 = threadIdx.x * 16; o0 < page_bytes; o0 += kThreads * 16 * kStageUnroll) {
-      u32x4 v[kStageUnroll];
-#pragma unroll
-      for (int u = 0; u < kStageUnroll; ++u) {
-        const int o = o0 + u * kThreads * 16;
-        if (o < page_bytes) v[u] = ld_stream(reinterpret_cast<const u32x4*>(src + o));
-      }
-#pragma unroll
-      for (int u = 0; u < kStageUnroll; ++u) {
-        const int o = o0 + u * kThreads * 16;
-        if (o < page_bytes) *reinterpret_cast<u32x4*>(lds + o) = v[u];
-      }
-    }
-  }
+  if (STAGED) stage_page<TEAM>(src, page_bytes, lds);
   const uint8_t* data = STAGED ? lds : src;
   float* s_mn = reinterpret_cast<float*>(lds + page_bytes);          // [H][G][16]
   float* s_sc = s_mn + 16 * H * G;                                   // [H][G][16]
   float* s_rc = s_sc + 16 * H * G;                                   // [H][G][16]
-  __syncthreads();
+  team_sync<TEAM>();
   const int n_groups = 16 * H * G;
-  for (int it = threadIdx.x; it < n_groups; it += kThreads) {
+  for (int it = team_lane<TEAM>(); it < n_groups; it += TEAM) {
     // it = (head, group, token): params are written in V order.
     const int t = it & 15;
     const int hg = it >> 4;
@@ -701,10 +734,10 @@ __device__ __forceinline__ void asym_quant_v(const uint8_t* __restrict__ src,
     s_rc[it] = p.rscale;
     params[it] = asym_param_word(p);
   }
-  __syncthreads();
+  team_sync<TEAM>();
   const int nb = D / 8;
   const int n_items = H * nb * 2;
-  for (int it = threadIdx.x; it < n_items; it += kThreads) {
+  for (int it = team_lane<TEAM>(); it < n_items; it += TEAM) {
     const int th = it & 1;
     const int b = (it >> 1) % nb;
     const int h = (it >> 1) / nb;
@@ -720,7 +753,8 @@ __device__ __forceinline__ void asym_quant_v(const uint8_t* __restrict__ src,
       float x[8];
       load8<DT>(data + ES * ((t * H + h) * D + 8 * b), x);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) w[k] |= asym_code(x[k], p) << (4 * i);
+      for (int k = 0; k < 8; ++k)
+        w[k] = asym_insert<TEAM>(w[k], i, x[k], p);
     }
     u32x4* cp = reinterpret_cast<u32x4*>(codes + (int64_t)h * g.hb_code_bytes + 64 * b + 32 * th);
     st_stream(u32x4{w[0], w[1], w[2], w[3]}, cp);
@@ -728,17 +762,28 @@ __device__ __forceinline__ void asym_quant_v(const uint8_t* __restrict__ src,
   }
 }
 
-template <int DT, bool STAGED>
-__global__ __launch_bounds__(kThreads) void int4_asym_quant_gather_kernel(
+// One page per team; KU: K items a lane loads at once.  A wave per page for
+// small pages (four to a workgroup; one K item per lane for one head, whose
+// registers allow 8 waves per SIMD): 80 layers x 777 pages of 1 x 128 213 ->
+// 122 us, 32 x 1000 of 2 x 128 152 -> 119 us (5.8 TB/s), where a workgroup per
+// page had 64 and 128 items for its 256 lanes.
+template <int DT, bool STAGED, int TEAM, int KU>
+__global__ __launch_bounds__(kThreads, TEAM == kThreads ? 1 : KU == 1 ? 8 : 5) void
+int4_asym_quant_gather_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    const uint64_t* __restrict__ param_planes, AsymGeom g, int32_t* err_flag) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const int64_t j = blockIdx.x;
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages,
+    const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
+    AsymGeom g, int team_lds, int32_t* err_flag) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t shared_lds[];
+  constexpr int kPages = kThreads / TEAM;
+  const int team = kPages > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM) : 0;
+  uint8_t* lds = shared_lds + team * team_lds;
+  const int64_t j = (int64_t)blockIdx.x * kPages + team;
+  if (kPages > 1 && j >= n_pages) return;
   const int plane = blockIdx.y;
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
   if (sp < 0 || sp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    if (team_lane<TEAM>() == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
     return;
   }
   const int H = g.num_heads;
@@ -754,27 +799,14 @@ __global__ __launch_bounds__(kThreads) void int4_asym_quant_gather_kernel(
       // instruction); the items' 64-byte reads then come from LDS.  Reading
       // the items straight from memory splits every line over four load
       // instructions, which the non-temporal policy would fetch repeatedly.
-      const int page_bytes = 16 * H * g.head_dim * elem_bytes<DT>();
-      for (int o0 = threadIdx.x * 16; o0 < page_bytes; o0 += kThreads * 16 * kStageUnroll) {
-        u32x4 v[kStageUnroll];
-#pragma unroll
-        for (int u = 0; u < kStageUnroll; ++u) {
-          const int o = o0 + u * kThreads * 16;
-          if (o < page_bytes) v[u] = ld_stream(reinterpret_cast<const u32x4*>(src + o));
-        }
-#pragma unroll
-        for (int u = 0; u < kStageUnroll; ++u) {
-          const int o = o0 + u * kThreads * 16;
-          if (o < page_bytes) *reinterpret_cast<u32x4*>(lds + o) = v[u];
-        }
-      }
-      __syncthreads();
-      asym_quant_k<DT>(lds, codes, params, g);
+      stage_page<TEAM>(src, 16 * H * g.head_dim * elem_bytes<DT>(), lds);
+      team_sync<TEAM>();
+      asym_quant_k<DT, TEAM, KU>(lds, codes, params, g);
     } else {
-      asym_quant_k<DT>(src, codes, params, g);
+      asym_quant_k<DT, TEAM, KU>(src, codes, params, g);
     }
   } else {
-    asym_quant_v<DT, STAGED>(src, codes, params, g, lds);
+    asym_quant_v<DT, STAGED, TEAM>(src, codes, params, g, lds);
   }
 }
 
@@ -1019,11 +1051,22 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
       return rc;
     if (n_pages == 0) return ok();
     const bool staged = lds_staged <= (size_t)kAsymLdsBytes;
-#define AMF_LAUNCH(ST)                                                                         \
-  int4_asym_quant_gather_kernel<DT, ST><<<grid, kThreads, ST ? lds_staged : lds_tables, s>>>(  \
-      cache_planes, cache_page_stride, block_ids, pool_pages, code_planes, param_planes, g, \
-      err_flag)
-    AMF_WITH_DTYPE(cache_dtype, if (staged) AMF_LAUNCH(true); else AMF_LAUNCH(false));
+#define AMF_LAUNCH(ST, TEAM, KU)                                                               \
+  int4_asym_quant_gather_kernel<DT, ST, TEAM, KU>                                              \
+      <<<dim3((unsigned)((n_pages + kThreads / TEAM - 1) / (kThreads / TEAM)),                 \
+              (unsigned)n_planes),                                                             \
+         kThreads, (ST ? lds_staged : lds_tables) * (kThreads / TEAM), s>>>(                   \
+          cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, code_planes,        \
+          param_planes, g, (int)(ST ? lds_staged : lds_tables), err_flag)
+    // four small pages to a workgroup while their staging fits
+    if (16 * num_heads * head_dim <= 8 * kSmallPageChunks &&
+        4 * lds_staged <= (size_t)kAsymLdsBytes) {
+      AMF_WITH_DTYPE(cache_dtype, if (16 * num_heads * g.groups <= 64) AMF_LAUNCH(true, 64, 1);
+                     else AMF_LAUNCH(true, 64, kKSaveUnroll));
+      return check_launch(who);
+    }
+    AMF_WITH_DTYPE(cache_dtype, if (staged) AMF_LAUNCH(true, kThreads, kKSaveUnroll);
+                   else AMF_LAUNCH(false, kThreads, kKSaveUnroll));
 #undef AMF_LAUNCH
     return check_launch(who);
   }
