@@ -155,7 +155,11 @@ inline int coop_blocks(const void* fn) {
 }
 
 // Smallest scale group (bytes of cache read) worth the cooperative path: a
-// smaller group's exchange costs more than its second read.
-constexpr int64_t kCoopMinGroupBytes = 4ll << 20;
+// smaller group's exchange (7 to 14 us, whatever its size) costs more than its
+// second read.  32 layers of 8 x 128, single read / two passes, us: 64 pages
+// 236 / 65, 256 pages (16 MiB) 305 / 215, 384 pages 372 / 332, 512 pages (32
+// MiB) 437 / 436, 768 pages 572 / 669; 80 layers x 777 pages of 1 x 128 (6 MiB)
+// 823 / 236.
+constexpr int64_t kCoopMinGroupBytes = 32ll << 20;
 
 }  // namespace amf

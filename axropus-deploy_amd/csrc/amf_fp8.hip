@@ -159,32 +159,49 @@ __device__ __forceinline__ float absmax16(const u32x4& v, float m) {
   return m;
 }
 
-template <int DT>
+// Small pages (kAbsUnroll / PPI vectors per lane or fewer) are read PPI at a
+// time, so that as many loads are in flight.
+template <int DT, int PPI>
 __global__ __launch_bounds__(kThreads) void fp8_absmax_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, PageGeom g,
     uint32_t* ws, int32_t* err_flag) {
+  constexpr int U = kAbsUnroll / PPI;
   const int plane = blockIdx.y;
   const int n16 = g.n_rows * g.head_dim * elem_bytes<DT>() / 16;
   float m = 0.0f;
-  for (int64_t j = blockIdx.x; j < n_pages; j += gridDim.x) {
-    const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
-    if (sp < 0 || sp >= pool) {
-      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
-      continue;
-    }
-    const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(
-        reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride);
-    for (int base = threadIdx.x; base < n16; base += kThreads * kAbsUnroll) {
-      u32x4 v[kAbsUnroll];
+  for (int64_t j0 = blockIdx.x; j0 < n_pages; j0 += (int64_t)gridDim.x * PPI) {
+    const u32x4* src[PPI];
 #pragma unroll
-      for (int u = 0; u < kAbsUnroll; ++u) {
-        const int k = base + u * kThreads;
-        if (k < n16) v[u] = ld_stream(src + k);
+    for (int p = 0; p < PPI; ++p) {
+      const int64_t j = j0 + (int64_t)p * gridDim.x;
+      src[p] = nullptr;
+      if (j < n_pages) {
+        const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
+        if (sp >= 0 && sp < pool)
+          src[p] = reinterpret_cast<const u32x4*>(
+              reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride);
+        else if (threadIdx.x == 0 && err_flag)
+          atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
       }
+    }
+    if (PPI == 1 && !src[0]) continue;
+    // PPI > 1: the page fits one step
+    for (int base = threadIdx.x; base < n16; base += kThreads * U) {
+      u32x4 v[PPI][U];
 #pragma unroll
-      for (int u = 0; u < kAbsUnroll; ++u)
-        if (base + u * kThreads < n16) m = absmax16<DT>(v[u], m);
+      for (int p = 0; p < PPI; ++p)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int k = base + u * kThreads;
+          if (PPI > 1) v[p][u] = u32x4{0, 0, 0, 0};
+          if ((PPI == 1 || src[p]) && k < n16) v[p][u] = ld_stream(src[p] + k);
+        }
+#pragma unroll
+      for (int p = 0; p < PPI; ++p)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (PPI > 1 || base + u * kThreads < n16) m = absmax16<DT>(v[p][u], m);
     }
   }
   m = wave_max_xor(m, 64);
@@ -478,19 +495,25 @@ __global__ __launch_bounds__(kThreads) void fp8_ph_quant_gather_kernel(
 }
 
 // Per-tensor save, pass 2 (after fp8_absmax_kernel): one lane = CPL
-// 8-element chunks kThreads apart, so each load instruction of a wave covers
+// 8-element chunks TEAM apart, so each load instruction of a wave covers
 // 1 KiB of whole lines (non-temporal: read once) and each code store 512
 // contiguous bytes.  Same arithmetic as fp8_quant_gather_kernel<PER_TENSOR>.
-template <int DT, int CPL>
+// TEAM lanes take a page: a wave for small pages.
+template <int DT, int CPL, int TEAM>
 __global__ __launch_bounds__(kThreads) void fp8_tensor_quant_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    PageGeom g, const uint32_t* __restrict__ ws, int32_t* err_flag) {
-  const int64_t j = blockIdx.x;
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages,
+    const uint64_t* __restrict__ code_planes, PageGeom g, const uint32_t* __restrict__ ws, int32_t* err_flag) {
+  constexpr int kPages = kThreads / TEAM;
+  const int64_t j =
+      (int64_t)blockIdx.x * kPages +
+      (kPages > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM) : 0);
+  if (kPages > 1 && j >= n_pages) return;
+  const int tid = kPages > 1 ? threadIdx.x % TEAM : threadIdx.x;
   const int plane = blockIdx.y;
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
   if (sp < 0 || sp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    if (tid == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
     return;
   }
   const int64_t page_elems = (int64_t)g.n_rows * g.head_dim;
@@ -501,7 +524,7 @@ __global__ __launch_bounds__(kThreads) void fp8_tensor_quant_kernel(
   float x[CPL][8];
 #pragma unroll
   for (int i = 0; i < CPL; ++i)
-    load8_stream<DT>(src + (int64_t)(threadIdx.x + i * kThreads) * (8 * elem_bytes<DT>()), x[i]);
+    load8_stream<DT>(src + (int64_t)(tid + i * TEAM) * (8 * elem_bytes<DT>()), x[i]);
   const float a = fmaxf(u2f(ws[plane / g.pps]), tensor_floor<DT>());
   // amf_codec.py:191 divides by max(scale, 1e-12); only a zero absmax (an
   // fp16 cache, whose floor rounds to 0) reaches that clamp.
@@ -514,7 +537,7 @@ __global__ __launch_bounds__(kThreads) void fp8_tensor_quant_kernel(
     u32x2 c;
     c[0] = f32x4_to_e4m3(x[i]);
     c[1] = f32x4_to_e4m3(x[i] + 4);
-    st_stream(c, codes + threadIdx.x + i * kThreads);
+    st_stream(c, codes + tid + i * TEAM);
   }
 }
 
@@ -903,10 +926,15 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
     const int64_t per_plane = std::max<int64_t>(
         1, std::min<int64_t>(n_pages, (kAbsBlocks + n_planes - 1) / n_planes));
     dim3 agrid((unsigned)per_plane, (unsigned)n_planes);
-    AMF_WITH_DTYPE(cache_dtype,
-                   fp8_absmax_kernel<DT><<<agrid, kThreads, 0, s>>>(
-                       cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, g, ws,
-                       err_flag));
+    const int64_t lane_vecs =
+        ((int64_t)g.n_rows * head_dim * cache_elem_bytes(cache_dtype) / 16 + kThreads - 1) /
+        kThreads;
+#define AMF_LAUNCH(P)                                                                     \
+  fp8_absmax_kernel<DT, P><<<agrid, kThreads, 0, s>>>(                                    \
+      cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, g, ws, err_flag)
+    AMF_WITH_DTYPE(cache_dtype, if (lane_vecs == 1) AMF_LAUNCH(8);
+                   else if (lane_vecs == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
+#undef AMF_LAUNCH
   }
   // Per-tensor pass 2: pages of 1-16 chunks of 8 elements per lane take the
   // register-resident whole-line kernel.
@@ -914,15 +942,18 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
   const int64_t tcpl = page_chunks % kThreads == 0 ? page_chunks / kThreads : 0;
   if (pt && cache_dtype != AMF_DTYPE_F32 &&
       (tcpl == 1 || tcpl == 2 || tcpl == 4 || tcpl == 8 || tcpl == 16)) {
-#define AMF_LAUNCH(C)                                                                          \
-  AMF_WITH_DTYPE(cache_dtype, fp8_tensor_quant_kernel<DT, C><<<grid, kThreads, 0, s>>>(        \
-                                  cache_planes, cache_page_stride, block_ids, pool_pages,      \
-                                  code_planes, g, ws, err_flag))
-    if (tcpl == 1) AMF_LAUNCH(1);
-    else if (tcpl == 2) AMF_LAUNCH(2);
-    else if (tcpl == 4) AMF_LAUNCH(4);
-    else if (tcpl == 8) AMF_LAUNCH(8);
-    else AMF_LAUNCH(16);
+    const dim3 tgrid((unsigned)((n_pages + kThreads / 64 - 1) / (kThreads / 64)),
+                     (unsigned)n_planes);
+#define AMF_LAUNCH(C, TEAM)                                                                    \
+  AMF_WITH_DTYPE(cache_dtype, fp8_tensor_quant_kernel<DT, C, TEAM>                             \
+                 <<<TEAM == 64 ? tgrid : grid, kThreads, 0, s>>>(                              \
+                     cache_planes, cache_page_stride, block_ids, pool_pages, n_pages,          \
+                     code_planes, g, ws, err_flag))
+    if (tcpl == 1) AMF_LAUNCH(4, 64);  // pages of at most kSmallPageChunks: a wave each
+    else if (tcpl == 2) AMF_LAUNCH(8, 64);
+    else if (tcpl == 4) AMF_LAUNCH(4, kThreads);
+    else if (tcpl == 8) AMF_LAUNCH(8, kThreads);
+    else AMF_LAUNCH(16, kThreads);
 #undef AMF_LAUNCH
     AMF_WITH_DTYPE(cache_dtype, fp8_tensor_finalize_kernel<DT>
                    <<<(n_planes + 255) / 256, 256, 0, s>>>(param_planes, ws, n_planes, g.pps));

@@ -143,13 +143,22 @@ constexpr int kBigThreads = 1024;
 // 108 us (6.19 TB/s); one layer's 64 blocks of 8 heads 39 -> 16 us.
 // SLOTS: the page's rows are cache rows named by token slots (zeros past the
 // sequence's end), read in place instead of from a gathered copy.
+// NT = 64: a wave per (small) page, four to a workgroup.
 template <bool BF16, int CPL, int NT, bool SLOTS>
-__global__ __launch_bounds__(NT, NT > kThreads && CPL <= 8 ? 8 : 1) void
+__global__ __launch_bounds__(NT < kThreads ? kThreads : NT,
+                             CPL <= 8 && (NT > kThreads || !BF16) ? 8 : 1) void
 int4_symblock_quant_gather_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    const uint64_t* __restrict__ param_planes, SymGeom g, SlotRows rows, int32_t* err_flag) {
-  const int64_t j = blockIdx.x;
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages,
+    const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes,
+    SymGeom g, SlotRows rows, int32_t* err_flag) {
+  static_assert(NT >= kThreads || (NT == 64 && !SLOTS), "the slot form takes whole workgroups");
+  constexpr int kPages = NT < kThreads ? kThreads / NT : 1;
+  const int64_t j =
+      (int64_t)blockIdx.x * kPages +
+      (kPages > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0);
+  if (kPages > 1 && j >= n_pages) return;
+  const int tid = kPages > 1 ? threadIdx.x % NT : threadIdx.x;
   const int plane = blockIdx.y;
   __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
   const int n8 = (int)((int64_t)g.n_rows * g.head_dim / 8);
@@ -159,7 +168,7 @@ int4_symblock_quant_gather_kernel(
   } else {
     const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
     if (sp < 0 || sp >= pool) {
-      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      if (tid == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
       return;
     }
     src += sp * cache_stride;
@@ -172,7 +181,7 @@ int4_symblock_quant_gather_kernel(
     const uint32_t cpt = (uint32_t)n8 / (uint32_t)rows.page_tokens;  // chunks per token row
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-      const uint32_t k = threadIdx.x + i * NT;
+      const uint32_t k = tid + i * NT;
       v[i] = u32x4{0, 0, 0, 0};
       if (k < (uint32_t)n8) {
         const uint32_t t = k / cpt;
@@ -183,31 +192,33 @@ int4_symblock_quant_gather_kernel(
   } else {
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-      const int k = threadIdx.x + i * NT;
+      const int k = tid + i * NT;
       if (k < n8) v[i] = ld_stream(reinterpret_cast<const u32x4*>(src) + k);
     }
   }
   float m = 0.0f;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    if (threadIdx.x + i * NT < n8) {
+    if (tid + i * NT < n8) {
       float x[8];
       unpack8<BF16>(v[i], x);
 #pragma unroll
       for (int n = 0; n < 8; ++n) m = fmaxf(m, fabsf(x[n]));
     }
   }
-  m = wave_max_xor(m, 64);
-  __shared__ float s_wmax[NT / 64];
-  if ((threadIdx.x & 63) == 0) s_wmax[threadIdx.x >> 6] = m;
-  __syncthreads();
-  float amax = s_wmax[0];
+  float amax = wave_max_xor(m, 64);
+  if constexpr (NT > 64) {
+    __shared__ float s_wmax[NT / 64];
+    if ((tid & 63) == 0) s_wmax[tid >> 6] = amax;
+    __syncthreads();
+    amax = s_wmax[0];
 #pragma unroll
-  for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
+    for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
+  }
   // amf_codec.py:392-394: absmax.clamp_min(1e-8) / 7 in fp32.
   const float scale = fmaxf(amax, 1e-8f) / kSymMax;
   const float rscale = 1.0f / scale;
-  if (threadIdx.x == 0) params[j] = (_Float16)scale;
+  if (tid == 0) params[j] = (_Float16)scale;
   // In the large workgroups, and for fp16, the words are unpacked again: kept
   // from the maximum they would take twice the registers of the page itself
   // (234 us instead of 144).
@@ -217,7 +228,7 @@ int4_symblock_quant_gather_kernel(
   }
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
-    const int k = threadIdx.x + i * NT;
+    const int k = tid + i * NT;
     if (k < n8) {
       float x[8];
       unpack8<BF16>(v[i], x);
@@ -308,11 +319,13 @@ __global__ __launch_bounds__(kBigThreads) void int4_symblock_quant_looped_kernel
 // per channel into ws[group][head_dim].
 constexpr int kAbsmaxUnroll = 8;
 
-template <int DT>
+// Small pages are read PPI at a time, so that as many loads are in flight.
+template <int DT, int PPI>
 __global__ __launch_bounds__(kThreads) void int4_channel_absmax_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, SymGeom g,
     uint32_t* ws, int32_t* err_flag) {
+  constexpr int U = kAbsmaxUnroll / PPI;
   const int plane = blockIdx.y;
   __shared__ uint32_t s_max[1024];
   for (int d = threadIdx.x; d < g.head_dim; d += kThreads) s_max[d] = 0;
@@ -320,27 +333,40 @@ __global__ __launch_bounds__(kThreads) void int4_channel_absmax_kernel(
   float m[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) m[q] = 0.0f;
-  for (int64_t j = blockIdx.x; j < n_pages; j += gridDim.x) {
-    const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
-    if (sp < 0 || sp >= pool) {
-      if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
-      continue;
+  for (int64_t j0 = blockIdx.x; j0 < n_pages; j0 += (int64_t)gridDim.x * PPI) {
+    const uint8_t* src[PPI];
+#pragma unroll
+    for (int p = 0; p < PPI; ++p) {
+      const int64_t j = j0 + (int64_t)p * gridDim.x;
+      src[p] = nullptr;
+      if (j < n_pages) {
+        const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
+        if (sp >= 0 && sp < pool)
+          src[p] = reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride;
+        else if (threadIdx.x == 0 && err_flag)
+          atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+      }
     }
-    const uint8_t* src = reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride;
-    for (int base = threadIdx.x; base < n8; base += kThreads * kAbsmaxUnroll) {
-      float x[kAbsmaxUnroll][8];
+    if (PPI == 1 && !src[0]) continue;
+    // PPI > 1: the page fits one step
+    for (int base = threadIdx.x; base < n8; base += kThreads * U) {
+      float x[PPI][U][8];
 #pragma unroll
-      for (int u = 0; u < kAbsmaxUnroll; ++u) {
-        const int k = base + u * kThreads;
-        if (k < n8) load8_stream<DT>(src + (int64_t)k * (8 * elem_bytes<DT>()), x[u]);
-      }
+      for (int p = 0; p < PPI; ++p)
 #pragma unroll
-      for (int u = 0; u < kAbsmaxUnroll; ++u) {
-        if (base + u * kThreads < n8) {
-#pragma unroll
-          for (int q = 0; q < 8; ++q) m[q] = fmaxf(m[q], fabsf(x[u][q]));
+        for (int u = 0; u < U; ++u) {
+          const int k = base + u * kThreads;
+          if ((PPI == 1 || src[p]) && k < n8) load8_stream<DT>(src[p] + (int64_t)k * (8 * elem_bytes<DT>()), x[p][u]);
         }
-      }
+#pragma unroll
+      for (int p = 0; p < PPI; ++p)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if ((PPI == 1 || src[p]) && base + u * kThreads < n8) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) m[q] = fmaxf(m[q], fabsf(x[p][u][q]));
+          }
+        }
     }
   }
   // Lanes lane, lane + L, lane + 2L, ... of a wave (L = head_dim / 8 chunks
@@ -375,25 +401,31 @@ __global__ void fill_u32_kernel(uint32_t* p, int64_t n, uint32_t v) {
 #endif
 constexpr int kChanUnroll = AMF_CHAN_UNROLL;
 
-template <int DT>
+// TEAM lanes take a page: a wave for small pages.
+template <int DT, int TEAM>
 __global__ __launch_bounds__(kThreads) void int4_channel_quant_gather_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
-    const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
-    const uint64_t* __restrict__ param_planes, SymGeom g, const uint32_t* __restrict__ ws,
+    const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages,
+    const uint64_t* __restrict__ code_planes, const uint64_t* __restrict__ param_planes, SymGeom g, const uint32_t* __restrict__ ws,
     int32_t* err_flag) {
-  const int64_t j = blockIdx.x;
+  constexpr int kPages = kThreads / TEAM;
+  const int64_t j =
+      (int64_t)blockIdx.x * kPages +
+      (kPages > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM) : 0);
+  if (kPages > 1 && j >= n_pages) return;
+  const int tid = kPages > 1 ? threadIdx.x % TEAM : threadIdx.x;
   const int plane = blockIdx.y;
   // The group's fp16 scales (amf_codec.py:312-313), written once per group
   // by its first plane's first page.
   if (j == 0 && plane % g.pps == 0) {
     _Float16* p = reinterpret_cast<_Float16*>(param_planes[plane]);
     const uint32_t* gw = ws + (int64_t)(plane / g.pps) * g.head_dim;
-    for (int d = threadIdx.x; d < g.head_dim; d += kThreads)
+    for (int d = tid; d < g.head_dim; d += TEAM)
       p[d] = (_Float16)(fmaxf(u2f(gw[d]), 1e-8f) / kSymMax);
   }
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
   if (sp < 0 || sp >= pool) {
-    if (threadIdx.x == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
+    if (tid == 0 && err_flag) atomicOr(err_flag, AMF_ERRFLAG_BLOCK_RANGE);
     return;
   }
   const int64_t page_elems = (int64_t)g.n_rows * g.head_dim;
@@ -402,7 +434,7 @@ __global__ __launch_bounds__(kThreads) void int4_channel_quant_gather_kernel(
       reinterpret_cast<const uint8_t*>(cache_planes[plane]) + sp * cache_stride;
   uint32_t* __restrict__ codes =
       reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(code_planes[plane]) + j * (page_elems / 2));
-  const int d0 = (threadIdx.x * 8) % g.head_dim;
+  const int d0 = (tid * 8) % g.head_dim;
   const uint32_t* lw = ws + (int64_t)(plane / g.pps) * g.head_dim + d0;
   float sc[8], rc[8];
 #pragma unroll
@@ -410,16 +442,16 @@ __global__ __launch_bounds__(kThreads) void int4_channel_quant_gather_kernel(
     sc[q] = fmaxf(u2f(lw[q]), 1e-8f) / kSymMax;  // amf_codec.py:312-313
     rc[q] = 1.0f / sc[q];
   }
-  for (int base = threadIdx.x; base < n8; base += kThreads * kChanUnroll) {
+  for (int base = tid; base < n8; base += TEAM * kChanUnroll) {
     float x[kChanUnroll][8];
 #pragma unroll
     for (int u = 0; u < kChanUnroll; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < n8) load8_stream<DT>(src + (int64_t)k * (8 * elem_bytes<DT>()), x[u]);
     }
 #pragma unroll
     for (int u = 0; u < kChanUnroll; ++u) {
-      const int k = base + u * kThreads;
+      const int k = base + u * TEAM;
       if (k < n8) {
         uint32_t w = 0;
 #pragma unroll
@@ -816,18 +848,33 @@ constexpr int64_t kMaxRegChunks = 16 * kBigThreads;
 // The register-resident INT4_SYM_BLOCK save of pages of n8 <= kMaxRegChunks
 // chunks of 8 bf16 / fp16 elements.
 template <bool SLOTS>
-void launch_symblock_quant(bool bf16, int64_t n8, dim3 grid, hipStream_t s,
+void launch_symblock_quant(bool bf16, int64_t n8, int64_t n_pages, int n_planes, hipStream_t s,
                            const uint64_t* cache_planes, int64_t cache_stride,
                            const int32_t* block_ids, int64_t pool, const uint64_t* code_planes,
                            const uint64_t* param_planes, const SymGeom& g, const SlotRows& rows,
                            int32_t* err_flag) {
+  const dim3 grid((unsigned)n_pages, (unsigned)n_planes);
+  const dim3 wgrid((unsigned)((n_pages + kThreads / 64 - 1) / (kThreads / 64)),
+                   (unsigned)n_planes);
 #define AMF_LAUNCH(C, NT)                                                                     \
-  (bf16 ? int4_symblock_quant_gather_kernel<true, C, NT, SLOTS><<<grid, NT, 0, s>>>(          \
-              cache_planes, cache_stride, block_ids, pool, code_planes, param_planes, g,      \
-              rows, err_flag)                                                                 \
-        : int4_symblock_quant_gather_kernel<false, C, NT, SLOTS><<<grid, NT, 0, s>>>(         \
-              cache_planes, cache_stride, block_ids, pool, code_planes, param_planes, g,      \
-              rows, err_flag))
+  (bf16 ? int4_symblock_quant_gather_kernel<true, C, NT, SLOTS>                               \
+              <<<NT == 64 ? wgrid : grid, NT == 64 ? kThreads : NT, 0, s>>>(                  \
+                  cache_planes, cache_stride, block_ids, pool, n_pages, code_planes,          \
+                  param_planes, g, rows, err_flag)                                            \
+        : int4_symblock_quant_gather_kernel<false, C, NT, SLOTS>                              \
+              <<<NT == 64 ? wgrid : grid, NT == 64 ? kThreads : NT, 0, s>>>(                  \
+                  cache_planes, cache_stride, block_ids, pool, n_pages, code_planes,          \
+                  param_planes, g, rows, err_flag))
+  if constexpr (!SLOTS) {
+    if (n8 <= 256) {
+      AMF_LAUNCH(4, 64);
+      return;
+    }
+    if (n8 <= kSmallPageChunks) {
+      AMF_LAUNCH(8, 64);
+      return;
+    }
+  }
   if (n8 <= 256) AMF_LAUNCH(1, 256);
   else if (n8 <= 512) AMF_LAUNCH(2, 256);
   else if (n8 <= 1024) AMF_LAUNCH(4, 256);
@@ -1018,9 +1065,8 @@ extern "C" int amf_int4_quant_gather_slots(
                 "%s: INT4_SYM_BLOCK pages of at most %lld bf16 / fp16 elements only", who,
                 (long long)(8 * kMaxRegChunks));
   if (n_pages == 0) return ok();
-  launch_symblock_quant<true>(cache_dtype == AMF_DTYPE_BF16, n8,
-                              dim3((unsigned)n_pages, (unsigned)n_planes), as_stream(stream),
-                              cache_planes, cache_page_stride, nullptr, 0, code_planes,
+  launch_symblock_quant<true>(cache_dtype == AMF_DTYPE_BF16, n8, n_pages, n_planes,
+                              as_stream(stream), cache_planes, cache_page_stride, nullptr, 0, code_planes,
                               param_planes, g, rows, err_flag);
   return check_launch(who);
 }
@@ -1088,7 +1134,7 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
                          param_planes, g, err_flag));
       return check_launch(who);
     }
-    launch_symblock_quant<false>(bf16, n8, grid, s, cache_planes, cache_page_stride, block_ids,
+    launch_symblock_quant<false>(bf16, n8, n_pages, n_planes, s, cache_planes, cache_page_stride, block_ids,
                                  pool_pages, code_planes, param_planes, g, SlotRows{}, err_flag);
     return check_launch(who);
   }
@@ -1104,11 +1150,22 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
 #define AMF_ABSMAX_WGS 64
 #endif
   dim3 rgrid((unsigned)(n_pages < AMF_ABSMAX_WGS ? n_pages : AMF_ABSMAX_WGS), (unsigned)n_planes);
-  AMF_WITH_DTYPE(cache_dtype, int4_channel_absmax_kernel<DT><<<rgrid, kThreads, 0, s>>>(
-                                  cache_planes, cache_page_stride, block_ids, pool_pages, n_pages,
-                                  g, ws, err_flag));
-  AMF_WITH_DTYPE(cache_dtype, int4_channel_quant_gather_kernel<DT><<<grid, kThreads, 0, s>>>(
-                                  cache_planes, cache_page_stride, block_ids, pool_pages,
-                                  code_planes, param_planes, g, ws, err_flag));
+  const int64_t lane_chunks = ((int64_t)g.n_rows * head_dim / 8 + kThreads - 1) / kThreads;
+#define AMF_LAUNCH(P)                                                                   \
+  int4_channel_absmax_kernel<DT, P><<<rgrid, kThreads, 0, s>>>(                         \
+      cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, g, ws, err_flag)
+  AMF_WITH_DTYPE(cache_dtype, if (lane_chunks == 1) AMF_LAUNCH(8);
+                 else if (lane_chunks == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
+#undef AMF_LAUNCH
+#define AMF_LAUNCH(TEAM)                                                                      \
+  AMF_WITH_DTYPE(cache_dtype, int4_channel_quant_gather_kernel<DT, TEAM>                      \
+                 <<<dim3((unsigned)((n_pages + kThreads / TEAM - 1) / (kThreads / TEAM)),     \
+                         (unsigned)n_planes),                                                 \
+                    kThreads, 0, s>>>(cache_planes, cache_page_stride, block_ids, pool_pages, \
+                                      n_pages, code_planes, param_planes, g, ws, err_flag))
+  // a wave's pass of 512 elements keeps a lane's channels as well
+  if ((int64_t)g.n_rows * head_dim <= 8 * kSmallPageChunks && 512 % head_dim == 0) AMF_LAUNCH(64);
+  else AMF_LAUNCH(kThreads);
+#undef AMF_LAUNCH
   return check_launch(who);
 }

@@ -198,7 +198,7 @@ int amf_kv_scatter_slots(const uint64_t* in_planes, int64_t in_row_stride,
  * buffer of amf_quant_workspace_bytes() bytes (may be NULL when that is 0);
  * its contents on entry do not matter.  The per-tensor format reads the cache
  * once through a cooperative launch when the device supports it and a scale
- * group (planes_per_scale planes of n_pages pages, at least 4 MiB) fits the
+ * group (planes_per_scale planes of n_pages pages, at least 32 MiB) fits the
  * resident grid, and twice (absmax kernel, then quantize kernel) otherwise
  * or when AMF_NO_COOP is set to a non-zero value in the environment (read
  * once; for processes that cannot have a cooperative launch, such as a

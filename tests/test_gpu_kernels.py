@@ -161,11 +161,10 @@ def test_fp8_tensor_format_bitexact(dtype, geom):
     _check_restored(target, dst_ids, want, dtype, geom)
 
 
-# Scale groups of at least 4 MiB whose pages are whole multiples of 256
-# 16-byte chunks take the single-read cooperative kernel: an odd group count
-# (the last group has no partner buffer), one page per workgroup (CPT 8),
-# several pages per workgroup (CPT 1), and two pages per workgroup of CPT 8
-# (1200-page groups: more than the 768 workgroups that 256 CUs keep resident).
+# Per-tensor saves on both sides of the 32 MiB scale group from which the
+# single-read cooperative kernel runs: an odd group count, small pages, and
+# two pages per workgroup of the cooperative kernel (1200-page groups: more
+# than the 768 workgroups that 256 CUs keep resident).
 COOP_CASES = [
     pytest.param(torch.bfloat16, dict(L=3, pool=512, n=160, bs=16, H=8, D=128), id="bf16-3groups"),
     pytest.param(torch.float16, dict(L=2, pool=2048, n=1200, bs=16, H=2, D=64), id="fp16-cpt1"),
