@@ -302,6 +302,13 @@ __device__ __forceinline__ int64_t sk_total_units(const DecodeArgs& a, int n_seq
   return uni64(wave_sum_i64(t) * a.num_kv_heads);
 }
 
+// Quotient of non-negative wave-uniform values, in 32 bits where they fit (a
+// 64-bit division is a chain of about a hundred scalar instructions).
+__device__ __forceinline__ int64_t sk_div(int64_t x, int64_t y) {
+  if ((uint64_t)(x | y) >> 32 == 0) return (int64_t)((uint32_t)x / (uint32_t)y);
+  return x / y;
+}
+
 // Sequence s holding unit u0 < C, and the units P before it.
 __device__ __forceinline__ void sk_locate(const DecodeArgs& a, int n_seqs, int64_t u0, int* s_out,
                                           int64_t* p_out) {
@@ -329,7 +336,7 @@ __device__ __forceinline__ void sk_locate(const DecodeArgs& a, int n_seqs, int64
 
 // Wave holding unit u: the largest w with w C / G <= u.
 __device__ __forceinline__ int64_t sk_wave_of(int64_t u, int64_t total, int64_t G) {
-  return ((u + 1) * G - 1) / total;
+  return sk_div((u + 1) * G - 1, total);
 }
 
 // 8 output elements at element offset `row` of the output, in its dtype.
@@ -966,7 +973,7 @@ void int4_decode_mfma_kernel(DecodeArgs a) {
   // The merge finds a pair's waves from the units before its sequence, which
   // the wave holding the sequence's first unit records, and from the total.
   if (w == 0 && lane == 0) a.sk_meta[a.num_seqs] = total;
-  const int64_t u0 = uni64(w * total / G), u1 = uni64((w + 1) * total / G);
+  const int64_t u0 = uni64(sk_div(w * total, G)), u1 = uni64(sk_div((w + 1) * total, G));
   if (u0 >= u1) return;
   int s = 0;
   int64_t P = 0;  // units before sequence s
@@ -1358,21 +1365,32 @@ __global__ __launch_bounds__(64) void int4_decode_valu_kernel(DecodeArgs a) {
 
 // ================================================================ merge ====
 
-// Stream-K merge: one wave per (query head, sequence).  The pair's parts are
+// Stream-K merge: W waves per (query head, sequence).  The pair's parts are
 // the slots of waves wf..wl (the first one's slot 1 when its share began in
 // an earlier pair), found from the units before the sequence (sk_meta, written
 // by the decode launch) with the decode's own share arithmetic; a pair one
-// wave held was finished by it.  Lane k reads (m, l) of part k; lane (half, c)
-// reads dims 4c .. 4c + 3 of parts half, half + 2, ...; the first kSkPre of
-// those are loaded with the (m, l) words, before the maximum is known, so the
-// merge waits on memory once for up to 2 kSkPre parts.  A map entry that
-// this call's decode launch did not write raises AMF_ERRFLAG_SYNC (the
-// output is then invalid) and is never used as an address.
+// wave held was finished by it.  Every wave reads all (m, l), lane k those of
+// part k, and finds the maximum and the sum; lane (half, c) of wave w reads
+// dims 4c .. 4c + 3 of parts 2w + half, 2w + half + 2W, ... with their m, the
+// first kSkPre of them before the maximum is known, so the merge waits on
+// memory once for up to 2 W kSkPre parts, and then kSkPre at a time.  A map
+// entry that this call's decode launch did not write raises
+// AMF_ERRFLAG_SYNC (the output is then invalid) and is never used as an
+// address.
+// Short batches cut a pair into many parts (one unit a wave): with one wave
+// per row 16 parts were loaded at once and the rest in a dependent loop.
+// Decode and merge, 32 / 8 heads, one wave before / now, us: 1 x 4000 tokens
+// 30.7 / 12.9, 4 x 2000 22.1 / 14.1, 2 x 1100 14.3 / 11.1; 8 / 1 heads 1 x 8000
+// 54.8 / 15.3.  Up to kSkWideParts parts one wave a row is the faster (32 x 500
+// tokens, 12 parts: 17.7 us, four waves 18.4).
+constexpr int64_t kSkWideParts = 16;
 constexpr int kSkPre = 8;
 
-template <int OUT_DTYPE>
-__global__ __launch_bounds__(64) void int4_decode_merge_sk_kernel(DecodeArgs a) {
-  const int qhd = blockIdx.x, s = blockIdx.y, lane = threadIdx.x;
+template <int OUT_DTYPE, int W>
+__global__ __launch_bounds__(64 * W) void int4_decode_merge_sk_kernel(DecodeArgs a) {
+  __shared__ __attribute__((aligned(16))) float red[W][kD];
+  const int qhd = blockIdx.x, s = blockIdx.y, lane = threadIdx.x & 63;
+  const int w = W > 1 ? uni32(threadIdx.x >> 6) : 0;
   const int half = lane >> 5, c = lane & 31;
   const int R = a.num_q_heads / a.num_kv_heads;
   // context length and the map are independent loads; an empty sequence
@@ -1385,7 +1403,8 @@ __global__ __launch_bounds__(64) void int4_decode_merge_sk_kernel(DecodeArgs a) 
   // a map entry outside [0, total - H nch] (not written by this call's decode
   // launch) is reported and leaves zeros instead of reading outside the slots
   const bool map_ok = P >= 0 && total > 0 && P <= total - H * nch;
-  if (nch > 0 && !map_ok && lane == 0 && a.err_flag) atomicOr(a.err_flag, AMF_ERRFLAG_SYNC);
+  if (nch > 0 && !map_ok && threadIdx.x == 0 && a.err_flag)
+    atomicOr(a.err_flag, AMF_ERRFLAG_SYNC);
   if (nch > 0 && map_ok) {
     const int64_t G = min((int64_t)a.sk_waves, total);  // as the decode launch uses it
     const int64_t pair0 = P + (int64_t)(qhd / R) * nch;
@@ -1393,18 +1412,26 @@ __global__ __launch_bounds__(64) void int4_decode_merge_sk_kernel(DecodeArgs a) 
     const int64_t wl = sk_wave_of(pair0 + nch - 1, total, G);
     if (wf == wl) return;  // one wave held the whole pair and wrote the output
     const int n_sp = (int)(wl - wf + 1);
-    const bool first_slot1 = wf * total / G < pair0;
+    const bool first_slot1 = sk_div(wf * total, G) < pair0;
     const float* base = a.ws + (wf * 2 * R + qhd % R) * kPartStride;
     auto part = [&](int k) -> const float* {
       const int slot = (k == 0 && first_slot1) ? 1 : 0;
       return base + (int64_t)((2 * k + slot) * R) * kPartStride;
     };
-    // accumulators of parts half, half + 2, ... (rows clamped into the pair's
-    // parts; a clamped row is loaded but never added)
-    float4 pre[kSkPre];
+    // accumulators and m of kSkPre of this half wave's parts from k0 on (past
+    // the last part: that one again, with a weight of zero)
+    float4 acc[kSkPre];
+    float mk[kSkPre];
+    auto load = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < kSkPre; ++j)
-      pre[j] = *reinterpret_cast<const float4*>(part(min(half + 2 * j, n_sp - 1)) + 4 * c);
+      for (int j = 0; j < kSkPre; ++j) {
+        const float* p = part(min(k0 + 2 * W * j, n_sp - 1));
+        acc[j] = *reinterpret_cast<const float4*>(p + 4 * c);
+        mk[j] = p[kD];
+      }
+    };
+    const int k_first = 2 * w + half;
+    load(k_first);
     float m0 = kNegBig, l0 = 0.0f;
     if (lane < n_sp) {
       const float2 ml = *reinterpret_cast<const float2*>(part(lane) + kD);
@@ -1414,51 +1441,42 @@ __global__ __launch_bounds__(64) void int4_decode_merge_sk_kernel(DecodeArgs a) 
     float M = m0;
     for (int k = lane + 64; k < n_sp; k += 64) M = fmaxf(M, part(k)[kD]);
     M = wave_max_xor(M, 64);
-    for (int k0 = 0; k0 < n_sp; k0 += 64) {
-      float wk = 0.0f;
-      if (k0 + lane < n_sp) {
-        float mk = m0, lk = l0;
-        if (k0 != 0) {
-          const float2 ml = *reinterpret_cast<const float2*>(part(k0 + lane) + kD);
-          mk = ml.x;
-          lk = ml.y;
-        }
-        wk = exp2_fast(mk - M);
-        L += wk * lk;
-      }
-      const int cnt = min(64, n_sp - k0);
-      int j0 = 0;
-      if (k0 == 0) {
+    L = l0 * exp2_fast(m0 - M);
+    for (int k = lane + 64; k < n_sp; k += 64) {
+      const float2 ml = *reinterpret_cast<const float2*>(part(k) + kD);
+      L += ml.y * exp2_fast(ml.x - M);
+    }
+    for (int k0 = k_first;;) {
 #pragma unroll
-        for (int j = 0; j < kSkPre; ++j) {
-          const float wj = __shfl(wk, half + 2 * j);  // every lane shuffles
-          if (half + 2 * j < cnt) {
-            o.x += wj * pre[j].x;
-            o.y += wj * pre[j].y;
-            o.z += wj * pre[j].z;
-            o.w += wj * pre[j].w;
-          }
-        }
-        j0 = 2 * kSkPre;
+      for (int j = 0; j < kSkPre; ++j) {
+        const float wk = k0 + 2 * W * j < n_sp ? exp2_fast(mk[j] - M) : 0.0f;
+        o.x += wk * acc[j].x;
+        o.y += wk * acc[j].y;
+        o.z += wk * acc[j].z;
+        o.w += wk * acc[j].w;
       }
-#pragma unroll 4
-      for (int j = j0; j < cnt; j += 2) {
-        const int jj = j + half;
-        const float wj = __shfl(wk, min(jj, 63));
-        if (jj < cnt) {
-          const float4 v = *reinterpret_cast<const float4*>(part(k0 + jj) + 4 * c);
-          o.x += wj * v.x;
-          o.y += wj * v.y;
-          o.z += wj * v.z;
-          o.w += wj * v.w;
-        }
-      }
+      k0 += 2 * W * kSkPre;
+      if (!__any(k0 < n_sp)) break;
+      load(k0);
     }
     o.x += __shfl_xor(o.x, 32);
     o.y += __shfl_xor(o.y, 32);
     o.z += __shfl_xor(o.z, 32);
     o.w += __shfl_xor(o.w, 32);
     for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
+  }
+  if constexpr (W > 1) {
+    if (half == 0) *reinterpret_cast<float4*>(&red[w][4 * c]) = o;
+    __syncthreads();
+    if (w != 0) return;
+#pragma unroll
+    for (int i = 1; i < W; ++i) {
+      const float4 r = *reinterpret_cast<const float4*>(&red[i][4 * c]);
+      o.x += r.x;
+      o.y += r.y;
+      o.z += r.z;
+      o.w += r.w;
+    }
   }
   if (half != 0) return;
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
@@ -1847,12 +1865,21 @@ extern "C" int amf_int4_paged_decode_attn(const void* q, int32_t q_dtype, void* 
   }
   dim3 mgrid((unsigned)num_q_heads, (unsigned)num_seqs);
   if (a.stream_k) {
-    if (out_dtype == AMF_DTYPE_BF16)
-      int4_decode_merge_sk_kernel<AMF_DTYPE_BF16><<<mgrid, 64, 0, st>>>(a);
-    else if (out_dtype == AMF_DTYPE_F16)
-      int4_decode_merge_sk_kernel<AMF_DTYPE_F16><<<mgrid, 64, 0, st>>>(a);
+    // parts of a pair if every sequence is as long as the longest
+    const int64_t parts =
+        std::min<int64_t>((int64_t)a.sk_waves / ((int64_t)num_seqs * num_kv_heads),
+                          (int64_t)max_context_len / 32);
+#define AMF_LAUNCH(W)                                                                \
+  (out_dtype == AMF_DTYPE_BF16                                                       \
+       ? int4_decode_merge_sk_kernel<AMF_DTYPE_BF16, W><<<mgrid, 64 * W, 0, st>>>(a) \
+   : out_dtype == AMF_DTYPE_F16                                                      \
+       ? int4_decode_merge_sk_kernel<AMF_DTYPE_F16, W><<<mgrid, 64 * W, 0, st>>>(a)  \
+       : int4_decode_merge_sk_kernel<AMF_DTYPE_F32, W><<<mgrid, 64 * W, 0, st>>>(a))
+    if (parts > kSkWideParts)
+      AMF_LAUNCH(4);
     else
-      int4_decode_merge_sk_kernel<AMF_DTYPE_F32><<<mgrid, 64, 0, st>>>(a);
+      AMF_LAUNCH(1);
+#undef AMF_LAUNCH
   } else if (out_dtype == AMF_DTYPE_BF16) {
     int4_decode_merge_kernel<AMF_DTYPE_BF16><<<mgrid, kMergeThreads, 0, st>>>(a);
   } else if (out_dtype == AMF_DTYPE_F16) {
