@@ -234,9 +234,17 @@ def check(func: str, rc: int) -> None:
         raise AmfHipError(func, rc, msg.decode() if msg else "")
 
 
+_FNS: dict = {}  # (name) -> bound entry point of the loaded library
+
+
 def call(func: str, *args) -> None:
     """Call a status-returning entry point and raise on failure."""
-    check(func, getattr(load(), func)(*args))
+    fn = _FNS.get(func)
+    if fn is None:
+        fn = _FNS[func] = getattr(load(), func)
+    rc = fn(*args)
+    if rc != OK:
+        check(func, rc)
 
 
 # ---------------------------------------------------------------- helpers --
@@ -308,8 +316,8 @@ def address_table(addrs: Sequence[int], device):
     reads."""
     import torch
 
-    dev = torch.device(device)
-    key = (dev.type, dev.index, tuple(map(int, addrs)))
+    dev = device if isinstance(device, torch.device) else torch.device(device)
+    key = (dev.type, dev.index, *addrs)
     sid = stream_handle(dev)
     with _lock:
         hit = _TABLES.get(key)
@@ -321,7 +329,7 @@ def address_table(addrs: Sequence[int], device):
             t.record_stream(torch.cuda.current_stream(dev))
             streams.add(sid)
         return t
-    t = to_device(torch.tensor(list(key[2]), dtype=torch.int64), dev)
+    t = to_device(torch.tensor([int(x) for x in addrs], dtype=torch.int64), dev)
     with _lock:
         _TABLES[key] = (t, {sid})
         while len(_TABLES) > _TABLES_MAX:

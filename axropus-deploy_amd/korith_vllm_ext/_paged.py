@@ -245,7 +245,11 @@ def cache_view(gpu_cache: Sequence[torch.Tensor]) -> CacheView:
     hit = _VIEWS.get(key)
     if hit is not None:
         refs, sigs, v = hit
-        if all(r() is t and _layout_sig(t) == sg for r, sg, t in zip(refs, sigs, gpu_cache)):
+        for r, (ptr, shape, stride), t in zip(refs, sigs, gpu_cache):
+            if (r() is not t or t.data_ptr() != ptr or t.shape != shape
+                    or t.stride() != stride):
+                break
+        else:
             _VIEWS.move_to_end(key)
             return CacheView(v.planes, v.page_stride, v.pool_pages, v.block_size, v.num_heads,
                              v.head_dim, v.dtype, v.device, keep=list(gpu_cache))
@@ -335,15 +339,25 @@ def _device_ids(ids, device) -> Optional[torch.Tensor]:
     if isinstance(ids, torch.Tensor):
         host = ids.to(torch.int32).contiguous()
     else:
-        host = torch.tensor(list(ids), dtype=torch.int32)
+        ids = ids if type(ids) is list else list(ids)
+        if torch.device(device).type == "cuda":  # straight into pinned memory
+            return torch.tensor(ids, dtype=torch.int32, pin_memory=True).to(
+                device, non_blocking=True)
+        host = torch.tensor(ids, dtype=torch.int32)
     return amf_hip.to_device(host, device)
 
 
 def check_block_ids(ids: Sequence[int], pool_pages: int, *, unique: bool) -> None:
     """Host-side validation of a block table (ValueError, like the reference's
     shape checks) so that the kernels' in-kernel skip never has to trigger."""
-    import numpy as np
-
+    if type(ids) is list and 0 < len(ids) <= 64 and set(map(type, ids)) == {int}:
+        # a short list of plain ints: cheaper without an array
+        lo, hi = min(ids), max(ids)
+        if lo < 0 or hi >= pool_pages:
+            raise ValueError(f"block id out of range [0, {pool_pages}): min {lo} max {hi}")
+        if unique and len(set(ids)) != len(ids):
+            raise ValueError("duplicate block ids in a scatter target")
+        return
     a = np.asarray(list(ids), dtype=np.int64)
     if a.size == 0:
         return
@@ -402,6 +416,21 @@ def blob_tables(layout: BlobLayout, blob_bases: Sequence[int], planes_per_blob: 
     return PlaneTables(amf_hip.address_table(codes, device), amf_hip.address_table(params, device))
 
 
+def _blob_table(layout: BlobLayout, blob_bases: Sequence[int], planes_per_blob: int,
+                device) -> Tuple[torch.Tensor, int, int]:
+    """The code and param plane tables of blob_tables in one device table:
+    (table, address of the code planes, address of the param planes)."""
+    P = planes_per_blob
+    co = [layout.code_offset(p) for p in range(P)]
+    po = [layout.param_offset(p) for p in range(P)]
+    addrs = [base + o for base in blob_bases for o in co]
+    n = len(addrs)
+    addrs += [base + o for base in blob_bases for o in po]
+    t = amf_hip.address_table(addrs, device)
+    ptr = t.data_ptr()
+    return t, ptr, ptr + 8 * n
+
+
 def quant_gather(layout: BlobLayout, view: CacheView, block_ids, blob_bases: Sequence[int],
                  planes_per_blob: int, workspace: Optional[torch.Tensor] = None,
                  err_flag: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
@@ -414,7 +443,7 @@ def quant_gather(layout: BlobLayout, view: CacheView, block_ids, blob_bases: Seq
     n_planes = len(view.planes)
     if n_planes != planes_per_blob * len(blob_bases):
         raise ValueError("plane count does not match the blobs")
-    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    _table, codes, params = _blob_table(layout, blob_bases, planes_per_blob, dev)
     ids = _device_ids(block_ids, dev)
     ws_bytes = amf_hip.quant_workspace_bytes(layout.fmt_id, n_planes, planes_per_blob, view.head_dim)
     if ws_bytes and (workspace is None or workspace.numel() * 4 < ws_bytes):
@@ -422,8 +451,8 @@ def quant_gather(layout: BlobLayout, view: CacheView, block_ids, blob_bases: Seq
     fn = "amf_fp8_quant_gather" if layout.family == "fp8" else "amf_int4_quant_gather"
     amf_hip.call(
         fn, layout.fmt_id, _ptr(amf_hip.address_table(view.planes, dev)), view.page_stride,
-        amf_hip.dtype_tag(view.dtype), _ptr(ids), view.pool_pages, _ptr(tables.codes),
-        _ptr(tables.params), n_planes, planes_per_blob, layout.n_pages, view.block_size,
+        amf_hip.dtype_tag(view.dtype), _ptr(ids), view.pool_pages, codes,
+        params, n_planes, planes_per_blob, layout.n_pages, view.block_size,
         view.num_heads, view.head_dim, _ptr(workspace),
         0 if workspace is None else workspace.numel() * 4, _ptr(err_flag),
         amf_hip.stream_handle(dev),
@@ -444,11 +473,11 @@ def dequant_scatter(layout: BlobLayout, blob_bases: Sequence[int], planes_per_bl
     n_planes = len(view.planes)
     if n_planes != planes_per_blob * len(blob_bases):
         raise ValueError("plane count does not match the blobs")
-    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    _table, codes, params = _blob_table(layout, blob_bases, planes_per_blob, dev)
     ids = _device_ids(block_ids, dev)
     fn = "amf_fp8_dequant_scatter" if layout.family == "fp8" else "amf_int4_dequant_scatter"
     amf_hip.call(
-        fn, layout.fmt_id, _ptr(tables.codes), _ptr(tables.params),
+        fn, layout.fmt_id, codes, params,
         _ptr(amf_hip.address_table(view.planes, dev)), view.page_stride,
         amf_hip.dtype_tag(view.dtype), _ptr(ids), view.pool_pages, n_planes, n,
         view.block_size, view.num_heads, view.head_dim, _ptr(err_flag), amf_hip.stream_handle(dev),
@@ -671,11 +700,11 @@ def quant_gather_slots(layout: BlobLayout, view: CacheView, slots: SlotMap,
     into the blobs at blob_bases, reading each row where it is."""
     layout.validate()
     dev = view.device
-    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    _table, codes, params = _blob_table(layout, blob_bases, planes_per_blob, dev)
     amf_hip.call(
         "amf_int4_quant_gather_slots", layout.fmt_id, _ptr(amf_hip.address_table(view.planes, dev)),
         view.page_stride, view.block_size, amf_hip.dtype_tag(view.dtype), _ptr(slots.on(dev)),
-        view.pool_pages * view.block_size, _ptr(tables.codes), _ptr(tables.params),
+        view.pool_pages * view.block_size, codes, params,
         len(view.planes), slots.n, layout.block_size, view.num_heads, view.head_dim, None,
         amf_hip.stream_handle(dev),
     )
@@ -687,11 +716,11 @@ def dequant_scatter_slots(layout: BlobLayout, blob_bases: Sequence[int], planes_
     into the cache rows of the first n slots."""
     layout.validate()
     dev = view.device
-    tables = blob_tables(layout, blob_bases, planes_per_blob, dev)
+    _table, codes, params = _blob_table(layout, blob_bases, planes_per_blob, dev)
     fn = ("amf_fp8_dequant_scatter_slots" if layout.family == "fp8"
           else "amf_int4_dequant_scatter_slots")
     amf_hip.call(
-        fn, layout.fmt_id, _ptr(tables.codes), _ptr(tables.params),
+        fn, layout.fmt_id, codes, params,
         _ptr(amf_hip.address_table(view.planes, dev)), view.page_stride, view.block_size,
         amf_hip.dtype_tag(view.dtype), _ptr(slots.on(dev)), view.pool_pages * view.block_size,
         len(view.planes), n, layout.block_size, view.num_heads, view.head_dim, None,

@@ -270,7 +270,10 @@ class _HipCodec(Codec):
         P, n, bs, H, D = (layout.n_planes, layout.n_pages, layout.block_size, layout.num_heads,
                           layout.head_dim)
         out = torch.empty(P, n, bs, H, D, dtype=target_dtype, device=blob.device)
-        view = _paged.planes_view([out[p] for p in range(P)])
+        page = bs * H * D * out.element_size()
+        base = out.data_ptr()
+        view = _paged.CacheView([base + p * n * page for p in range(P)], page, n, bs, H, D,
+                                out.dtype, out.device, keep=[out])
         _paged.dequant_scatter(layout, [blob.data_ptr()], P, view, None)
         T = compressed.meta["n_tokens"]
         return out.view(P, n * bs, H, D)[:, :T].reshape(compressed.shape)

@@ -305,6 +305,18 @@ def _check_buffer(t: torch.Tensor, what: str, dev: torch.device) -> None:
         raise ValueError(f"paged decode: {what} must be contiguous")
 
 
+def _index_tensor(t: Any, dev: torch.device) -> torch.Tensor:
+    """t as a contiguous int32 tensor on dev (itself when it is one)."""
+    if (isinstance(t, torch.Tensor) and t.dtype == torch.int32 and t.device == dev
+            and t.is_contiguous()):
+        return t
+    return torch.as_tensor(t, dtype=torch.int32).to(dev).contiguous()
+
+
+_ALGOS = {"auto": amf_hip.DECODE_AUTO, "valu": amf_hip.DECODE_VALU, "mfma": amf_hip.DECODE_MFMA,
+          "mfma_precise": amf_hip.DECODE_MFMA_PRECISE}
+
+
 def paged_int4_decode(q: torch.Tensor, kv: CompressedKV, block_tables: torch.Tensor,
                       context_lens: torch.Tensor, *, scale: Optional[float] = None,
                       max_context_len: Optional[int] = None, out: Optional[torch.Tensor] = None,
@@ -339,10 +351,10 @@ def paged_int4_decode(q: torch.Tensor, kv: CompressedKV, block_tables: torch.Ten
         raise ValueError(f"q must be [seqs, heads, D] or [seqs, heads, 1, D], got {tuple(q.shape)}")
     if q3.dtype not in (torch.bfloat16, torch.float16):
         raise TypeError(f"paged decode: q dtype {q3.dtype} is not bf16/fp16")
-    q3 = q3.to(dev).contiguous()
+    if q3.device != dev or not q3.is_contiguous():
+        q3 = q3.to(dev).contiguous()
     S, Hq, D = q3.shape
-    bt = torch.as_tensor(block_tables, dtype=torch.int32).to(dev).contiguous()
-    cl = torch.as_tensor(context_lens, dtype=torch.int32).to(dev).contiguous()
+    bt, cl = _index_tensor(block_tables, dev), _index_tensor(context_lens, dev)
     if bt.dim() != 2 or bt.shape[0] != S or cl.shape != (S,):
         raise ValueError(f"block_tables {tuple(bt.shape)} / context_lens {tuple(cl.shape)} do "
                          f"not match {S} sequences")
@@ -366,8 +378,6 @@ def paged_int4_decode(q: torch.Tensor, kv: CompressedKV, block_tables: torch.Ten
     stream = amf_hip.stream_handle(dev)
     if workspace is None or workspace.numel() * workspace.element_size() < wsb:
         workspace = _scratch(dev, stream, max(wsb, 4))
-    algos = {"auto": amf_hip.DECODE_AUTO, "valu": amf_hip.DECODE_VALU, "mfma": amf_hip.DECODE_MFMA,
-             "mfma_precise": amf_hip.DECODE_MFMA_PRECISE}
     amf_hip.call(
         "amf_int4_paged_decode_attn", q3.data_ptr(), amf_hip.dtype_tag(q3.dtype), out.data_ptr(),
         amf_hip.dtype_tag(out.dtype), blob.data_ptr() + layout.code_offset(0),
@@ -375,7 +385,7 @@ def paged_int4_decode(q: torch.Tensor, kv: CompressedKV, block_tables: torch.Ten
         blob.data_ptr() + layout.param_offset(1), layout.n_pages, bt.data_ptr(), bt.shape[1],
         cl.data_ptr(), S, Hq, layout.num_heads, D, layout.block_size, int(max_context_len),
         float(scale) if scale else 0.0, workspace.data_ptr(),
-        workspace.numel() * workspace.element_size(), algos[algo], None, stream)
+        workspace.numel() * workspace.element_size(), _ALGOS[algo], None, stream)
     return out.view(q.shape) if q.dim() == 4 else out
 
 
