@@ -18,9 +18,10 @@
 // and enter the PV tiles as a sum of 16-bit terms: three bf16 terms hold an
 // fp32 weight exactly, two fp16 terms (scaled by 2^15) hold it to 22 bits of
 // itself and 2^-38 of the row's largest.  Accumulators, maxima and sums are
-// fp32.  (Two bf16 terms would take 103 instead of 114 us at 32 / 8 heads, 512
-// rows, 4096 tokens, but are 16 bits.)
+// fp32.  (Two bf16 terms would be a tenth faster at 32 / 8 heads, 512 rows,
+// 4096 tokens, but are 16 bits.)
 #include <algorithm>
+#include <type_traits>
 
 #include "amf_attn.h"
 #include "amf_prefill.h"
@@ -105,10 +106,14 @@ __device__ __forceinline__ void weight_split(float p0, float p1,
 }
 
 // Measured (bf16, 32 / 8 heads, head_dim 128, causal mask): 512 rows x 4096
-// tokens 1285 -> 111 us (25 -> 290 TFLOP/s), 128 rows x 8192 tokens 913 ->
-// 67 us; the one-row kernel ran every row's products on the VALU and read
-// K/V from L2 once per row.  Now bound by the chain staging -> scores ->
-// softmax -> PV of two waves per SIMD (254 VGPRs), not by the MFMAs (27 us).
+// tokens 1285 -> 90 us (25 -> 360 TFLOP/s), 128 rows x 8192 tokens 913 ->
+// 65 us; the one-row kernel ran every row's products on the VALU and read
+// K/V from L2 once per row.  Now bound by the matrix cores and the VALU beside
+// them at two waves per SIMD (254 VGPRs): QK^T and three PV terms are 69 GFLOP
+// of tiles, 55 us at the rate a large library product reaches here, and the
+// softmax and the weights' terms take about as many cycles.  A second LDS
+// buffer (one barrier per tile instead of two) and other orders of the PV
+// tiles measured the same.
 //
 // NW waves of 32 query rows each share the K/V tiles.  Unit u is (b, KV head, split), served by `tiles`
 // workgroups; with xcd_map they take consecutive slots of one XCD (its L2
@@ -183,24 +188,34 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
     }
   }
   Raw kr[CH], vr[CH];
+  constexpr int RB = INT4 ? D / 2 : 2 * D, CB = INT4 ? 4 : 16;  // bytes of a row, of a chunk
+  const uint32_t lane_off = (uint32_t)(r0 * RB + c * CB);
+  // Loads of the tile at t0: a uniform base and one fixed offset per lane, or
+  // (a tile that the split's end cuts) rows clamped into the split.
   auto fetch = [&](int64_t t0) {
+    if (t0 + BT <= t_end) {
+      const uint8_t* kb = static_cast<const uint8_t*>(a.k) + (kv_base + t0) * RB;
+      const uint8_t* vb = static_cast<const uint8_t*>(a.v) + (kv_base + t0) * RB;
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int64_t t = t0 + r0 + RSTEP * i;
-      kr[i] = Raw::load(a.k, kv_base + (t < t_end ? t : t_begin), c, D);
-    }
+      for (int i = 0; i < CH; ++i) kr[i] = Raw::load(kb + i * RSTEP * RB + lane_off, 0, 0, D);
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int64_t t = t0 + r0 + RSTEP * i;
-      vr[i] = Raw::load(a.v, kv_base + (t < t_end ? t : t_begin), c, D);
+      for (int i = 0; i < CH; ++i) vr[i] = Raw::load(vb + i * RSTEP * RB + lane_off, 0, 0, D);
+    } else if (t0 < t_end) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int64_t t = t0 + r0 + RSTEP * i;
+        kr[i] = Raw::load(a.k, kv_base + (t < t_end ? t : t_begin), c, D);
+        vr[i] = Raw::load(a.v, kv_base + (t < t_end ? t : t_begin), c, D);
+      }
     }
   };
   // rows past the split are zeros (their scores are -inf below)
-  auto stage = [&](int64_t t0) {
+  auto stage = [&](auto full_c, int64_t t0) {
+    constexpr bool full = decltype(full_c)::value;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int r = r0 + RSTEP * i;
-      const bool in = t0 + r < t_end;
+      const bool in = full || t0 + r < t_end;
       uint32_t kp[4], vp[4];
       kr[i].pairs(ksc, kz, kp);
       vr[i].pairs(vsc, vz, vp);
@@ -223,29 +238,37 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   const int l16 = lane & 15;
   const uint8_t* v_rd = v_lds + (4 * h + (l16 >> 2)) * VS + 32 * ((lane >> 4) & 1) + 8 * (l16 & 3);
 
-  fetch(t_begin);
-  for (int64_t t0 = t_begin; t0 < t_end; t0 += BT) {
+  // One tile; `full` when it lies inside the split: nothing is clamped or
+  // masked per element then, which was half of the kernel's VALU work.
+  auto tile_step = [&](auto full_c, int64_t t0) {
+    constexpr bool full = decltype(full_c)::value;
     __syncthreads();  // the previous tile has been read
-    stage(t0);
+    stage(full_c, t0);
     __syncthreads();
     // token of score element i of block tb: t0 + 32 tb + 8 (i / 4) + 4 h + i % 4
     f32x4 mk[BT / 32][4];
     if (mrow) {
+      const float* mp = mrow + (t0 + 4 * h) * a.ms3;
 #pragma unroll
       for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const int64_t t = t0 + 32 * tb + 8 * g + 4 * h;
+          const int dt = 32 * tb + 8 * g;
           if (mvec) {
-            mk[tb][g] = *reinterpret_cast<const f32x4*>(mrow + (t < t_end ? t : t_begin));
+            const int64_t t = t0 + dt + 4 * h;
+            mk[tb][g] = *reinterpret_cast<const f32x4*>(full ? mp + dt
+                                                             : mrow + (t < t_end ? t : t_begin));
           } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              mk[tb][g][e] = mrow[(t + e < t_end ? t + e : t_begin) * a.ms3];
+            for (int e = 0; e < 4; ++e) {
+              const int64_t t = t0 + dt + 4 * h + e;
+              mk[tb][g][e] =
+                  full ? mp[(dt + e) * a.ms3] : mrow[(t < t_end ? t : t_begin) * a.ms3];
+            }
           }
         }
     }
-    if (t0 + BT < t_end) fetch(t0 + BT);
+    fetch(t0 + BT);
 
     f32x16 s[BT / 32];
 #pragma unroll
@@ -257,18 +280,28 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
         s[tb] = mfma32<DT>(*reinterpret_cast<const u32x4*>(k_rd + 32 * tb * KS + 32 * ks), qb[ks],
                            s[tb]);
     }
-    const bool full = t0 + BT <= t_end;
+#pragma unroll
+    for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[tb][i] *= qs;
+    if (mrow) {
+#pragma unroll
+      for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[tb][i] = fmaf(mk[tb][i >> 2][i & 3], kLog2e, s[tb][i]);
+    }
+    if constexpr (!full) {
+#pragma unroll
+      for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (t0 + 32 * tb + 8 * (i >> 2) + 4 * h + (i & 3) >= t_end) s[tb][i] = -INFINITY;
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        float x = s[tb][i] * qs;
-        if (mrow) x = fmaf(mk[tb][i >> 2][i & 3], kLog2e, x);
-        if (!full && t0 + 32 * tb + 8 * (i >> 2) + 4 * h + (i & 3) >= t_end) x = -INFINITY;
-        s[tb][i] = x;
-        mx = fmaxf(mx, x);
-      }
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[tb][i]);
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx);
     // a row with every score so far -inf keeps l = 0 and acc = 0
@@ -310,7 +343,11 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
         for (int k = 0; k < TERMS; ++k) acc[d] = mfma32<DT>(va, pb[k], acc[d]);
       }
     }
-  }
+  };
+  fetch(t_begin);
+  int64_t t0 = t_begin;
+  for (; t0 + BT <= t_end; t0 += BT) tile_step(std::true_type{}, t0);
+  if (t0 < t_end) tile_step(std::false_type{}, t0);
 
   const float l = l_run + __shfl_xor(l_run, 32);
   if (!row_ok) return;
