@@ -559,10 +559,26 @@ class CompressedVRAMPool:
             if _paged.slot_save_fits(layout, view.dtype):
                 return self._insert(prefix_hash, fmt, layout, view, None, T, (2, T, H, D),
                                     view.dtype, savings_ms, slots=slots)
-        staging = torch.empty(L, 2, T, H, D, dtype=view.dtype, device=view.device)
-        outs = [staging[l, kv].data_ptr() for l in range(L) for kv in range(2)]
-        _paged.gather_slots(view, slots, T, outs, H * D * staging.element_size())
-        return self.put_from_raw(prefix_hash, staging, format=fmt, savings_ms=savings_ms)
+        # gathered straight into the entry's pages, the last one zero-padded
+        n_pages = -(-T // page)
+        layout = self._layout(fmt, n_pages, page, H, D, view.dtype)
+        dense = self._dense_pages(2 * L, n_pages, page, H, D, view.dtype)
+        staging = dense.keep[0]
+        if n_pages * page != T:
+            staging.view(2 * L, n_pages * page, H, D)[:, T:].zero_()
+        _paged.gather_slots(view, slots, T, dense.planes, H * D * view.dtype.itemsize)
+        return self._insert(prefix_hash, fmt, layout, dense, None, T, (2, T, H, D), view.dtype,
+                            savings_ms, keep=staging)
+
+    def _dense_pages(self, n_planes: int, n_pages: int, page: int, H: int, D: int,
+                     dtype: torch.dtype) -> _paged.CacheView:
+        """n_planes dense planes of n_pages pages of page tokens, in a new
+        buffer [n_planes, n_pages, page, H, D] (the view's keep[0])."""
+        buf = torch.empty(n_planes, n_pages, page, H, D, dtype=dtype, device=self.device)
+        stride = page * H * D * dtype.itemsize
+        base = buf.data_ptr()
+        return _paged.CacheView([base + i * n_pages * stride for i in range(n_planes)], stride,
+                                n_pages, page, H, D, dtype, buf.device, keep=[buf])
 
     def restore_to_slots(self, prefix_hash: str, gpu_cache: list, slot_mapping, *,
                          first_layer: int = 0) -> int:
@@ -628,12 +644,9 @@ class CompressedVRAMPool:
                 _paged.dequant_scatter_slots(lay, bases, 2, view, slots, n)
             else:
                 pages = -(-n // P)
-                staging = torch.empty(2 * layers, pages, P, H, D, dtype=view.dtype,
-                                      device=view.device)
-                planes = [staging[i] for i in range(2 * layers)]
-                _paged.dequant_scatter(lay, bases, 2, _paged.planes_view(planes), None,
-                                       n_pages=pages)
-                _paged.scatter_slots([t.data_ptr() for t in planes], row, view, slots, n)
+                dense = self._dense_pages(2 * layers, pages, P, H, D, view.dtype)
+                _paged.dequant_scatter(lay, bases, 2, dense, None, n_pages=pages)
+                _paged.scatter_slots(dense.planes, row, view, slots, n)
             self._fence(entry)
             return n
 
