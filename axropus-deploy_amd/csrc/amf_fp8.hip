@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kThreads) void fp8_dequant_scatter_kernel(
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
     PageGeom g, SlotRows rows, int32_t* err_flag) {
   __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
-    const PageWork pw = page_work<TEAM>(n_pages, n_planes);
+  const PageWork pw = xcd_page_work<TEAM>(n_pages, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j;
   const int plane = pw.plane;
@@ -745,10 +745,10 @@ void launch_restore(int32_t format, int64_t n_pages, hipStream_t s, const uint64
                     int32_t* err_flag) {
   const bool pt = format == AMF_FMT_FP8_E4M3;
   // the slot form's row table counts towards the pad
-    const unsigned pad = kRestoreLdsPad - (SLOTS ? kMaxSlotPage * sizeof(int64_t) : 0);
+  const unsigned pad = kRestoreLdsPad - (SLOTS ? kMaxSlotPage * sizeof(int64_t) : 0);
 #define AMF_LAUNCH(T, TEAM)                                                                  \
   fp8_dequant_scatter_kernel<DT, T, SLOTS, TEAM>                                             \
-      <<<page_grid<TEAM>(n_pages, n_planes), kThreads, TEAM == kPageTeam ? pad : 0, s>>>( \
+      <<<xcd_page_grid<TEAM>(n_pages, n_planes), kThreads, TEAM == kPageTeam ? pad : 0, s>>>( \
           code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,   \
           n_planes, g, rows, err_flag)
   if constexpr (!SLOTS) {

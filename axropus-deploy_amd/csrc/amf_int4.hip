@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kThreads) void int4_sym_dequant_scatter_kernel(
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, int n_planes,
     int parts, SymGeom g, SlotRows rows, int32_t* err_flag) {
   __shared__ int64_t s_row[SLOTS ? kMaxSlotPage : 1];
-    const PageWork pw = page_work<TEAM>(n_pages * parts, n_planes);
+  const PageWork pw = xcd_page_work<TEAM>(n_pages * parts, n_planes);
   if (!pw.valid) return;
   const int64_t j = pw.j / parts;
   const int part = (int)(pw.j % parts);
@@ -546,8 +546,9 @@ __global__ __launch_bounds__(kThreads) void int4_asym_dequant_scatter_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, int64_t n_pages, AsymGeom g,
     int32_t* err_flag) {
-  // A (page, plane) grid: all XCDs work on one plane at a time, as in the other
-  // restores.
+  // A (page, plane) grid, page-major: all XCDs work on one plane at a time,
+  // which measured faster here than the XCD-contiguous map of the other
+  // restores (1.025 vs 1.065 ms at 32 layers x 2048 pages).
   constexpr int kPages = kThreads / TEAM;
   const int64_t j =
       (int64_t)blockIdx.x * kPages +
@@ -904,7 +905,7 @@ int launch_sym_restore(const char* who, int32_t format, int64_t n_pages, hipStre
                 who, (long long)n_pages, parts, n_planes);
 #define AMF_LAUNCH(C, TEAM)                                                                  \
   int4_sym_dequant_scatter_kernel<DT, C, SLOTS, TEAM>                                        \
-      <<<page_grid<TEAM>(n_pages * parts, n_planes), kThreads, 0, s>>>(                  \
+      <<<xcd_page_grid<TEAM>(n_pages * parts, n_planes), kThreads, 0, s>>>(                  \
           code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,   \
           n_planes, parts, g, rows, err_flag)
   if constexpr (!SLOTS) {

@@ -19,25 +19,23 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ---- restore work mapping ------------------------------------------------------
 // The FP8 and INT4-sym restores write whole pages at block-table-chosen
-// places, on a 1-D grid over the plane-major (plane, page) list, so the pages
-// in flight come from one or two planes.  (Handing each XCD a contiguous
-// eighth of that list measured slower: 32 layers x 512 pages of 8 x 128, us,
-// fp8_e4m3_ph 294 against 278, int4_sym 255 against 238.)  The FP8 restore is
-// launched with kRestoreLdsPad bytes of (unused) dynamic LDS, which holds a CU
-// to four of its workgroups: fewer pages in flight, still enough bytes in
-// flight for the HBM (two / three / four / five / eight workgroups: 330 / 280 /
-// 278 / 281 / 282 us there, 330 / 273 / 267 / 285 / 291 us at 1000 pages of 4 x
-// 128; the INT4 restores, which write four times what they read, lose with
-// the pad).
-constexpr unsigned kRestoreLdsPad = 39u << 10;
+// places.  Their grid is 1-D: workgroup id runs on XCD id % 8 (round-robin
+// dispatch), and xcd_page_work gives XCD x the contiguous eighth x of the
+// plane-major (plane, page) list, so each XCD's in-flight pages come from one
+// or two planes instead of from every plane.  The FP8 restore is launched
+// with kRestoreLdsPad bytes of (unused) dynamic LDS, which holds a CU to
+// three of its workgroups: fewer pages in flight per XCD, still enough bytes
+// in flight for the HBM (the INT4 restores, which write four times what they
+// read, lose with the pad).
+constexpr unsigned kRestoreLdsPad = 52u << 10;
 
 // A page takes one workgroup of kPageTeam lanes, or, when it is small (at most
 // kSmallPageChunks chunks of 8 elements: one or two KV heads of a
 // tensor-parallel rank), one wave, four pages to a workgroup: with a 4 KiB page
 // per workgroup the chip waits for workgroups to start.  80 layers x 777 pages
 // of 1 x 128, a workgroup / a wave per page, us: fp8_e4m3 279 / 138,
-// fp8_e4m3_ph 312 / 139, int4_sym 193 / 107; 32 x 1000 of 2 x 128: 164 / 138,
-// 205 / 138, 150 / 116.  Pages of 4 x 128 run at 5.7 TB/s as workgroups.
+// fp8_e4m3_ph 312 / 138, int4_sym 193 / 117; 32 x 1000 of 2 x 128: 164 / 148,
+// 205 / 146, 150 / 127.  Pages of 4 x 128 run at 5.2-5.6 TB/s as workgroups.
 constexpr int kPageTeam = 256;
 constexpr int64_t kSmallPageChunks = 512;
 
@@ -47,11 +45,19 @@ struct PageWork {
   bool valid;  // false for the padding teams
 };
 
+// Workgroups of each XCD over n_pages x n_planes pages, TEAM lanes a page.
+template <int TEAM>
+__host__ __device__ inline uint32_t xcd_page_groups(int64_t n_pages, int n_planes) {
+  constexpr int kPages = kPageTeam / TEAM;
+  return (uint32_t)((n_pages * n_planes + 8 * kPages - 1) / (8 * kPages));
+}
+
 // n_pages * n_planes < 2^31 (checked on the host).
 template <int TEAM>
-__device__ __forceinline__ PageWork page_work(int64_t n_pages, int n_planes) {
+__device__ __forceinline__ PageWork xcd_page_work(int64_t n_pages, int n_planes) {
   constexpr int kPages = kPageTeam / TEAM;
-  uint32_t w = blockIdx.x * kPages;
+  const uint32_t id = blockIdx.x;
+  uint32_t w = ((id & 7) * xcd_page_groups<TEAM>(n_pages, n_planes) + (id >> 3)) * kPages;
   if constexpr (kPages > 1) w += __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM);
   PageWork r;
   r.valid = w < (uint32_t)(n_pages * n_planes);
@@ -61,9 +67,8 @@ __device__ __forceinline__ PageWork page_work(int64_t n_pages, int n_planes) {
 }
 
 template <int TEAM>
-inline dim3 page_grid(int64_t n_pages, int n_planes) {
-  constexpr int kPages = kPageTeam / TEAM;
-  return dim3((unsigned)((n_pages * n_planes + kPages - 1) / kPages));
+inline dim3 xcd_page_grid(int64_t n_pages, int n_planes) {
+  return dim3(8 * xcd_page_groups<TEAM>(n_pages, n_planes));
 }
 
 // ---- token slots ----------------------------------------------------------------
