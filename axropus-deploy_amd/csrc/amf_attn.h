@@ -32,6 +32,15 @@ struct AttnArgs {
   const _Float16* v_scales;
 };
 
+// Scores, maxima and the splits' m are base-2 logarithms (scaled by log2(e))
+// without a mask.  With one they stay natural logarithms and their differences
+// are scaled before 2^x: a mask's lowest finite value times log2(e) would be
+// -inf, and a row masked with it everywhere NaN instead of its tokens' mean.
+__host__ __device__ inline float score_scale(const AttnArgs& a) {
+  return a.mask ? a.scale : a.scale * kLog2e;
+}
+__host__ __device__ inline float exp2_factor(const AttnArgs& a) { return a.mask ? kLog2e : 1.0f; }
+
 constexpr int kPartPad = 4;            // a split partial: acc[D], m, l, 2 pad (16-byte rows)
 constexpr int64_t kXcds = 8;           // XCDs of the chip, dealt workgroups round-robin
 

@@ -117,6 +117,7 @@ __global__ __launch_bounds__(kThreads) void dense_attn_kernel(AttnArgs a) {
 
   const int64_t kv_base = (b * a.num_kv_heads + hkv) * T;  // first token row of this (b, hkv)
   const float* mrow = a.mask ? a.mask + b * a.ms0 + (int64_t)h * a.ms1 + tq * a.ms2 : nullptr;
+  const float e2 = exp2_factor(a);
 
   float m_run = -INFINITY, l_run = 0.0f;
   float acc[kAccPerLane];
@@ -140,15 +141,14 @@ __global__ __launch_bounds__(kThreads) void dense_attn_kernel(AttnArgs a) {
         for (int d = 0; d < D; ++d) dot = fmaf(q_s[d], elem<DT>(a.k, kr + d), dot);
       }
       s = dot * a.scale;
-      if (mrow) s += mrow[t * a.ms3];
-      s *= kLog2e;
+      s = mrow ? s + mrow[t * a.ms3] : s * kLog2e;
     }
     float m_chunk = s;
     for (int off = 32; off > 0; off >>= 1) m_chunk = fmaxf(m_chunk, __shfl_xor(m_chunk, off));
     const float m_new = fmaxf(m_run, m_chunk);
     if (m_new == -INFINITY) continue;  // every score so far is -inf (wave-uniform)
-    const float alpha = exp2f(m_run - m_new);
-    const float p = (s == -INFINITY) ? 0.0f : exp2f(s - m_new);
+    const float alpha = exp2f((m_run - m_new) * e2);
+    const float p = (s == -INFINITY) ? 0.0f : exp2f((s - m_new) * e2);
     l_run = l_run * alpha + wave_sum(p);
 #pragma unroll
     for (int j = 0; j < kAccPerLane; ++j) acc[j] *= alpha;
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kThreads) void dense_attn_kernel(AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < kWaves; ++i) {
         if (m_s[i] == -INFINITY) continue;
-        const float f = exp2f(m_s[i] - M);
+        const float f = exp2f((m_s[i] - M) * e2);
         num = fmaf(acc_s[i][d], f, num);
         den = fmaf(l_s[i], f, den);
       }
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(64) void dense_attn_split_kernel(AttnArgs a, float*
   const int64_t T = a.kv_len;
   const int64_t t_begin = split * split_tokens, t_end = min(T, t_begin + split_tokens);
   const int64_t kv_base = (b * a.num_kv_heads + hkv) * T;
-  const float qs = a.scale * kLog2e;
+  const float qs = score_scale(a), e2 = exp2_factor(a);
   // query row of head h0 + j: (b, h0 + j, tq) flattened
   auto qrow = [&](int j) { return (b * a.num_q_heads + h0 + j) * a.q_len + tq; };
 
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(64) void dense_attn_split_kernel(AttnArgs a, float*
 #pragma unroll
         for (int i = 0; i < SB; ++i) {
           const int64_t t = t0 + TPS * i + g;
-          sc[j][i] = fmaf(mrow[(t < t_end ? t : t_begin) * a.ms3], kLog2e, sc[j][i]);
+          sc[j][i] += mrow[(t < t_end ? t : t_begin) * a.ms3];
         }
       }
     }
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(64) void dense_attn_split_kernel(AttnArgs a, float*
 #pragma unroll
     for (int j = 0; j < GH; ++j) {
       // a head with every score so far -inf keeps l = 0, acc = 0
-      const float alpha = m_new[j] == -INFINITY ? 1.0f : exp2f(m_run[j] - m_new[j]);
+      const float alpha = m_new[j] == -INFINITY ? 1.0f : exp2f((m_run[j] - m_new[j]) * e2);
       l_run[j] *= alpha;
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[j][e] *= alpha;
@@ -455,7 +455,7 @@ __global__ __launch_bounds__(64) void dense_attn_split_kernel(AttnArgs a, float*
         vd[i].decode(vsc, vz, x);
 #pragma unroll
       for (int j = 0; j < GH; ++j) {
-        const float p = sc[j][i] == -INFINITY ? 0.0f : exp2f(sc[j][i] - m_new[j]);
+        const float p = sc[j][i] == -INFINITY ? 0.0f : exp2f((sc[j][i] - m_new[j]) * e2);
         l_run[j] += p;
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[j][e] = fmaf(p, x[e], acc[j][e]);
@@ -807,7 +807,7 @@ void int4_sym_attn_mfma_kernel(AttnArgs a, float* part,
 }
 
 // One workgroup of kMergeWaves waves per query row:
-// out = sum_k 2^(m_k - M) acc_k / sum_k 2^(m_k - M) l_k.  Every wave finds M
+// out = sum_k f_k acc_k / sum_k f_k l_k, f_k = 2^((m_k - M) exp2_factor).  Every wave finds M
 // and the denominator over all splits, wave 0 puts the split weights in LDS;
 // wave w then sums the splits w, w + kMergeWaves, ..., lane (phase, quad)
 // taking the f32x4 quad `quad` of every P-th of them (P = 256 / D phases).
@@ -833,6 +833,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void dense_attn_merge_kernel(Attn
   const float* pr = part + row * n_splits * (int64_t)STRIDE;
   const int quad = lane % Q, phase = lane / Q;
   const int k0 = wv * P + phase;  // this lane's splits: k0, k0 + S, ...
+  const float e2 = exp2_factor(a);
   f32x4 x[kMergeBatch];
 #pragma unroll
   for (int i = 0; i < kMergeBatch; ++i) {
@@ -853,13 +854,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void dense_attn_merge_kernel(Attn
   // every wave finds the denominator; wave 0 writes the weights
   float den = 0.0f;
   if (lane < ns) {
-    const float f = (M == -INFINITY || m0 == -INFINITY) ? 0.0f : exp2f(m0 - M);
+    const float f = (M == -INFINITY || m0 == -INFINITY) ? 0.0f : exp2f((m0 - M) * e2);
     den = l0 * f;
     if (wv == 0) f_s[lane] = f;
   }
   for (int k = lane + 64; k < ns; k += 64) {
     const float mk = pr[(int64_t)k * STRIDE + D];
-    const float f = (M == -INFINITY || mk == -INFINITY) ? 0.0f : exp2f(mk - M);
+    const float f = (M == -INFINITY || mk == -INFINITY) ? 0.0f : exp2f((mk - M) * e2);
     den = fmaf(pr[(int64_t)k * STRIDE + D + 1], f, den);
     if (wv == 0) f_s[k] = f;
   }

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) qb[ks] = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
   }
-  const float qs = a.scale * kLog2e;
+  const float qs = score_scale(a), e2 = exp2_factor(a);
   const float* mrow = a.mask ? a.mask + b * a.ms0 + (int64_t)head * a.ms1 + tq * a.ms2 : nullptr;
   // four mask values at once where every group of four tokens is aligned and
   // lies inside or outside the row as a whole
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
 #pragma unroll
       for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[tb][i] = fmaf(mk[tb][i >> 2][i & 3], kLog2e, s[tb][i]);
+        for (int i = 0; i < 16; ++i) s[tb][i] += mk[tb][i >> 2][i & 3];
     }
     if constexpr (!full) {
 #pragma unroll
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
     // a row with every score so far -inf keeps l = 0 and acc = 0
     const float m_use = m_new == -INFINITY ? 0.0f : m_new;
     if (__any(m_new > m_run)) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * e2);
       l_run *= alpha;
 #pragma unroll
       for (int d = 0; d < D / 32; ++d)
@@ -315,7 +315,6 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
         for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
     }
     m_run = m_new;
-    const float m_sub = m_use - weight_shift<DT>();
 
 #pragma unroll
     for (int st = 0; st < BT / 16; ++st) {
@@ -323,8 +322,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
       u32x4 pb[TERMS];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float p0 = __builtin_amdgcn_exp2f(s[st >> 1][8 * (st & 1) + 2 * j] - m_sub);
-        const float p1 = __builtin_amdgcn_exp2f(s[st >> 1][8 * (st & 1) + 2 * j + 1] - m_sub);
+        const float d0 = s[st >> 1][8 * (st & 1) + 2 * j] - m_use;
+        const float d1 = s[st >> 1][8 * (st & 1) + 2 * j + 1] - m_use;
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(d0, e2, weight_shift<DT>()));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(d1, e2, weight_shift<DT>()));
         l_run += p0;
         l_run += p1;
         uint32_t w[TERMS];
@@ -379,13 +380,14 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
 
 constexpr int kFewSplits = 8;
 
-// out = sum_k 2^(m_k - M) acc_k / sum_k 2^(m_k - M) l_k over a row's splits,
+// out = sum_k f_k acc_k / sum_k f_k l_k, f_k = 2^((m_k - M) e2), over a row's splits,
 // one lane per four dims, each reading every (m, l) of its row itself: for up
 // to kFewSplits splits; more go to the one-row kernel's merge (a workgroup
 // per row).
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(void* out, int out_dtype, int64_t rows,
-                                                            const float* part, int n_splits) {
+                                                            const float* part, int n_splits,
+                                                            float e2) {
   constexpr int Q = D / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t row = i / Q;
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(void* out, int out_d
   for (int k = 0; k < n_splits; ++k) {
     const float* p = pr + k * (D + kPartPad);
     const float m = p[D];
-    const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+    const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * e2);
     den = fmaf(p[D + 1], f, den);
     const f32x4 x = *reinterpret_cast<const f32x4*>(p + 4 * quad);
 #pragma unroll
@@ -423,7 +425,7 @@ void launch_one(const AttnArgs& a, int32_t out_dtype, float* part, const Prefill
     launch_merge(a, out_dtype, rows, part, p.n_splits, st);
   } else if (p.n_splits > 1) {
     prefill_merge_kernel<D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), 256, 0, st>>>(
-        a.out, out_dtype, rows, part, (int)p.n_splits);
+        a.out, out_dtype, rows, part, (int)p.n_splits, exp2_factor(a));
   }
 }
 

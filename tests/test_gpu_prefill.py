@@ -107,10 +107,7 @@ def test_many_rows_non_finite(dtype):
     k[0, 2, 70] = float("nan")
     v[0, 3, 149, 5] = float("inf")
     out = dense_attention(q, k, v, None, mask, torch.float32)
-    assert torch.isnan(out[:, :, 5]).all()  # the lowest value times log2(e) is -inf here
-    ref = _ref(q, k, v, D ** -0.5, mask)
-    keep = [i for i in range(Tq) if i != 5]
-    out, ref = out[:, :, keep].double(), ref[:, :, keep]
+    out, ref = out.double(), _ref(q, k, v, D ** -0.5, mask)
     assert torch.equal(torch.isnan(out), torch.isnan(ref))
     assert torch.equal(torch.isinf(out), torch.isinf(ref)) and torch.isinf(ref).any()
     ok = torch.isfinite(ref)
