@@ -15,11 +15,11 @@
 //
 // Precision.  The bf16 / fp16 products of Q and K are exact and summed in
 // fp32, as the one-row kernel's v_dot2 does.  The softmax weights are fp32
-// and enter the PV tiles as a sum of 16-bit terms: three bf16 terms hold an
-// fp32 weight exactly, two fp16 terms (scaled by 2^15) hold it to 22 bits of
-// itself and 2^-38 of the row's largest.  Accumulators, maxima and sums are
-// fp32.  (Two bf16 terms would be a tenth faster at 32 / 8 heads, 512 rows,
-// 4096 tokens, but are 16 bits.)
+// and enter the PV tiles as three bf16 terms, whose sum is exactly the weight;
+// an fp16 V enters as two, which hold its 11 bits exactly as well.  (fp16
+// terms would lose the weights below 2^-14 of the row's largest, and two bf16
+// terms, a tenth faster at 32 / 8 heads, 512 rows, 4096 tokens, are 16 bits.)
+// Accumulators, maxima and sums are fp32.
 #include <algorithm>
 #include <type_traits>
 
@@ -57,52 +57,36 @@ constexpr int tile_tokens(int D, int NW) { return D == 256 || NW == 1 ? 32 : 64;
 constexpr int k_stride(int D) { return 2 * D + 16; }
 constexpr int v_stride(int D) { return 2 * D + 64; }
 
-// 16-bit terms of a softmax weight.
-template <int DT>
-constexpr int weight_terms() {
-  return DT == AMF_DTYPE_BF16 ? 3 : 2;
-}
-// The fp16 weights carry 2^15, so that their low terms stay representable.
-template <int DT>
-constexpr float weight_shift() {
-  return DT == AMF_DTYPE_F16 ? 15.0f : 0.0f;
+// bf16 terms of a softmax weight.
+constexpr int kTerms = 3;
+
+// The terms of the weights p0 and p1 (low and high half of each word).  A
+// positive weight has only positive terms, a zero one only zeros: inf in V
+// then gives inf under a positive weight (mixed signs or a zero term would
+// make it NaN) and NaN under a zero one, as the product with the weight itself
+// does.  Each term is the top half of the bit pattern below the remainder's,
+// so the next remainder is positive and exact and the third fits 8 bits.
+__device__ __forceinline__ void weight_split(float p0, float p1, uint32_t (&w)[kTerms]) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t a = __builtin_elementwise_sub_sat(f2u(p0), 1u) & 0xFFFF0000u;
+    const uint32_t b = __builtin_elementwise_sub_sat(f2u(p1), 1u) & 0xFFFF0000u;
+    w[k] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    p0 -= u2f(a);
+    p1 -= u2f(b);
+  }
+  w[2] = __builtin_amdgcn_perm(f2u(p1), f2u(p0), 0x07060302u);
 }
 
-// Terms of the weights p0 and p1 (low and high half of each word).  A positive
-// weight has only positive terms, a zero one only zeros: inf in V then gives
-// inf under a positive weight (mixed signs or a zero term would make it NaN)
-// and NaN under a zero one, as the product with the weight itself does.  Each
-// bf16 term is the top half of the bit pattern below the remainder's, so the
-// next remainder is positive and exact and the third fits 8 bits; fp16 terms
-// are rounded toward zero from below and raised to the least subnormal.
-template <int DT>
-__device__ __forceinline__ void weight_split(float p0, float p1,
-                                             uint32_t (&w)[weight_terms<DT>()]) {
-  if constexpr (DT == AMF_DTYPE_BF16) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const uint32_t a = __builtin_elementwise_sub_sat(f2u(p0), 1u) & 0xFFFF0000u;
-      const uint32_t b = __builtin_elementwise_sub_sat(f2u(p1), 1u) & 0xFFFF0000u;
-      w[k] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-      p0 -= u2f(a);
-      p1 -= u2f(b);
-    }
-    w[2] = __builtin_amdgcn_perm(f2u(p1), f2u(p0), 0x07060302u);
-  } else {
-    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-    const u16x2 least = __builtin_bit_cast(u16x2, min(f2u(p0), 1u) | (min(f2u(p1), 1u) << 16));
-    auto raised = [&](uint32_t x) {
-      return __builtin_bit_cast(
-          uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), least));
-    };
-    w[0] = raised(__builtin_bit_cast(
-        uint32_t,
-        __builtin_amdgcn_cvt_pkrtz(u2f(__builtin_elementwise_sub_sat(f2u(p0), 1u)),
-                                   u2f(__builtin_elementwise_sub_sat(f2u(p1), 1u)))));
-    p0 = fmaxf(p0 - half_lo<false>(w[0]), 0.0f);
-    p1 = fmaxf(p1 - half_hi<false>(w[0]), 0.0f);
-    w[1] = raised(pack2<false>(p0, p1));
-  }
+// A pair of fp16 V values as two bf16 pairs, hi + lo: the top 8 bits of each
+// value's 11 and the rest, below 2^8.  The clamp only meets the NaN of an
+// infinite value's remainder and makes it -256: hi alone is then infinite.
+__device__ __forceinline__ void v_split(uint32_t w, uint32_t& hi, uint32_t& lo) {
+  const uint32_t a = f2u(half_lo<false>(w)), b = f2u(half_hi<false>(w));
+  hi = __builtin_amdgcn_perm(b, a, 0x07060302u);
+  const float ra = __builtin_amdgcn_fmed3f(u2f(a) - u2f(a & 0xFFFF0000u), -256.0f, 256.0f);
+  const float rb = __builtin_amdgcn_fmed3f(u2f(b) - u2f(b & 0xFFFF0000u), -256.0f, 256.0f);
+  lo = __builtin_amdgcn_perm(f2u(rb), f2u(ra), 0x07060302u);
 }
 
 // Measured (bf16, 32 / 8 heads, head_dim 128, causal mask): 512 rows x 4096
@@ -127,10 +111,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   constexpr int CH = BT * LPR / (64 * NW);       // chunks per lane of a tile
   constexpr int RSTEP = 64 * NW / LPR;           // rows between a lane's chunks
   static_assert(CH >= 1 && (64 * NW) % LPR == 0, "a tile is whole chunks per lane");
-  constexpr int TERMS = weight_terms<DT>();
+  // fp16 V: split where it is staged, for all waves of the workgroup, or, for a
+  // single wave, where it is read (as much work, and half the LDS)
+  constexpr bool F16 = DT == AMF_DTYPE_F16, SPLIT_STAGE = F16 && NW > 1;
   using Raw = RawRow<DT, INT4>;
   __shared__ __attribute__((aligned(16))) uint8_t k_lds[BT * KS];
-  __shared__ __attribute__((aligned(16))) uint8_t v_lds[BT * VS];
+  __shared__ __attribute__((aligned(16))) uint8_t v_lds[(SPLIT_STAGE ? 2 : 1) * BT * VS];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lc = lane & 31, h = lane >> 5;
@@ -221,8 +207,21 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
       vr[i].pairs(vsc, vz, vp);
       *reinterpret_cast<u32x4*>(k_lds + r * KS + 16 * c) =
           in ? u32x4{kp[0], kp[1], kp[2], kp[3]} : u32x4{0, 0, 0, 0};
-      *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) =
-          in ? u32x4{vp[0], vp[1], vp[2], vp[3]} : u32x4{0, 0, 0, 0};
+      if constexpr (SPLIT_STAGE) {
+        u32x4 vh, vl;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          uint32_t x, y;
+          v_split(in ? vp[w] : 0u, x, y);
+          vh[w] = x;
+          vl[w] = y;
+        }
+        *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) = vh;
+        *reinterpret_cast<u32x4*>(v_lds + BT * VS + r * VS + 16 * c) = vl;
+      } else {
+        *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) =
+            in ? u32x4{vp[0], vp[1], vp[2], vp[3]} : u32x4{0, 0, 0, 0};
+      }
     }
   };
 
@@ -237,6 +236,14 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   const uint8_t* k_rd = k_lds + lc * KS + 16 * h;
   const int l16 = lane & 15;
   const uint8_t* v_rd = v_lds + (4 * h + (l16 >> 2)) * VS + 32 * ((lane >> 4) & 1) + 8 * (l16 & 3);
+
+  // A operand of V^T: dims 32 d .. + 31, 16 tokens in the order of the scores
+  auto read_v = [](const uint8_t* vp) {
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 8 * VS));
+    const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+    return u32x4{l2[0], l2[1], h2[0], h2[1]};
+  };
 
   // One tile; `full` when it lies inside the split: nothing is clamped or
   // masked per element then, which was half of the kernel's VALU work.
@@ -318,30 +325,47 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
 
 #pragma unroll
     for (int st = 0; st < BT / 16; ++st) {
-      // weights of the step's 16 tokens in 16-bit terms, 8 per lane
-      u32x4 pb[TERMS];
+      // weights of the step's 16 tokens in bf16 terms, 8 per lane
+      u32x4 pb[kTerms];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float d0 = s[st >> 1][8 * (st & 1) + 2 * j] - m_use;
         const float d1 = s[st >> 1][8 * (st & 1) + 2 * j + 1] - m_use;
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(d0, e2, weight_shift<DT>()));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(d1, e2, weight_shift<DT>()));
+        const float p0 = __builtin_amdgcn_exp2f(d0 * e2);
+        const float p1 = __builtin_amdgcn_exp2f(d1 * e2);
         l_run += p0;
         l_run += p1;
-        uint32_t w[TERMS];
-        weight_split<DT>(p0, p1, w);
+        uint32_t w[kTerms];
+        weight_split(p0, p1, w);
 #pragma unroll
-        for (int k = 0; k < TERMS; ++k) pb[k][j] = w[k];
+        for (int k = 0; k < kTerms; ++k) pb[k][j] = w[k];
       }
 #pragma unroll
       for (int d = 0; d < D / 32; ++d) {
         const uint8_t* vp = v_rd + 16 * st * VS + 64 * d;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 8 * VS));
-        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-        const u32x4 va = {l2[0], l2[1], h2[0], h2[1]};
+        const u32x4 va = read_v(vp);
+        if constexpr (F16) {
+          u32x4 vh = va, vl;
+          if constexpr (SPLIT_STAGE) {
+            vl = read_v(vp + BT * VS);
+          } else {
 #pragma unroll
-        for (int k = 0; k < TERMS; ++k) acc[d] = mfma32<DT>(va, pb[k], acc[d]);
+            for (int w = 0; w < 4; ++w) {
+              uint32_t x, y;
+              v_split(va[w], x, y);
+              vh[w] = x;
+              vl[w] = y;
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < kTerms; ++k) {
+            acc[d] = mfma32<AMF_DTYPE_BF16>(vh, pb[k], acc[d]);
+            acc[d] = mfma32<AMF_DTYPE_BF16>(vl, pb[k], acc[d]);
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < kTerms; ++k) acc[d] = mfma32<DT>(va, pb[k], acc[d]);
+        }
       }
     }
   };

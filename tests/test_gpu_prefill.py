@@ -112,3 +112,28 @@ def test_many_rows_non_finite(dtype):
     assert torch.equal(torch.isinf(out), torch.isinf(ref)) and torch.isinf(ref).any()
     ok = torch.isfinite(ref)
     assert float((out[ok] - ref[ok]).abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Tq,T,D", [(2, 12, 77, 64), (4, 20, 200, 128), (1, 40, 130, 128),
+                                       (1, 33, 97, 256)])
+def test_many_rows_small_weights(dtype, Hq, Tq, T, D):
+    """The softmax weights keep their 32 bits however small they are: one token
+    of zeros holds the row's largest weight, so the output is what the weights
+    of 2^-20 to 2^-59 give the others."""
+    from korith_vllm_ext.kernels import dense_attention
+
+    g = torch.Generator().manual_seed(Tq)
+    q = torch.zeros(1, Hq, Tq, D, dtype=dtype, device=DEV)
+    k = torch.zeros(1, 1, T, D, dtype=dtype, device=DEV)
+    v = (torch.rand(1, 1, T, D, generator=g) + 0.5).to(dtype).to(DEV)
+    v[:, :, 3] = 0
+    # a row's tokens all weigh about 2^-(20 + row)
+    mask = -0.6931471805599453 * (20.0 + torch.arange(Tq)[:, None] + torch.rand(Tq, T, generator=g))
+    mask[:, 3] = 0.0
+    mask = mask.to(DEV)
+    out = dense_attention(q, k, v, None, mask, torch.float32).double()
+    ref = _ref(q, k, v, D ** -0.5, mask)
+    # 2^x at |x| < 61: its rounded argument puts the weights off by at most
+    # 61 ln(2) 2^-23, 5e-6, and the sums of 200 positive terms by less
+    assert float(((out - ref).abs() / ref).max()) <= 2e-5
