@@ -1419,7 +1419,8 @@ __global__ __launch_bounds__(64 * W) void int4_decode_merge_sk_kernel(DecodeArgs
       return base + (int64_t)((2 * k + slot) * R) * kPartStride;
     };
     // accumulators and m of kSkPre of this half wave's parts from k0 on (past
-    // the last part: that one again, with a weight of zero)
+    // the last part: that one again, not added; a weight of zero would turn an
+    // infinite accumulator into NaN)
     float4 acc[kSkPre];
     float mk[kSkPre];
     auto load = [&](int k0) {
@@ -1449,11 +1450,12 @@ __global__ __launch_bounds__(64 * W) void int4_decode_merge_sk_kernel(DecodeArgs
     for (int k0 = k_first;;) {
 #pragma unroll
       for (int j = 0; j < kSkPre; ++j) {
-        const float wk = k0 + 2 * W * j < n_sp ? exp2_fast(mk[j] - M) : 0.0f;
-        o.x += wk * acc[j].x;
-        o.y += wk * acc[j].y;
-        o.z += wk * acc[j].z;
-        o.w += wk * acc[j].w;
+        const bool in = k0 + 2 * W * j < n_sp;
+        const float wk = exp2_fast(mk[j] - M);
+        o.x = in ? __builtin_fmaf(wk, acc[j].x, o.x) : o.x;
+        o.y = in ? __builtin_fmaf(wk, acc[j].y, o.y) : o.y;
+        o.z = in ? __builtin_fmaf(wk, acc[j].z, o.z) : o.z;
+        o.w = in ? __builtin_fmaf(wk, acc[j].w, o.w) : o.w;
       }
       k0 += 2 * W * kSkPre;
       if (!__any(k0 < n_sp)) break;
