@@ -33,6 +33,7 @@ using namespace amf;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef s16x4 __attribute__((address_space(3))) lds_s16x4;
 
@@ -89,21 +90,31 @@ __device__ __forceinline__ void v_split(uint32_t w, uint32_t& hi, uint32_t& lo) 
   lo = __builtin_amdgcn_perm(f2u(rb), f2u(ra), 0x07060302u);
 }
 
-// Measured (bf16, 32 / 8 heads, head_dim 128, causal mask): 512 rows x 4096
-// tokens 1285 -> 90 us (25 -> 360 TFLOP/s), 128 rows x 8192 tokens 913 ->
-// 65 us; the one-row kernel ran every row's products on the VALU and read
-// K/V from L2 once per row.  Now bound by the matrix cores and the VALU beside
-// them at two waves per SIMD (254 VGPRs): QK^T and three PV terms are 69 GFLOP
-// of tiles, 55 us at the rate a large library product reaches here, and the
-// softmax and the weights' terms take about as many cycles.  A second LDS
-// buffer (one barrier per tile instead of two) and other orders of the PV
-// tiles measured the same.
+// Measured (32 / 8 heads, head_dim 128, causal mask): bf16 512 rows x 4096
+// tokens 1285 -> 85 us (25 -> 380 TFLOP/s), 128 rows x 8192 tokens 913 -> 56 us;
+// fp16 1490 -> 118 and 938 -> 71 us; the one-row kernel ran every row's products
+// on the VALU and read K/V from L2 once per row.  Now bound by the matrix cores
+// and the VALU beside them at two waves per SIMD: QK^T and three PV terms are 69
+// GFLOP of tiles, 55 us at the rate a large library product reaches here, and
+// the softmax and the weights' terms take about as many cycles.  A second LDS
+// buffer (one barrier per tile instead of two) and other orders of the PV tiles
+// measured the same.
 //
-// NW waves of 32 query rows each share the K/V tiles.  Unit u is (b, KV head, split), served by `tiles`
-// workgroups; with xcd_map they take consecutive slots of one XCD (its L2
-// holds the unit's K/V), else they are consecutive workgroups.
+// Registers: at head_dim 64 and 128 nothing spills.  What kept it from that was
+// a second copy of the tile's body for the split's last tile (42 VGPRs in
+// scratch at 128), the int4 scales (in LDS now), and the mask's scalar
+// addresses.  At head_dim 256 the tile after next is not prefetched and the
+// mask is read after the scores, so that four waves keep 8 to 15 VGPRs in
+// scratch (before 69 to 80; 256 rows x 4096 tokens, 16 / 2 heads 77 -> 67 us),
+// and one wave, of which LDS lets four on a CU, may use 512 (4 heads x 16 x 16
+// rows x 4096 tokens 379 -> 66 us).
+//
+// NW waves of 32 query rows each share the K/V tiles.  Unit u is (b, KV head,
+// split), served by `tiles` workgroups; with xcd_map they take consecutive
+// slots of one XCD (its L2 holds the unit's K/V), else they are consecutive
+// workgroups.
 template <int DT, int D, int NW, bool INT4>
-__global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
+__global__ __launch_bounds__(64 * NW, D == 256 && NW == 1 ? 1 : 2) void prefill_attn_kernel(
     AttnArgs a, int out_dtype, float* part, int64_t split_tokens, int64_t n_splits, int64_t units,
     int tiles, bool xcd_map) {
   constexpr int BT = tile_tokens(D, NW), KS = k_stride(D), VS = v_stride(D);
@@ -114,6 +125,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   // fp16 V: split where it is staged, for all waves of the workgroup, or, for a
   // single wave, where it is read (as much work, and half the LDS)
   constexpr bool F16 = DT == AMF_DTYPE_F16, SPLIT_STAGE = F16 && NW > 1;
+  constexpr bool AHEAD = D <= 128;  // the next tile's rows and the mask read early
   using Raw = RawRow<DT, INT4>;
   __shared__ __attribute__((aligned(16))) uint8_t k_lds[BT * KS];
   __shared__ __attribute__((aligned(16))) uint8_t v_lds[(SPLIT_STAGE ? 2 : 1) * BT * VS];
@@ -156,23 +168,28 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   }
   const float qs = score_scale(a), e2 = exp2_factor(a);
   const float* mrow = a.mask ? a.mask + b * a.ms0 + (int64_t)head * a.ms1 + tq * a.ms2 : nullptr;
-  // four mask values at once where every group of four tokens is aligned and
-  // lies inside or outside the row as a whole
-  const bool mvec = a.ms3 == 1 && T % 4 == 0 && (reinterpret_cast<uintptr_t>(a.mask) & 15) == 0 &&
-                    ((a.ms0 | a.ms1 | a.ms2) & 3) == 0;
-
   // staging: chunk (row r0 + RSTEP i, dims 8 c ..) of the tile
   const int c = tid % LPR, r0 = tid / LPR;
-  float ksc[8], kz[8], vsc[8], vz[8];
+  // int4: K and V channel scales (read per tile: 32 registers less across it)
+  __shared__ __attribute__((aligned(16))) float s_lds[INT4 ? 2 * D : 4];
   if constexpr (INT4) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      ksc[e] = (float)a.k_scales[8 * c + e];
-      vsc[e] = (float)a.v_scales[8 * c + e];
-      kz[e] = -8.0f * ksc[e];
-      vz[e] = -8.0f * vsc[e];
+    for (int d = tid; d < D; d += 64 * NW) {
+      s_lds[d] = (float)a.k_scales[d];
+      s_lds[D + d] = (float)a.v_scales[d];
     }
   }
+  // this lane's scales s and -8 s of K or V
+  auto scales = [&](int base, float (&sc)[8], float (&z)[8]) {
+    if constexpr (INT4) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(s_lds + base + 8 * c);
+      const f32x4 x = p[0], y = p[1];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        sc[e] = e < 4 ? x[e & 3] : y[e & 3];
+        z[e] = -8.0f * sc[e];
+      }
+    }
+  };
   Raw kr[CH], vr[CH];
   constexpr int RB = INT4 ? D / 2 : 2 * D, CB = INT4 ? 4 : 16;  // bytes of a row, of a chunk
   const uint32_t lane_off = (uint32_t)(r0 * RB + c * CB);
@@ -195,32 +212,45 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
       }
     }
   };
-  // rows past the split are zeros (their scores are -inf below)
-  auto stage = [&](auto full_c, int64_t t0) {
-    constexpr bool full = decltype(full_c)::value;
+  auto stage = [&](int64_t t0, bool full) {
+    float sc[8], z[8];
+    scales(0, sc, z);
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-      const int r = r0 + RSTEP * i;
-      const bool in = full || t0 + r < t_end;
-      uint32_t kp[4], vp[4];
-      kr[i].pairs(ksc, kz, kp);
-      vr[i].pairs(vsc, vz, vp);
-      *reinterpret_cast<u32x4*>(k_lds + r * KS + 16 * c) =
-          in ? u32x4{kp[0], kp[1], kp[2], kp[3]} : u32x4{0, 0, 0, 0};
+      uint32_t kp[4];
+      kr[i].pairs(sc, z, kp);
+      *reinterpret_cast<u32x4*>(k_lds + (r0 + RSTEP * i) * KS + 16 * c) =
+          u32x4{kp[0], kp[1], kp[2], kp[3]};
+    }
+    scales(D, sc, z);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      uint8_t* dst = v_lds + (r0 + RSTEP * i) * VS + 16 * c;
+      uint32_t vp[4];
+      vr[i].pairs(sc, z, vp);
       if constexpr (SPLIT_STAGE) {
         u32x4 vh, vl;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           uint32_t x, y;
-          v_split(in ? vp[w] : 0u, x, y);
+          v_split(vp[w], x, y);
           vh[w] = x;
           vl[w] = y;
         }
-        *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) = vh;
-        *reinterpret_cast<u32x4*>(v_lds + BT * VS + r * VS + 16 * c) = vl;
+        *reinterpret_cast<u32x4*>(dst) = vh;
+        *reinterpret_cast<u32x4*>(dst + BT * VS) = vl;
       } else {
-        *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) =
-            in ? u32x4{vp[0], vp[1], vp[2], vp[3]} : u32x4{0, 0, 0, 0};
+        *reinterpret_cast<u32x4*>(dst) = u32x4{vp[0], vp[1], vp[2], vp[3]};
+      }
+    }
+    if (!full) {  // V rows past the split: zeros (their scores are -inf below)
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int r = r0 + RSTEP * i;
+        if (t0 + r < t_end) continue;
+        *reinterpret_cast<u32x4*>(v_lds + r * VS + 16 * c) = u32x4{0, 0, 0, 0};
+        if constexpr (SPLIT_STAGE)
+          *reinterpret_cast<u32x4*>(v_lds + BT * VS + r * VS + 16 * c) = u32x4{0, 0, 0, 0};
       }
     }
   };
@@ -246,36 +276,46 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
   };
 
   // One tile; `full` when it lies inside the split: nothing is clamped or
-  // masked per element then, which was half of the kernel's VALU work.
-  auto tile_step = [&](auto full_c, int64_t t0) {
-    constexpr bool full = decltype(full_c)::value;
+  // masked per element then.
+  auto tile_step = [&](int64_t t0, auto full) {
+    if constexpr (!AHEAD) fetch(t0);
     __syncthreads();  // the previous tile has been read
-    stage(full_c, t0);
+    stage(t0, full);
     __syncthreads();
     // token of score element i of block tb: t0 + 32 tb + 8 (i / 4) + 4 h + i % 4
+    // A contiguous mask row is read four values at once (at any multiple of 4
+    // bytes), others and the row's end one at a time.
     f32x4 mk[BT / 32][4];
-    if (mrow) {
-      const float* mp = mrow + (t0 + 4 * h) * a.ms3;
+    auto load_mask = [&] {
+      if (a.ms3 == 1 && full) {
+        const float* mp = mrow + t0 + 4 * h;
 #pragma unroll
-      for (int tb = 0; tb < BT / 32; ++tb)
+        for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int dt = 32 * tb + 8 * g;
-          if (mvec) {
-            const int64_t t = t0 + dt + 4 * h;
-            mk[tb][g] = *reinterpret_cast<const f32x4*>(full ? mp + dt
-                                                             : mrow + (t < t_end ? t : t_begin));
-          } else {
+          for (int g = 0; g < 4; ++g)
+            mk[tb][g] = *reinterpret_cast<const f32x4u*>(mp + 32 * tb + 8 * g);
+      } else if (full) {
+        const float* mp = mrow + (t0 + 4 * h) * a.ms3;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int64_t t = t0 + dt + 4 * h + e;
-              mk[tb][g][e] =
-                  full ? mp[(dt + e) * a.ms3] : mrow[(t < t_end ? t : t_begin) * a.ms3];
-            }
+        for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            mk[tb][i >> 2][i & 3] = *mp;
+            mp += (i & 3) == 3 ? 5 * a.ms3 : a.ms3;
+            asm("" : "+v"(mp));  // one address at a time
           }
-        }
-    }
-    fetch(t0 + BT);
+      } else {
+#pragma unroll
+        for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int64_t t = t0 + 32 * tb + 8 * (i >> 2) + 4 * h + (i & 3);
+            mk[tb][i >> 2][i & 3] = mrow[(t < t_end ? t : t_begin) * a.ms3];
+          }
+      }
+    };
+    if (AHEAD && mrow) load_mask();
+    if constexpr (AHEAD) fetch(t0 + BT);
 
     f32x16 s[BT / 32];
 #pragma unroll
@@ -287,17 +327,19 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
         s[tb] = mfma32<DT>(*reinterpret_cast<const u32x4*>(k_rd + 32 * tb * KS + 32 * ks), qb[ks],
                            s[tb]);
     }
-#pragma unroll
-    for (int tb = 0; tb < BT / 32; ++tb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[tb][i] *= qs;
     if (mrow) {
+      if constexpr (!AHEAD) load_mask();
 #pragma unroll
       for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[tb][i] += mk[tb][i >> 2][i & 3];
+        for (int i = 0; i < 16; ++i) s[tb][i] = fmaf(s[tb][i], qs, mk[tb][i >> 2][i & 3]);
+    } else {
+#pragma unroll
+      for (int tb = 0; tb < BT / 32; ++tb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[tb][i] *= qs;
     }
-    if constexpr (!full) {
+    if (!full) {
 #pragma unroll
       for (int tb = 0; tb < BT / 32; ++tb)
 #pragma unroll
@@ -369,10 +411,16 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(
       }
     }
   };
-  fetch(t_begin);
-  int64_t t0 = t_begin;
-  for (; t0 + BT <= t_end; t0 += BT) tile_step(std::true_type{}, t0);
-  if (t0 < t_end) tile_step(std::false_type{}, t0);
+  if constexpr (AHEAD) fetch(t_begin);
+  if constexpr (D == 64) {
+    int64_t t0 = t_begin;
+    for (; t0 + BT <= t_end; t0 += BT) tile_step(t0, std::true_type{});
+    if (t0 < t_end) tile_step(t0, std::false_type{});
+  } else {
+    // one copy of the body, with uniform branches: a second one spilled 42 VGPRs
+    // at head_dim 128 (head_dim 64 has the registers, and is 5% faster with two)
+    for (int64_t t0 = t_begin; t0 < t_end; t0 += BT) tile_step(t0, t0 + BT <= t_end);
+  }
 
   const float l = l_run + __shfl_xor(l_run, 32);
   if (!row_ok) return;
