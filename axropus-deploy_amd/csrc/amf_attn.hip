@@ -1055,14 +1055,16 @@ int64_t split_workspace_bytes(int64_t batch, int32_t num_q_heads, int32_t num_kv
   return rows * n_splits * (int64_t)(head_dim + kPartPad) * (int64_t)sizeof(float);
 }
 
-// The many-row kernel's plan for a call with this workspace: as many splits
-// as it has room for (one split needs none).
+// Whether a call with this workspace takes the many-row kernel, and its plan: as
+// many splits as there is room for (one split needs none).
 bool plan_prefill(const AttnArgs& a, int32_t dtype, int64_t workspace_bytes, PrefillPlan* p) {
   if (dtype == AMF_DTYPE_F32) return false;
   const int64_t room = std::max<int64_t>(
       1, workspace_bytes / prefill_split_bytes(a.batch, a.num_q_heads, a.q_len, a.head_dim));
   return prefill_plan(a.batch, a.num_q_heads, a.num_kv_heads, a.q_len, a.kv_len, a.head_dim, room,
-                      p);
+                      p) &&
+         prefill_pays(*p, a.batch, a.num_q_heads, a.num_kv_heads, a.q_len, a.kv_len, a.head_dim,
+                      dtype == AMF_DTYPE_F16);
 }
 
 }  // namespace

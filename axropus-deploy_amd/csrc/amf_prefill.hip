@@ -450,13 +450,14 @@ __global__ __launch_bounds__(64 * NW, D == 256 && NW == 1 ? 1 : 2) void prefill_
   }
 }
 
+// out = sum_k f_k acc_k / sum_k f_k l_k, f_k = 2^((m_k - M) e2), over a row's splits,
+// one lane per four dims, each reading every (m, l) of its row itself; all of
+// the at most N splits' loads are in flight together (in a loop over the splits
+// they followed each other: 64 rows of 8 splits 6 us instead of 3).  More than
+// kFewSplits splits go to the one-row kernel's merge (a workgroup per row).
 constexpr int kFewSplits = 8;
 
-// out = sum_k f_k acc_k / sum_k f_k l_k, f_k = 2^((m_k - M) e2), over a row's splits,
-// one lane per four dims, each reading every (m, l) of its row itself: for up
-// to kFewSplits splits; more go to the one-row kernel's merge (a workgroup
-// per row).
-template <int D>
+template <int D, int N>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(void* out, int out_dtype, int64_t rows,
                                                             const float* part, int n_splits,
                                                             float e2) {
@@ -466,18 +467,28 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(void* out, int out_d
   const int quad = (int)(i % Q);
   if (row >= rows) return;
   const float* pr = part + row * n_splits * (int64_t)(D + kPartPad);
-  float M = -INFINITY;
-  for (int k = 0; k < n_splits; ++k) M = fmaxf(M, pr[k * (D + kPartPad) + D]);
+  f32x2 ml[N];
+  f32x4 x[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {  // past the last split: that one again
+    const float* p = pr + min(k, n_splits - 1) * (D + kPartPad);
+    ml[k] = *reinterpret_cast<const f32x2*>(p + D);
+    x[k] = *reinterpret_cast<const f32x4*>(p + 4 * quad);
+  }
+  float M = ml[0][0];
+#pragma unroll
+  for (int k = 1; k < N; ++k) M = fmaxf(M, ml[k][0]);
   float den = 0.0f;
   f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k = 0; k < n_splits; ++k) {
-    const float* p = pr + k * (D + kPartPad);
-    const float m = p[D];
-    const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * e2);
-    den = fmaf(p[D + 1], f, den);
-    const f32x4 x = *reinterpret_cast<const f32x4*>(p + 4 * quad);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = fmaf(x[e], f, o[e]);
+  for (int k = 0; k < N; ++k) {
+    if (k < n_splits) {
+      const float m = ml[k][0];
+      const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - M) * e2);
+      den = fmaf(ml[k][1], f, den);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = fmaf(x[k][e], f, o[e]);
+    }
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = o[e] / den;
@@ -496,8 +507,17 @@ void launch_one(const AttnArgs& a, int32_t out_dtype, float* part, const Prefill
   if (p.n_splits > kFewSplits) {
     launch_merge(a, out_dtype, rows, part, p.n_splits, st);
   } else if (p.n_splits > 1) {
-    prefill_merge_kernel<D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), 256, 0, st>>>(
-        a.out, out_dtype, rows, part, (int)p.n_splits, exp2_factor(a));
+    const dim3 mgrid((unsigned)((rows * (D / 4) + 255) / 256));
+#define AMF_MERGE(N)                                                                   \
+  prefill_merge_kernel<D, N><<<mgrid, 256, 0, st>>>(a.out, out_dtype, rows, part,      \
+                                                    (int)p.n_splits, exp2_factor(a))
+    if (p.n_splits <= 2)
+      AMF_MERGE(2);
+    else if (p.n_splits <= 4)
+      AMF_MERGE(4);
+    else
+      AMF_MERGE(kFewSplits);
+#undef AMF_MERGE
   }
 }
 
@@ -532,11 +552,21 @@ bool prefill_plan(int64_t batch, int32_t num_q_heads, int32_t num_kv_heads, int6
   int64_t n = (want + base - 1) / base;
   const int64_t mc = p->waves == 1 ? kPrefillMinChunks1 : kPrefillMinChunks4;
   n = std::min<int64_t>(n, (chunks + mc - 1) / mc);
-  n = std::max<int64_t>(1, std::min<int64_t>({n, max_splits, kMaxPrefillSplits}));
+  const int64_t most = std::max<int64_t>(kPrefillSplits, kMaxPrefillSplits / base);
+  n = std::max<int64_t>(1, std::min<int64_t>({n, max_splits, most}));
   const int64_t per = (chunks + n - 1) / n;
   p->split_tokens = per * 64;
   p->n_splits = (chunks + per - 1) / per;
   return base <= (0x7FFFFFFF) / p->n_splits;
+}
+
+bool prefill_pays(const PrefillPlan& p, int64_t batch, int32_t num_q_heads, int32_t num_kv_heads,
+                  int64_t q_len, int64_t kv_len, int32_t head_dim, bool fp16) {
+  if (head_dim < 256 || num_q_heads / num_kv_heads % (fp16 ? 4 : 2) == 0) return true;
+  int64_t least = kPrefillMinPairs;
+  if (fp16) least *= 2;
+  if (p.waves > 1 && p.n_splits > 1) least *= 2;
+  return (double)batch * num_q_heads * q_len * kv_len > (double)least;
 }
 
 int64_t prefill_split_bytes(int64_t batch, int32_t num_q_heads, int64_t q_len, int32_t head_dim) {

@@ -46,6 +46,9 @@ def _mask(kind, B, Hq, Tq, T, g):
     (torch.bfloat16, 2, 14, 2, 37, 300, 64, "causal"),  # group of 7
     (torch.bfloat16, 1, 16, 2, 40, 1000, 256, "causal"),
     (torch.float16, 1, 4, 2, 16, 515, 256, "strided"),
+    (torch.float16, 1, 8, 2, 7, 515, 256, "strided"),   # a group of 4: tiles at any size
+    (torch.bfloat16, 1, 2, 2, 16, 2049, 256, "causal"),  # past the pairs that 256 dims take
+    (torch.float16, 2, 2, 1, 70, 1000, 256, "causal"),
     (torch.bfloat16, 3, 8, 8, 9, 4099, 128, "causal"),  # 9 rows, many splits, ragged end
     (torch.bfloat16, 1, 32, 8, 64, 2048, 128, "strided"),
     (torch.float16, 1, 6, 3, 50, 1, 128, None),         # a single token
@@ -116,7 +119,7 @@ def test_many_rows_non_finite(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Hq,Tq,T,D", [(2, 12, 77, 64), (4, 20, 200, 128), (1, 40, 130, 128),
-                                       (1, 33, 97, 256)])
+                                       (4, 8, 90, 256), (4, 33, 97, 256)])
 def test_many_rows_small_weights(dtype, Hq, Tq, T, D):
     """The softmax weights keep their 32 bits however small they are: one token
     of zeros holds the row's largest weight, so the output is what the weights
