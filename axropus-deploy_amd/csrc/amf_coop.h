@@ -28,7 +28,9 @@ namespace amf {
 
 constexpr int kCoopChunks = 16;   // 16-byte chunks per lane per register buffer
 constexpr int kCoopThreads = 256;
-constexpr uint32_t kCoopSpinLimit = 1u << 20;  // polls before a wait gives up
+// Polls before a wait gives up (about 0.4 us each; an exchange between resident
+// workgroups takes some 20): what a group that cannot complete costs a launch.
+constexpr uint32_t kCoopSpinLimit = 1u << 12;
 constexpr int kCoopClusters = kFp8CoopClusters;
 constexpr int kLineWords = kFp8CoopLineWords;
 constexpr uint32_t kReady = 0x80000000u;  // above every non-negative float's bits
@@ -47,15 +49,12 @@ struct CoopGeom {
   int32_t* err_flag;
 };
 
-// kCoopSpinLimit, or AMF_COOP_SPIN_LIMIT from the environment (read once):
-// the tests set it to 0 to drive every wait down its give-up path, which
-// must leave the kernel to finish normally with its group scales poisoned.
+// kCoopSpinLimit, or AMF_COOP_SPIN_LIMIT from the environment: the tests set it
+// to 0, with which every wait gives up at once and every group is quantized
+// from a second read.
 inline uint32_t coop_spin_limit() {
-  static const uint32_t limit = [] {
-    const char* e = getenv("AMF_COOP_SPIN_LIMIT");
-    return e ? (uint32_t)strtoul(e, nullptr, 10) : kCoopSpinLimit;
-  }();
-  return limit;
+  const char* e = getenv("AMF_COOP_SPIN_LIMIT");
+  return e ? (uint32_t)strtoul(e, nullptr, 10) : kCoopSpinLimit;
 }
 
 // AMF_NO_COOP set to a non-zero value in the environment (read once) turns

@@ -231,10 +231,11 @@ __device__ __forceinline__ float tensor_scale_from(uint32_t amax_bits) {
 // = [s, s, 1, 1] (FP8ScaleSidecar(k_scale=scale, v_scale=scale),
 // amf_codec.py:200) from the first plane of the group.
 template <int DT>
-__global__ void fp8_tensor_finalize_kernel(const uint64_t* __restrict__ param_planes,
-                                           const uint32_t* __restrict__ ws, int n_planes, int pps) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_planes && i % pps == 0) {
+__device__ __forceinline__ void write_sidecars(const uint64_t* __restrict__ param_planes,
+                                               const uint32_t* __restrict__ ws, int n_planes,
+                                               int pps) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_planes; i += gridDim.x * blockDim.x) {
+    if (i % pps != 0) continue;
     float* sc = reinterpret_cast<float*>(param_planes[i]);
     const float s = tensor_scale_from<DT>(ws[i / pps]);
     sc[0] = s;
@@ -244,10 +245,16 @@ __global__ void fp8_tensor_finalize_kernel(const uint64_t* __restrict__ param_pl
   }
 }
 
+template <int DT>
+__global__ void fp8_tensor_finalize_kernel(const uint64_t* __restrict__ param_planes,
+                                           const uint32_t* __restrict__ ws, int n_planes, int pps) {
+  write_sidecars<DT>(param_planes, ws, n_planes, pps);
+}
+
 // Per-tensor save in one read of the cache.  The two-pass form (absmax
 // kernel, then a quantize kernel that reads every page again) moves two
-// reads and a write through HBM.  Here a cooperative grid (every workgroup
-// resident) walks the scale groups in order and keeps its share of a group
+// reads and a write through HBM.  Here a cooperative grid (as many workgroups
+// as the chip holds) walks the scale groups in order and keeps its share of a group
 // in registers from the load to the store: the group's absmax is one atomic
 // max per workgroup into ws[group], a per-group arrival counter says when
 // every workgroup has contributed, and only then are the held values
@@ -265,6 +272,14 @@ __global__ void fp8_tensor_finalize_kernel(const uint64_t* __restrict__ param_pl
 // of each page (tid + 256 m), so page addresses are workgroup-uniform.  The
 // host takes this path only when a group fits the grid; others take the
 // two-pass kernels.
+// Nothing depends on the workgroups being resident together.  Three waves of
+// 166 VGPRs fill a SIMD's 512, so where another stream's wave came between two
+// of them the third has no room even after that wave has ended, until one of
+// the two does: waiting for it could last forever.  A workgroup whose wait runs
+// out of its bound marks the group, leaves its pages of it unwritten and goes
+// on.  It still reports its share of every group, so that every group's max is
+// complete when the kernel ends, and fp8_tensor_finish_kernel, which writes the
+// scales, quantizes the marked groups from a second read.
 struct CoopArgs {
   CoopGeom geo;
   const uint64_t* code_planes;
@@ -272,8 +287,11 @@ struct CoopArgs {
   uint32_t* ws;         // [n_groups] absmax bits, written by each group's root
   // Per group, kCoopClusters + 1 lines, zeroed before the launch.  Cluster
   // line k: [0] arrivals, [1] max bits, [2] the group's max | kReady once
-  // complete.  Root line: [0] clusters complete, [1] max bits.
+  // complete.  Root line: [0] clusters complete, [1] max bits, [2] marked for
+  // the second read; [3] of group 0: some group is.
   uint32_t* sync;
+  const uint64_t* param_planes;
+  int n_planes;
 };
 
 // The absmax works on the 16-bit patterns (abs_bits16): not converting to
@@ -340,30 +358,30 @@ __device__ __forceinline__ void coop_arrive(const CoopArgs& a, int gi,
 }
 
 // Waits (lane 0, bounded) for group gi's max on this workgroup's cluster
-// line and returns it to the whole workgroup.  Every workgroup of a
-// cooperative launch is resident, so the max arrives; the bound only keeps a
-// broken launch from spinning forever.  A workgroup whose wait runs out
-// raises AMF_ERRFLAG_SYNC, waits no more (no workgroup spins longer than one
-// bound in a launch), and raises the group's absmax slot to +inf, so the
-// scale written for that group is infinite and a restore of it yields
-// inf/NaN rather than plausible values.
+// line and returns it, with kReady, to the whole workgroup.  A workgroup whose
+// wait runs out waits no more (none spins longer than one bound in a launch);
+// for a group it finds incomplete it returns a value without kReady and has
+// marked the group.
 __device__ __forceinline__ uint32_t coop_wait(const CoopArgs& a, int gi, uint32_t* s_bits,
                                               bool& gave_up) {
   if (threadIdx.x == 0) {
     const uint32_t* go = coop_line(a.sync, gi, (int)blockIdx.x % kCoopClusters) + 2;
-    uint32_t v = __hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t spins = 0;
+    uint32_t v = 0, spins = 0;
+    if (a.geo.spin_limit != 0)  // 0: no group is ever found complete
+      v = __hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while (!gave_up && !(v & kReady)) {
-      if (++spins > a.geo.spin_limit) {
-        if (a.geo.err_flag) atomicOr(a.geo.err_flag, AMF_ERRFLAG_SYNC);
-        gave_up = true;
-      }
+      gave_up = ++spins > a.geo.spin_limit;
+      if (gave_up) break;
       __builtin_amdgcn_s_sleep(2);
       v = __hip_atomic_load(go, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (!(v & kReady))
-      __hip_atomic_fetch_max(a.ws + gi, 0x7F800000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *s_bits = v & ~kReady;
+    if (!(v & kReady)) {
+      __hip_atomic_store(coop_line(a.sync, gi, kCoopClusters) + 2, 1u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(coop_line(a.sync, 0, kCoopClusters) + 3, 1u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *s_bits = v;
   }
   __syncthreads();
   const uint32_t bits = *s_bits;
@@ -416,13 +434,27 @@ __global__ __launch_bounds__(kCoopThreads) void fp8_tensor_coop_kernel(CoopArgs 
   for (int gi = 0; gi < ng; gi += 2) {
     const uint32_t m0 = coop_wait(a, gi, &s_bits, gave_up);
     if (gi + 1 < ng) coop_arrive<DT>(a, gi + 1, b1, s_max);
-    coop_store<DT, CPT>(a, gi, b0, m0);
+    if (m0 & kReady) coop_store<DT, CPT>(a, gi, b0, m0 & ~kReady);
     if (gi + 2 < ng) coop_load<CPT>(a.geo, gi + 2, b0);
     if (gi + 1 >= ng) break;
     const uint32_t m1 = coop_wait(a, gi + 1, &s_bits, gave_up);
     if (gi + 2 < ng) coop_arrive<DT>(a, gi + 2, b0, s_max);
-    coop_store<DT, CPT>(a, gi + 1, b1, m1);
+    if (m1 & kReady) coop_store<DT, CPT>(a, gi + 1, b1, m1 & ~kReady);
     if (gi + 3 < ng) coop_load<CPT>(a.geo, gi + 3, b1);
+  }
+}
+
+// After fp8_tensor_coop_kernel, on the same grid: the scale sidecars, and the
+// pages of marked groups from a second read.
+template <int DT, int CPT>
+__global__ __launch_bounds__(kCoopThreads) void fp8_tensor_finish_kernel(CoopArgs a) {
+  write_sidecars<DT>(a.param_planes, a.ws, a.n_planes, a.geo.pps);
+  if (!coop_line(a.sync, 0, kCoopClusters)[3]) return;
+  for (int gi = 0; gi < a.geo.n_groups; ++gi) {
+    if (!coop_line(a.sync, gi, kCoopClusters)[2]) continue;
+    u32x4 buf[kCoopChunks];
+    coop_load<CPT>(a.geo, gi, buf);
+    coop_store<DT, CPT>(a, gi, buf, a.ws[gi]);
   }
 }
 
@@ -717,10 +749,18 @@ int make_geom(const char* who, int32_t block_size, int32_t num_heads, int32_t he
   return ok();
 }
 
-// The cooperative kernel for a cache dtype and chunks per page row (CPT),
-// or nullptr for combinations it does not cover.
-const void* coop_kernel(int dt, int cpt) {
-#define AMF_COOP(D, C) reinterpret_cast<const void*>(&fp8_tensor_coop_kernel<D, C>)
+// The cooperative kernel and the one that finishes its work, for a cache dtype
+// and chunks per page row (CPT), or nulls for combinations they do not cover.
+struct CoopKernels {
+  const void* save;
+  const void* finish;
+};
+CoopKernels coop_kernels(int dt, int cpt) {
+#define AMF_COOP(D, C)                                                   \
+  CoopKernels {                                                          \
+    reinterpret_cast<const void*>(&fp8_tensor_coop_kernel<D, C>),        \
+        reinterpret_cast<const void*>(&fp8_tensor_finish_kernel<D, C>)   \
+  }
 #define AMF_COOP_CPT(D)                                               \
   switch (cpt) {                                                      \
     case 1: return AMF_COOP(D, 1);                                    \
@@ -728,11 +768,11 @@ const void* coop_kernel(int dt, int cpt) {
     case 4: return AMF_COOP(D, 4);                                    \
     case 8: return AMF_COOP(D, 8);                                    \
     case 16: return AMF_COOP(D, 16);                                  \
-    default: return nullptr;                                          \
+    default: return CoopKernels{};                                    \
   }
   if (dt == AMF_DTYPE_BF16) { AMF_COOP_CPT(AMF_DTYPE_BF16) }
   if (dt == AMF_DTYPE_F16) { AMF_COOP_CPT(AMF_DTYPE_F16) }
-  return nullptr;
+  return CoopKernels{};
 #undef AMF_COOP_CPT
 #undef AMF_COOP
 }
@@ -773,14 +813,16 @@ constexpr int kCoopNotTaken = 1;
 // arrival counters.
 int try_tensor_coop(int32_t dt, const uint64_t* cache_planes, int64_t cache_page_stride,
                     const int32_t* block_ids, int64_t pool_pages, const uint64_t* code_planes,
-                    int64_t n_pages, const PageGeom& g, int n_groups, uint32_t* ws,
-                    int32_t* err_flag, hipStream_t s) {
+                    const uint64_t* param_planes, int n_planes, int64_t n_pages,
+                    const PageGeom& g, int n_groups, uint32_t* ws, int32_t* err_flag,
+                    hipStream_t s) {
   if (coop_disabled() || !aligned16(cache_page_stride)) return kCoopNotTaken;
   const int64_t page_elems = (int64_t)g.n_rows * g.head_dim;
   const int64_t chunks_pp = page_elems / 8;  // head_dim % 16 == 0: whole 16-byte chunks
   if (chunks_pp % kCoopThreads != 0) return kCoopNotTaken;
   const int cpt = (int)(chunks_pp / kCoopThreads);
-  const void* fn = coop_kernel(dt, cpt);
+  const CoopKernels kernels = coop_kernels(dt, cpt);
+  const void* fn = kernels.save;
   if (!fn) return kCoopNotTaken;
   const int64_t group_pages = (int64_t)g.pps * n_pages;
   if (group_pages * chunks_pp * 16 < kCoopMinGroupBytes) return kCoopNotTaken;
@@ -810,6 +852,8 @@ int try_tensor_coop(int32_t dt, const uint64_t* cache_planes, int64_t cache_page
   a.page_elems = page_elems;
   a.ws = ws;
   a.sync = ws + fp8_tensor_sync_offset(n_groups);
+  a.param_planes = param_planes;
+  a.n_planes = n_planes;
   void* args[] = {&a};
   const hipError_t e =
       hipLaunchCooperativeKernel(fn, dim3((unsigned)grid), dim3(kCoopThreads), args, 0, s);
@@ -817,6 +861,9 @@ int try_tensor_coop(int32_t dt, const uint64_t* cache_planes, int64_t cache_page
     (void)hipGetLastError();
     return kCoopNotTaken;
   }
+  if (hipLaunchKernel(kernels.finish, dim3((unsigned)grid), dim3(kCoopThreads), args, 0, s) !=
+      hipSuccess)
+    return check_launch("fp8_tensor_finish_kernel");
   return ok();
 }
 
@@ -916,13 +963,9 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
     const int n_words = (int)fp8_tensor_workspace_words(n_groups);
     fill_u32_kernel<<<(n_words + 255) / 256, 256, 0, s>>>(ws, n_words, 0u);
     rc = try_tensor_coop(cache_dtype, cache_planes, cache_page_stride, block_ids, pool_pages,
-                         code_planes, n_pages, g, n_groups, ws, err_flag, s);
-    if (rc != kCoopNotTaken) {
-      if (rc != AMF_OK) return rc;
-      AMF_WITH_DTYPE(cache_dtype, fp8_tensor_finalize_kernel<DT>
-                     <<<(n_planes + 255) / 256, 256, 0, s>>>(param_planes, ws, n_planes, g.pps));
-      return check_launch(who);
-    }
+                         code_planes, param_planes, n_planes, n_pages, g, n_groups, ws, err_flag,
+                         s);
+    if (rc != kCoopNotTaken) return rc;
     const int64_t per_plane = std::max<int64_t>(
         1, std::min<int64_t>(n_pages, (kAbsBlocks + n_planes - 1) / n_planes));
     dim3 agrid((unsigned)per_plane, (unsigned)n_planes);

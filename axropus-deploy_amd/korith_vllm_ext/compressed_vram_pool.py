@@ -774,10 +774,8 @@ class CompressedVRAMPool:
         """Per-tensor FP8: turn the asynchronously copied absmax into the
         reference's Python-double tensor_scale and FP8ScaleSidecar.
 
-        A non-finite layer absmax means the save failed (the single-read
-        kernel writes +inf for a scale group whose cross-workgroup wait gave
-        up, and a cache holding inf has no usable FP8 scale either): the
-        entry is dropped and its spans freed, and False is returned so that
+        A non-finite layer absmax (a cache holding inf) gives no usable FP8
+        scale: the entry is dropped and its spans freed, and False is returned so that
         the lookup is a miss instead of a restore of inf/NaN pages."""
         if entry.pending_absmax is None:
             return True

@@ -67,7 +67,7 @@ extern "C" {
 /* bits ORed into *err_flag by kernels */
 #define AMF_ERRFLAG_BLOCK_RANGE 1    /* a block id was outside [0, pool_pages) */
 #define AMF_ERRFLAG_CONTEXT     2    /* a context length exceeded its block table */
-#define AMF_ERRFLAG_SYNC        4    /* a cross-workgroup wait gave up (that call's output is invalid) */
+#define AMF_ERRFLAG_SYNC        4    /* a launch missed words its predecessor writes (that call's output is invalid) */
 
 /* ---- element types: same numbering as the AMFK header dtype field
  *      (core/amf_direct_kv.h AmfKvDtype; amf_kv_manager.py:60-64) --------- */
@@ -202,10 +202,10 @@ int amf_kv_scatter_slots(const uint64_t* in_planes, int64_t in_row_stride,
  * resident grid, and twice (absmax kernel, then quantize kernel) otherwise
  * or when AMF_NO_COOP is set to a non-zero value in the environment (read
  * once; for processes that cannot have a cooperative launch, such as a
- * profiler session or graph capture); both give the same bytes.  A
- * cooperative wait that gives up (never in a
- * correct launch) raises AMF_ERRFLAG_SYNC and writes an infinite scale for
- * its group.
+ * profiler session or graph capture); both give the same bytes, and so does
+ * a cooperative launch that other streams' kernels keep from being resident
+ * as a whole: its waits are bounded, and the groups they give up on are read
+ * a second time.
  * Replaces compressed_vram_pool.py:481-508 with FP8E4M3Codec.compress
  * (amf_codec.py:186-209). */
 int amf_fp8_quant_gather(int32_t format,

@@ -200,6 +200,24 @@ def test_fp8_tensor_single_read_bitexact(dtype, geom):
         assert torch.equal(side, oc.fp8_sidecar(scale)), l
 
 
+# A 16-bit per-tensor save that the single-read kernel takes: an odd group
+# count, two pages per workgroup for some of the 768 resident ones.
+SINGLE_READ_GEOM = dict(L=3, pool=530, n=513, bs=16, H=8, D=128)
+
+
+def _assert_single_read(geom):
+    """The scale groups reach the kernel's least size, as its source states it
+    (a save below it would quietly test the two-pass kernels)."""
+    import os
+    import re
+    src = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                       "axropus-deploy_amd", "csrc", "amf_coop.h")
+    with open(src) as f:
+        m = re.search(r"kCoopMinGroupBytes = (\d+)ll << (\d+);", f.read())
+    group = 2 * geom["n"] * geom["bs"] * geom["H"] * geom["D"] * 2
+    assert group >= int(m[1]) << int(m[2]), (group, m[0])
+
+
 def _tensor_save_digest(dtype, geom):
     import hashlib
     values, src_ids, _ = _codec_case(dtype, 12, geom)
@@ -219,7 +237,8 @@ def test_fp8_tensor_no_coop_environment_same_bytes():
     import os
     import subprocess
     import sys
-    geom = dict(L=3, pool=512, n=160, bs=16, H=8, D=128)
+    geom = SINGLE_READ_GEOM
+    _assert_single_read(geom)
     want = _tensor_save_digest(torch.bfloat16, geom)
     here = os.path.dirname(os.path.abspath(__file__))
     root = os.path.dirname(here)
@@ -236,9 +255,11 @@ def test_fp8_tensor_no_coop_environment_same_bytes():
 
 def test_fp8_tensor_single_read_beside_another_stream():
     """The cooperative per-tensor save issued while restores run on a second
-    stream (default priority): it completes without a sync give-up and its
-    codes still equal the oracle's."""
-    dtype, geom = torch.bfloat16, dict(L=3, pool=512, n=160, bs=16, H=8, D=128)
+    stream (default priority), whose waves can keep some of its workgroups from
+    being resident with the others: its codes and scales still equal the
+    oracle's, and nothing is flagged."""
+    dtype, geom = torch.bfloat16, SINGLE_READ_GEOM
+    _assert_single_read(geom)
     values, src_ids, dst_ids = _codec_case(dtype, 14, geom)
     L, n, bs, H, D = geom["L"], geom["n"], geom["bs"], geom["H"], geom["D"]
     cache = _cache_from(values)
@@ -269,57 +290,35 @@ def test_fp8_tensor_single_read_beside_another_stream():
         assert torch.equal(side_scale, oc.fp8_sidecar(scale)), l
 
 
-_GIVE_UP_SCRIPT = r"""
-import sys, torch
-sys.path[:0] = sys.argv[2:4]
-from korith_vllm_ext import _paged
-cache = torch.load(sys.argv[1] + "/cache.pt", weights_only=True)
-ids = torch.load(sys.argv[1] + "/ids.pt", weights_only=True)
-L, n = len(cache), ids.numel()
-layout = _paged.BlobLayout("fp8_e4m3", 2, n, 16, 8, 128)
-blobs = [torch.zeros(layout.total_bytes, dtype=torch.uint8, device="cuda") for _ in range(L)]
-flag = torch.zeros(1, dtype=torch.int32, device="cuda")
-view = _paged.cache_view([c.cuda() for c in cache])
-_paged.quant_gather(layout, view, ids, [b.data_ptr() for b in blobs], 2, err_flag=flag)
-torch.cuda.synchronize()
-torch.save({"flag": flag.cpu(), "blobs": [b.cpu() for b in blobs]}, sys.argv[1] + "/out.pt")
-"""
-
-
-def test_fp8_tensor_single_read_give_up_path(tmp_path):
-    """With the wait bound forced to zero polls (AMF_COOP_SPIN_LIMIT=0, read
-    once per process, hence a child process) a workgroup that finds its
-    group not yet complete takes the give-up path at once.  Whether any does
-    depends on timing (a workgroup's loads of the next group usually outlast
-    the exchange), so the check is the invariant: the launch finishes, and
-    each layer holds either the oracle's codes or an infinite scale (never
-    plausible wrong values), with AMF_ERRFLAG_SYNC raised exactly when some
-    layer is poisoned."""
-    import os
-    import subprocess
-    import sys
-
-    geom = dict(L=3, pool=512, n=160, bs=16, H=8, D=128)
+def test_fp8_tensor_single_read_give_up_path(monkeypatch):
+    """With the wait bound forced to zero polls every wait gives up at once and
+    every group is quantized from a second read: the launch finishes, and every
+    layer holds the oracle's codes and scale.  (In this process: a second
+    process beside one that has made a cooperative launch may be refused its
+    own, and would test the two-pass kernels.)"""
+    geom = SINGLE_READ_GEOM
+    _assert_single_read(geom)
     values, src_ids, _ = _codec_case(torch.bfloat16, 16, geom)
-    torch.save([values[l].contiguous() for l in range(geom["L"])], tmp_path / "cache.pt")
-    torch.save(src_ids, tmp_path / "ids.pt")
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    env = dict(os.environ, AMF_COOP_SPIN_LIMIT="0")
-    subprocess.run([sys.executable, "-c", _GIVE_UP_SCRIPT, str(tmp_path), root,
-                    os.path.join(root, "axropus-deploy_amd")], env=env, check=True, timeout=90)
-    out = torch.load(tmp_path / "out.pt", weights_only=True)
-    gave_up = bool(int(out["flag"].item()) & amf_hip.ERRFLAG_SYNC)
-    layout = _paged.BlobLayout("fp8_e4m3", 2, geom["n"], 16, 8, 128)
-    poisoned = 0
-    for l, blob in enumerate(out["blobs"]):
-        side = blob[layout.scale_offset:layout.scale_offset + 16].view(torch.float32)
-        if torch.isinf(side[0]):
-            poisoned += 1
-            continue
+    L, n = geom["L"], geom["n"]
+    layout = _paged.BlobLayout("fp8_e4m3", 2, n, 16, 8, 128)
+    blobs = [torch.zeros(layout.total_bytes, dtype=torch.uint8, device=DEV) for _ in range(L)]
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    view = _paged.cache_view(_cache_from(values))
+    monkeypatch.setenv("AMF_COOP_SPIN_LIMIT", "0")
+    ws = _paged.quant_gather(layout, view, src_ids, [b.data_ptr() for b in blobs], 2,
+                             err_flag=flag)
+    torch.cuda.synchronize()
+    # group l's root line, after 32 absmax words and 32 cluster lines of 32 words:
+    # all clusters reported; left to the second read
+    lines = ws.view(torch.int32)[32:].view(-1, 32).cpu()
+    for l in range(L):
+        assert lines[33 * l + 32, 0] == 32 and lines[33 * l + 32, 2] == 1, l
+    assert int(flag.item()) == 0
+    for l, blob in enumerate(blobs):
         codes, scale = oc.fp8_tensor_compress(_pages(values, l, src_ids))
-        assert np.array_equal(bytes_of(blob[:layout.data_bytes]), bytes_of(codes)), l
+        assert np.array_equal(bytes_of(_seg(blob, 0, layout.data_bytes)), bytes_of(codes)), l
+        side = _seg(blob, layout.scale_offset, 16).view(torch.float32).cpu()
         assert torch.equal(side, oc.fp8_sidecar(scale)), l
-    assert gave_up == (poisoned > 0), (gave_up, poisoned)
 
 
 @pytest.mark.parametrize("dtype,geom", CODEC_CASES)

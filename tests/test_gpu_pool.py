@@ -173,8 +173,7 @@ def test_vllm_roundtrip_bitexact(fmt, dtype):
 
 
 def test_failed_per_tensor_fp8_save_is_a_miss():
-    """A per-tensor FP8 save whose layer absmax comes back non-finite (what
-    the single-read kernel writes for a scale group whose wait gave up) is
+    """A per-tensor FP8 save whose layer absmax comes back non-finite is
     dropped on first lookup: get() misses, restore_to_vllm restores nothing
     and returns 0, and the entry's spans are free again."""
     L, pool_pages, n, H, D = 2, 32, 8, 2, 64
@@ -185,7 +184,7 @@ def test_failed_per_tensor_fp8_save_is_a_miss():
     assert p.put_from_vllm("bad", cache, list(range(n)), n * 16)
     host, ev = p._index["bad"].pending_absmax
     ev.synchronize()
-    host.view(torch.float32)[1] = float("inf")   # layer 1's save "gave up"
+    host.view(torch.float32)[1] = float("inf")   # as from an infinite value in layer 1
     target = sentinel_cache(L, pool_pages, 16, H, D, torch.bfloat16, DEV)
     before = p.stats()["misses"]
     assert p.restore_to_vllm("bad", target, list(range(n))) == 0

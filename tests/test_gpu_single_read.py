@@ -17,6 +17,5 @@ pytestmark = pytest.mark.gpu
     pytest.param(torch.float16, dict(L=1, pool=4200, n=4100, bs=16, H=2, D=64), id="fp16-cpt1"),
 ])
 def test_single_read_large_groups(dtype, geom):
-    group = 2 * geom["n"] * geom["bs"] * geom["H"] * geom["D"] * 2
-    assert group >= 32 << 20
+    kernels._assert_single_read(geom)
     kernels.test_fp8_tensor_single_read_bitexact(dtype, geom)
