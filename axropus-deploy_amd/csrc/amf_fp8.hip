@@ -1006,9 +1006,12 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
   const int cpl = (int)(head_chunks / 32);
   if (!pt && cache_dtype != AMF_DTYPE_F32 && head_chunks % 32 == 0 &&
       n_pages * num_heads <= 0x7FFFFFF0ll && (cpl == 2 || cpl == 4 || cpl == 8 || cpl == 16)) {
-    // Pages that leave most of a workgroup's half-waves idle share workgroups:
-    // 80 layers x 777 pages of 1 head 181 -> 119 us; no gain from 2 heads on.
-    const bool pack = num_heads < 4;
+    // Pages of one or two heads share workgroups, which they would leave mostly
+    // idle (a workgroup per page / shared, us: 80 layers x 777 pages of 1 x 128 188 /
+    // 129; 32 x 100 of 2 x 128 18.9 / 16.0, 32 x 1000 124.8 / 125.2).  Pages of
+    // three would lie across two workgroups: 32 x 700 of 3 x 128 152 / 165, of 3 x
+    // 64 76 / 87.
+    const bool pack = num_heads < 3;
     const dim3 pgrid(
         (unsigned)((n_pages * num_heads + kThreads / 32 - 1) / (kThreads / 32)),
         (unsigned)n_planes);
