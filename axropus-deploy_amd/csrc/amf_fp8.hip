@@ -792,7 +792,7 @@ void launch_restore(int32_t format, int64_t n_pages, hipStream_t s, const uint64
           code_planes, param_planes, cache_planes, cache_stride, block_ids, pool, n_pages,   \
           n_planes, g, rows, err_flag)
   if constexpr (!SLOTS) {
-    if ((int64_t)g.n_rows * g.head_dim <= 8 * kSmallPageChunks) {
+    if (small_restore_page((int64_t)g.n_rows * g.head_dim / 8, cache_dtype)) {
       AMF_WITH_DTYPE(cache_dtype, if (pt) AMF_LAUNCH(true, 64); else AMF_LAUNCH(false, 64));
       return;
     }
@@ -975,8 +975,14 @@ extern "C" int amf_fp8_quant_gather(int32_t format, const uint64_t* cache_planes
 #define AMF_LAUNCH(P)                                                                     \
   fp8_absmax_kernel<DT, P><<<agrid, kThreads, 0, s>>>(                                    \
       cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, g, ws, err_flag)
-    AMF_WITH_DTYPE(cache_dtype, if (lane_vecs == 1) AMF_LAUNCH(8);
-                   else if (lane_vecs == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
+    // Several 16-bit pages at a time where a workgroup has more than one, but not
+    // pages of one vector for some lanes and two for others (32 x 300 pages of 3 x
+    // 64 64 / 66 us one / four at a time; fp32 of 1 x 64 48 / 50, 16-bit 47 / 45).
+    const bool even = lane_vecs == 1 || (int64_t)g.n_rows * head_dim / 8 % kThreads == 0;
+    const int64_t step =
+        cache_dtype != AMF_DTYPE_F32 && even && n_pages > per_plane ? lane_vecs : 0;
+    AMF_WITH_DTYPE(cache_dtype, if (step == 1) AMF_LAUNCH(8);
+                   else if (step == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
 #undef AMF_LAUNCH
   }
   // Per-tensor pass 2: pages of 1-16 chunks of 8 elements per lane take the

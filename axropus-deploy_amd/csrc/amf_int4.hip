@@ -36,10 +36,6 @@ struct SymGeom {
   int pps;        // planes per scale group (per-channel format)
 };
 
-__device__ __forceinline__ int sym_col(const SymGeom& g) { return threadIdx.x & ((1 << g.cpr_log2) - 1); }
-__device__ __forceinline__ int sym_row0(const SymGeom& g) { return threadIdx.x >> g.cpr_log2; }
-__device__ __forceinline__ int sym_rpi(const SymGeom& g) { return kThreads >> g.cpr_log2; }
-
 // 32 cache elements at byte address `p` -> fp32.
 template <int DT>
 __device__ __forceinline__ void load32(const uint8_t* p, float* x) {
@@ -244,18 +240,21 @@ int4_symblock_quant_gather_kernel(
 // INT4_SYM_BLOCK save of pages larger than the register-resident kernels
 // hold, and of fp32 caches: the page absmax in a first read, the codes in a
 // second (which hits in cache).  One lane = one 8-element chunk per step,
-// kLoopUnroll of them loaded before any is used: a page is one workgroup
+// U of them loaded before any is used: a page is one workgroup
 // however large it is, so the bytes that workgroup keeps in flight set its
 // rate (a page of 2M elements 500 -> 121 us with 1024 lanes of 4 chunks for 256
-// of one).  Same arithmetic as int4_symblock_quant_gather_kernel.
-constexpr int kLoopUnroll = 4;
+// of one).  An fp32 page of at most kLoopChunks chunks leaves such a workgroup
+// mostly idle and takes 256 lanes of one (32 x 300 pages of 1 x 64 71 / 21 us
+// with 1024 / 256 lanes, 32 x 250 of 5 x 128 205 / 195, 32 x 200 of 8 x 128 224 /
+// 248).  Same arithmetic as int4_symblock_quant_gather_kernel.
+constexpr int64_t kLoopChunks = 1536;
 
-template <int DT>
-__global__ __launch_bounds__(kBigThreads) void int4_symblock_quant_looped_kernel(
+template <int DT, int NT, int U>
+__global__ __launch_bounds__(NT) void int4_symblock_quant_looped_kernel(
     const uint64_t* __restrict__ cache_planes, int64_t cache_stride,
     const int32_t* __restrict__ block_ids, int64_t pool, const uint64_t* __restrict__ code_planes,
     const uint64_t* __restrict__ param_planes, SymGeom g, int32_t* err_flag) {
-  constexpr int ES = elem_bytes<DT>(), U = kLoopUnroll;
+  constexpr int ES = elem_bytes<DT>();
   const int64_t j = blockIdx.x;
   const int plane = blockIdx.y;
   const int64_t sp = block_ids ? (int64_t)block_ids[j] : j;
@@ -269,11 +268,11 @@ __global__ __launch_bounds__(kBigThreads) void int4_symblock_quant_looped_kernel
   uint32_t* __restrict__ codes = reinterpret_cast<uint32_t*>(code_planes[plane]) + j * n8;
   _Float16* __restrict__ params = reinterpret_cast<_Float16*>(param_planes[plane]);
   float m = 0.0f;
-  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * kBigThreads) {
+  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * NT) {
     float x[U][8];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = k0 + u * kBigThreads;  // past the end: the lane's first chunk again
+      const int64_t k = k0 + u * NT;  // past the end: the lane's first chunk again
       load8<DT>(src + (k < n8 ? k : k0) * (8 * ES), x[u]);
     }
 #pragma unroll
@@ -282,25 +281,25 @@ __global__ __launch_bounds__(kBigThreads) void int4_symblock_quant_looped_kernel
       for (int n = 0; n < 8; ++n) m = fmaxf(m, fabsf(x[u][n]));
   }
   m = wave_max_xor(m, 64);
-  __shared__ float s_wmax[kBigThreads / 64];
+  __shared__ float s_wmax[NT / 64];
   if ((threadIdx.x & 63) == 0) s_wmax[threadIdx.x >> 6] = m;
   __syncthreads();
   float amax = s_wmax[0];
 #pragma unroll
-  for (int w = 1; w < kBigThreads / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
+  for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, s_wmax[w]);
   const float scale = fmaxf(amax, 1e-8f) / kSymMax;
   const float rscale = 1.0f / scale;
   if (threadIdx.x == 0) params[j] = (_Float16)scale;
-  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * kBigThreads) {
+  for (int64_t k0 = threadIdx.x; k0 < n8; k0 += U * NT) {
     float x[U][8];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = k0 + u * kBigThreads;
+      const int64_t k = k0 + u * NT;
       load8<DT>(src + (k < n8 ? k : k0) * (8 * ES), x[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = k0 + u * kBigThreads;
+      const int64_t k = k0 + u * NT;
       uint32_t w = 0;
 #pragma unroll
       for (int n = 0; n < 8; ++n)
@@ -537,7 +536,9 @@ constexpr int kKUnroll = AMF_ASYM_K_UNROLL;
 // TEAM lanes take a page (four pages a workgroup when it is small), and a V
 // item writes 8 / VSPLIT of its tokens, so that a page of few heads still has
 // an item for each lane.  P2: head_dim and the head count are powers of two,
-// so the items' indices are shifts.  80 layers x 777 pages of 1 x 128 235 ->
+// so the items' indices are shifts (others divide, a workgroup to a page: no
+// model of the sizes served here has such pages).  fp32 pages, twice the bytes,
+// keep a workgroup each.  80 layers x 777 pages of 1 x 128 235 ->
 // 113 us, 32 x 1000 of 2 x 128 153 -> 115 us (6.0 TB/s), 32 x 512 of 8 x 128
 // 245 -> 241 us.
 template <int DT, int TEAM, int VSPLIT, bool P2>
@@ -866,11 +867,14 @@ void launch_symblock_quant(bool bf16, int64_t n8, int64_t n_pages, int n_planes,
                   cache_planes, cache_stride, block_ids, pool, n_pages, code_planes,          \
                   param_planes, g, rows, err_flag))
   if constexpr (!SLOTS) {
-    if (n8 <= 256) {
+    // a wave per small page once there are pages enough to wait for: 2560 pages
+    // of 1 x 128 6.2 / 6.5 us as workgroups / waves, 4096 7.8 / 7.2
+    const bool many = n_pages * n_planes >= 4096;
+    if (many && n8 <= 256) {
       AMF_LAUNCH(4, 64);
       return;
     }
-    if (n8 <= kSmallPageChunks) {
+    if (many && n8 <= kSmallPageChunks) {
       AMF_LAUNCH(8, 64);
       return;
     }
@@ -910,7 +914,7 @@ int launch_sym_restore(const char* who, int32_t format, int64_t n_pages, hipStre
           n_planes, parts, g, rows, err_flag)
   if constexpr (!SLOTS) {
     // a wave's pass of 512 elements keeps a lane's channels as well
-    if (n8 <= kSmallPageChunks && (!ch || 512 % g.head_dim == 0)) {
+    if (small_restore_page(n8, cache_dtype) && (!ch || 512 % g.head_dim == 0)) {
       AMF_WITH_DTYPE(cache_dtype, if (ch) AMF_LAUNCH(true, 64); else AMF_LAUNCH(false, 64));
       return check_launch(who);
     }
@@ -1003,9 +1007,10 @@ extern "C" int amf_int4_dequant_scatter(int32_t format, const uint64_t* code_pla
                                       cache_page_stride, block_ids, pool_pages, n_pages, g,    \
                                       err_flag))
     const int64_t v_items = (int64_t)num_heads * head_dim / 8 * 2;
+    const bool small = cache_dtype != AMF_DTYPE_F32 && 8 * v_items <= kSmallPageChunks;
     if (g.kpr_log2 < 0 || g.h_log2 < 0) AMF_LAUNCH(256, 1, false);
-    else if (8 * v_items > kSmallPageChunks && v_items < kThreads) AMF_LAUNCH(256, 2, true);
-    else if (8 * v_items > kSmallPageChunks) AMF_LAUNCH(256, 1, true);
+    else if (!small && v_items < kThreads) AMF_LAUNCH(256, 2, true);
+    else if (!small) AMF_LAUNCH(256, 1, true);
     else if (v_items <= 16) AMF_LAUNCH(64, 4, true);
     else if (v_items <= 32) AMF_LAUNCH(64, 2, true);
     else AMF_LAUNCH(64, 1, true);
@@ -1128,10 +1133,14 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
     // Pages that fit lanes' registers (at most kMaxRegChunks chunks) take the
     // single-read kernel; larger pages and fp32 caches the two-read one.
     if (cache_dtype == AMF_DTYPE_F32 || n8 > kMaxRegChunks) {
-      AMF_WITH_DTYPE(cache_dtype,
-                     int4_symblock_quant_looped_kernel<DT><<<grid, kBigThreads, 0, s>>>(
-                         cache_planes, cache_page_stride, block_ids, pool_pages, code_planes,
-                         param_planes, g, err_flag));
+#define AMF_LAUNCH(DT, NT, U)                                                          \
+  int4_symblock_quant_looped_kernel<DT, NT, U><<<grid, NT, 0, s>>>(                    \
+      cache_planes, cache_page_stride, block_ids, pool_pages, code_planes, param_planes, g, err_flag)
+      if (n8 <= kLoopChunks)
+        AMF_LAUNCH(AMF_DTYPE_F32, kThreads, 1);
+      else
+        AMF_WITH_DTYPE(cache_dtype, AMF_LAUNCH(DT, kBigThreads, 4));
+#undef AMF_LAUNCH
       return check_launch(who);
     }
     launch_symblock_quant<false>(bf16, n8, n_pages, n_planes, s, cache_planes, cache_page_stride, block_ids,
@@ -1154,8 +1163,12 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
 #define AMF_LAUNCH(P)                                                                   \
   int4_channel_absmax_kernel<DT, P><<<rgrid, kThreads, 0, s>>>(                         \
       cache_planes, cache_page_stride, block_ids, pool_pages, n_pages, g, ws, err_flag)
-  AMF_WITH_DTYPE(cache_dtype, if (lane_chunks == 1) AMF_LAUNCH(8);
-                 else if (lane_chunks == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
+  // several pages at a time where a workgroup has more than one (fp32, 32 x 300
+  // pages of 3 x 64: 102 / 109 us one / four at a time)
+  const int64_t step =
+      cache_dtype != AMF_DTYPE_F32 && n_pages > AMF_ABSMAX_WGS ? lane_chunks : 0;
+  AMF_WITH_DTYPE(cache_dtype, if (step == 1) AMF_LAUNCH(8);
+                 else if (step == 2) AMF_LAUNCH(4); else AMF_LAUNCH(1));
 #undef AMF_LAUNCH
 #define AMF_LAUNCH(TEAM)                                                                      \
   AMF_WITH_DTYPE(cache_dtype, int4_channel_quant_gather_kernel<DT, TEAM>                      \
@@ -1164,7 +1177,10 @@ extern "C" int amf_int4_quant_gather(int32_t format, const uint64_t* cache_plane
                     kThreads, 0, s>>>(cache_planes, cache_page_stride, block_ids, pool_pages, \
                                       n_pages, code_planes, param_planes, g, ws, err_flag))
   // a wave's pass of 512 elements keeps a lane's channels as well
-  if ((int64_t)g.n_rows * head_dim <= 8 * kSmallPageChunks && 512 % head_dim == 0) AMF_LAUNCH(64);
+  // (fp32: up to half the chunks, 32 x 300 pages of 1 x 64 58 / 47 us with a
+  // workgroup / a wave, of 3 x 64 105 / 110)
+  const int64_t small = kSmallPageChunks / (cache_dtype == AMF_DTYPE_F32 ? 2 : 1);
+  if ((int64_t)g.n_rows * head_dim <= 8 * small && 512 % head_dim == 0) AMF_LAUNCH(64);
   else AMF_LAUNCH(kThreads);
 #undef AMF_LAUNCH
   return check_launch(who);

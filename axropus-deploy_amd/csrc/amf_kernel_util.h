@@ -40,8 +40,15 @@ constexpr unsigned kRestoreLdsPad = 52u << 10;
 // of 1 x 128, a workgroup / a wave per page, us: fp8_e4m3 279 / 138,
 // fp8_e4m3_ph 312 / 138, int4_sym 193 / 117; 32 x 1000 of 2 x 128: 164 / 148,
 // 205 / 146, 150 / 127.  Pages of 4 x 128 run at 5.2-5.6 TB/s as workgroups.
+// fp32 pages hold twice the bytes a chunk: restores keep the workgroup from 256
+// chunks on (int4_sym, 80 layers x 300 pages of 1 x 128 114 / 170, fp8_e4m3 of
+// 1 x 64 45 / 34).
 constexpr int kPageTeam = 256;
 constexpr int64_t kSmallPageChunks = 512;
+
+inline bool small_restore_page(int64_t chunks, int32_t cache_dtype) {
+  return chunks <= (cache_dtype == AMF_DTYPE_F32 ? kSmallPageChunks / 4 : kSmallPageChunks);
+}
 
 struct PageWork {
   int64_t j;   // position in the gathered sequence

@@ -18,6 +18,12 @@ GEOMS = [  # heads, head_dim, pages
     (4, 128, 6), (5, 128, 2), (8, 128, 3), (16, 64, 2),
 ]
 
+# the asymmetric format also takes head_dims that are no power of two
+ASYM_GEOMS = [(1, 96, 5), (2, 96, 3), (3, 96, 2)]
+# pages enough for the block save's wave per page (4096 in the three layers) and
+# for the per-tensor and per-channel formats' maxima over several pages at a time
+MANY_GEOMS = [(1, 32, 701), (3, 64, 690), (2, 128, 690)]
+
 
 def _oracle(fmt, x, dtype):
     """The oracle's restored values of one layer's pages [2, n, 16, H, D]."""
@@ -35,11 +41,12 @@ def _oracle(fmt, x, dtype):
 
 @pytest.mark.parametrize("fmt", ["fp8_e4m3", "fp8_e4m3_ph", "int4_sym", "int4_sym_block",
                                  "int4_asym_g32"])
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_small_pages_match_oracle(fmt, dtype):
     from korith_vllm_ext import _paged
 
-    for H, D, n in GEOMS:
+    for H, D, n in GEOMS + (ASYM_GEOMS if fmt == "int4_asym_g32" else
+                            MANY_GEOMS if fmt != "fp8_e4m3_ph" else []):
         g = torch.Generator().manual_seed(H * 1000 + D + n)
         L, pool = 3, n + 4
         x = torch.randn(L, 2, pool, 16, H, D, generator=g)
@@ -51,7 +58,7 @@ def test_small_pages_match_oracle(fmt, dtype):
         blobs = torch.zeros(L, (lay.total_bytes + 15) // 16 * 16, dtype=torch.uint8, device=DEV)
         bases = [blobs[l].data_ptr() for l in range(L)]
         cache, target = x.to(DEV), torch.full_like(x, -7.25, device=DEV)
-        # one block id out of the pool: skipped on both ways, and flagged
+        # one block id out of the pool: skipped, and flagged
         err = torch.zeros(1, dtype=torch.int32, device=DEV)
         _paged.quant_gather(lay, _paged.cache_view(list(cache)), src, bases, 2)
         bad = dst.clone()
@@ -64,3 +71,42 @@ def test_small_pages_match_oracle(fmt, dtype):
             keep = [i for i in range(n) if i != n // 2]
             want[l][:, dst[keep].long()] = y.reshape(2, n, 16, H, D)[:, keep]
         assert (bits(target) == bits(want)).all(), (fmt, dtype, H, D, n)
+
+
+@pytest.mark.parametrize("fmt", ["fp8_e4m3", "fp8_e4m3_ph", "int4_sym", "int4_sym_block",
+                                 "int4_asym_g32"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_small_page_save_skips_a_bad_id(fmt, dtype):
+    """A source block id out of the pool is flagged, leaves its page's codes and
+    params as they were, and the pages that share its workgroup get the bytes
+    they get without it (a page of zeros in its place: no scale changes)."""
+    from korith_vllm_ext import _paged
+
+    for H, D, n in GEOMS + MANY_GEOMS[:2]:
+        g = torch.Generator().manual_seed(H * 1000 + D + n)
+        L, pool = 3, n + 4
+        x = torch.randn(L, 2, pool, 16, H, D, generator=g).to(dtype)
+        src = torch.randperm(pool, generator=g)[:n].to(torch.int32)
+        bad = n // 2
+        x[:, :, int(src[bad])] = 0
+        cache = _paged.cache_view(list(x.to(DEV)))
+        lay = _paged.BlobLayout(fmt, 2, n, 16, H, D)
+        wrong = src.clone()
+        wrong[bad] = pool
+        blobs = [torch.full((L, (lay.total_bytes + 15) // 16 * 16), 0xA5, dtype=torch.uint8,
+                            device=DEV) for _ in range(2)]
+        err = torch.zeros(1, dtype=torch.int32, device=DEV)
+        for ids, b in ((src, blobs[0]), (wrong, blobs[1])):
+            _paged.quant_gather(lay, cache, ids, [b[l].data_ptr() for l in range(L)], 2,
+                                err_flag=err)
+            assert int(err) == (0 if ids is src else 1)
+        want, got = blobs
+        code = lay.code_bytes_per_page
+        for p in range(2):
+            at = lay.code_offset(p) + bad * code
+            want[:, at:at + code] = 0xA5
+            if not lay.shared_params:
+                each = lay.plane_param_bytes // n
+                at = lay.param_offset(p) + bad * each
+                want[:, at:at + each] = 0xA5
+        assert torch.equal(got, want), (fmt, dtype, H, D, n)
