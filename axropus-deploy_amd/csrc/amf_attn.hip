@@ -819,7 +819,7 @@ constexpr int kMergeWaves = 4;
 constexpr int kMergeBatch = 16;  // accumulator loads per lane in flight
 static_assert(kSplitWaves <= kMaxSplits, "dense_splits gives at most kSplitWaves splits");
 
-template <int OUT_DT, int D>
+template <int OUT_DT, int D, bool MASK>
 __global__ __launch_bounds__(64 * kMergeWaves) void dense_attn_merge_kernel(AttnArgs a,
                                                                           const float* part,
                                                                           int64_t n_splits) {
@@ -833,7 +833,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void dense_attn_merge_kernel(Attn
   const float* pr = part + row * n_splits * (int64_t)STRIDE;
   const int quad = lane % Q, phase = lane / Q;
   const int k0 = wv * P + phase;  // this lane's splits: k0, k0 + S, ...
-  const float e2 = exp2_factor(a);
+  constexpr float e2 = MASK ? kLog2e : 1.0f;  // exp2_factor(a)
   f32x4 x[kMergeBatch];
 #pragma unroll
   for (int i = 0; i < kMergeBatch; ++i) {
@@ -929,13 +929,19 @@ void launch_split_gh(const AttnArgs& a, float* part, int64_t split_tokens, int64
 void amf::launch_merge(const AttnArgs& a, int32_t out_dtype, int64_t rows, const float* part,
                   int64_t n_splits, hipStream_t st) {
   const dim3 mgrid((unsigned)rows);
-#define AMF_MERGE(OUT)                                                                            \
-  if (a.head_dim == 64)                                                                           \
-    dense_attn_merge_kernel<OUT, 64><<<mgrid, 64 * kMergeWaves, 0, st>>>(a, part, n_splits);      \
-  else if (a.head_dim == 128)                                                                     \
-    dense_attn_merge_kernel<OUT, 128><<<mgrid, 64 * kMergeWaves, 0, st>>>(a, part, n_splits);     \
+#define AMF_MERGE_D(OUT, D)                                                                       \
+  if (a.mask)                                                                                     \
+    dense_attn_merge_kernel<OUT, D, true><<<mgrid, 64 * kMergeWaves, 0, st>>>(a, part, n_splits); \
   else                                                                                            \
-    dense_attn_merge_kernel<OUT, 256><<<mgrid, 64 * kMergeWaves, 0, st>>>(a, part, n_splits)
+    dense_attn_merge_kernel<OUT, D, false><<<mgrid, 64 * kMergeWaves, 0, st>>>(a, part, n_splits)
+#define AMF_MERGE(OUT)                                \
+  if (a.head_dim == 64) {                             \
+    AMF_MERGE_D(OUT, 64);                             \
+  } else if (a.head_dim == 128) {                     \
+    AMF_MERGE_D(OUT, 128);                            \
+  } else {                                            \
+    AMF_MERGE_D(OUT, 256);                            \
+  }
   if (out_dtype == AMF_DTYPE_F32) {
     AMF_MERGE(AMF_DTYPE_F32);
   } else if (out_dtype == AMF_DTYPE_BF16) {
@@ -944,6 +950,7 @@ void amf::launch_merge(const AttnArgs& a, int32_t out_dtype, int64_t rows, const
     AMF_MERGE(AMF_DTYPE_F16);
   }
 #undef AMF_MERGE
+#undef AMF_MERGE_D
 }
 
 namespace {
