@@ -1191,7 +1191,12 @@ extern "C" int amf_int4_sym_dense_attn(const void* q, int32_t dtype, const void*
   dense_splits(rows, heads_per_wave(num_q_heads, num_kv_heads), kv_len, &n_splits,
                &split_tokens);
   float* part = static_cast<float*>(workspace);
-  // the MFMA kernel addresses a (batch, KV head) row of codes with 32-bit offsets
+  // The MFMA kernel addresses a (batch, KV head) row of codes with 32-bit
+  // offsets.  It also serves many rows without a mask, though the tiles are the
+  // faster from about 16 on (32 / 8 heads, 16 / 128 / 512 rows x 4096 tokens 23 /
+  // 139 / 359 us against 18 / 45 / 94): they attend over K and V rounded to q's
+  // dtype, it over the exact (code - 8) * scale (error against 64 bits, bf16 2.9e-3
+  // against 1.7e-3).
   const bool mfma = head_dim == 128 && !mask && dtype != AMF_DTYPE_F32 &&
                     kv_len < ((int64_t)1 << 32) / 64;
   PrefillPlan plan;

@@ -158,7 +158,8 @@ inline int coop_blocks(const void* fn) {
 // second read.  32 layers of 8 x 128, single read / two passes, us: 64 pages
 // 236 / 65, 256 pages (16 MiB) 305 / 215, 384 pages 372 / 332, 512 pages (32
 // MiB) 437 / 436, 768 pages 572 / 669; 80 layers x 777 pages of 1 x 128 (6 MiB)
-// 823 / 236.
+// 823 / 214.  Groups of 32 to 47 MiB of 4 to 16 KiB pages take the same either way
+// (within 1 us of each other from 119 to 167 us).
 constexpr int64_t kCoopMinGroupBytes = 32ll << 20;
 
 }  // namespace amf

@@ -453,7 +453,8 @@ __global__ __launch_bounds__(64 * NW, D == 256 && NW == 1 ? 1 : 2) void prefill_
 // out = sum_k f_k acc_k / sum_k f_k l_k, f_k = 2^((m_k - M) e2), over a row's splits,
 // one lane per four dims, each reading every (m, l) of its row itself; all of
 // the at most N splits' loads are in flight together (in a loop over the splits
-// they followed each other: 64 rows of 8 splits 6 us instead of 3).  More than
+// they followed each other: a call of 64 rows x 1024 tokens, 8 heads over one of
+// 128 dims, 14.5 us instead of 11.5).  More than
 // kFewSplits splits go to the one-row kernel's merge (a workgroup per row).
 constexpr int kFewSplits = 8;
 
